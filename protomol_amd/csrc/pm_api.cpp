@@ -120,13 +120,13 @@ struct pm_context {
 
   // bonded terms
   int nbonds = 0, nangles = 0;
-  int *d_b_a = nullptr, *d_b_b = nullptr, *d_b_row = nullptr, *d_b_idx = nullptr;
+  int *d_b_a = nullptr, *d_b_b = nullptr;
   double *d_b_k = nullptr, *d_b_r0 = nullptr;
-  int *d_a_a = nullptr, *d_a_b = nullptr, *d_a_c = nullptr, *d_a_row = nullptr, *d_a_idx = nullptr;
+  int *d_a_a = nullptr, *d_a_b = nullptr, *d_a_c = nullptr;
   double *d_a_k = nullptr, *d_a_t0 = nullptr, *d_a_kub = nullptr, *d_a_rub = nullptr;
   // torsions: kind 0 dihedrals, kind 1 impropers
   int ntors[2] = {0, 0};
-  int *d_t_row[2] = {nullptr, nullptr}, *d_t_idx[2] = {nullptr, nullptr}, *d_t_term[2] = {nullptr, nullptr};
+  int* d_t_term[2] = {nullptr, nullptr};
   int4* d_t_atoms[2] = {nullptr, nullptr};
   double *d_t_k[2] = {nullptr, nullptr}, *d_t_phase[2] = {nullptr, nullptr};
   int* d_t_n[2] = {nullptr, nullptr};
@@ -173,6 +173,7 @@ struct pm_context {
   // state
   double *d_pos = nullptr, *d_vel = nullptr;
   long long* d_force = nullptr;
+  long long* d_force_side = nullptr;   // [3n] forces of the second stream (PME, correction), added by the fold
   double* d_energy = nullptr;     // [PM_NE]
   double* d_scratch3 = nullptr;   // [3n] double conversions
 
@@ -1116,12 +1117,12 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     }
   }
   std::vector<PairPass> passes = plan_passes(c, handles);
-  bool any_pme_recip = false;
-  for (int h : handles) if (c->forces[h].pme && c->forces[h].recip) any_pme_recip = true;
+  bool any_pme = false;
+  for (int h : handles) any_pme |= c->forces[h].pme;
 
   // binning and slot layout (shared by every pass and by PME)
   if ((r = ensure_cells(c))) return r;
-  if (!c->d_force || !c->d_pos || !c->d_q || !c->d_type || !c->d_stats || !c->d_overflow || !c->d_energy ||
+  if (!c->d_force || !c->d_force_side || !c->d_pos || !c->d_q || !c->d_type || !c->d_stats || !c->d_overflow || !c->d_energy ||
       !c->d_rebuild || !c->d_xbuild)
     return fail(c, PM_ERR_STATE, "internal: device buffer missing before launch");
   const int nc = c->ncells;
@@ -1152,7 +1153,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   const bool binned = prebinned && c->prebin_gen == c->layout_gen;
   if (!binned) {
     pm_launch_zero_force_cells(s, rb, c->d_force, 3LL * n, c->d_force_slot,
-                               passes.empty() ? 0 : 3LL * c->nslot_max, nullptr, 0);
+                               passes.empty() && !any_pme ? 0 : 3LL * c->nslot_max, nullptr, 0);
     pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, rb);
   }
   pm_launch_scan_cells(s, nc, c->box.n[2], c->d_bin_count, c->d_cell_count, c->d_cell_start, c->d_cell_slot, c->d_counts,
@@ -1301,7 +1302,8 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       a.tw = c->d_tw;
       a.err = c->d_overflow;
       a.prio = pme_priority(c);
-      a.force_fix = c->d_force;
+      a.force_fix = c->d_force_side;
+      a.accumulate = pme_launch.empty() ? 0 : 1;
       a.epart = c->d_epart + off * PM_NE;
       a.want_virial = vir ? 1 : 0;
       a.want_energy = want_energy ? 1 : 0;
@@ -1373,7 +1375,8 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       pm_launch_adjoint(s, c->box, pl.first, pl.second, c->precision, adj->mode, adj->slot_v, adj->slot);
     }
     if (!pair_launch.empty())
-      pm_launch_fold_slots(s, c->nslot_max, c->d_counts, c->d_atom_of_slot, adj->slot, adj->fix, nullptr, nullptr, 0);
+      pm_launch_fold_slots(s, c->nslot_max, c->d_counts, c->d_atom_of_slot, adj->slot, nullptr, adj->fix, nullptr,
+                           nullptr, 0);
     for (auto& pl : pme_launch)
       pm_launch_pme_adjoint(s, pl.first, c->plans, c->d_slot_pos64, c->precision, adj->mode == 1 ? 1 : 0,
                             adj->slot_v, adj->mode == 1 ? adj->hv : adj->dq);
@@ -1401,9 +1404,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   }
   PmBondedLaunch b{};
   if (any_bonded) {
-    b.n = n;
     b.pos = c->d_pos;
-    b.b_row = c->d_b_row; b.b_idx = c->d_b_idx; b.a_row = c->d_a_row; b.a_idx = c->d_a_idx;
     b.nb = c->nbonds; b.na = c->nangles;
     b.b_a = c->d_b_a; b.b_b = c->d_b_b; b.b_k = c->d_b_k; b.b_r0 = c->d_b_r0;
     b.a_a = c->d_a_a; b.a_b = c->d_a_b; b.a_c = c->d_a_c; b.a_k = c->d_a_k; b.a_t0 = c->d_a_t0;
@@ -1411,7 +1412,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     b.do_bond = do_bond ? 1 : 0;
     b.do_angle = do_angle ? 1 : 0;
     for (int k = 0; k < 2; k++) {
-      b.t_row[k] = c->d_t_row[k]; b.t_idx[k] = c->d_t_idx[k]; b.nt[k] = c->ntors[k];
+      b.nt[k] = c->ntors[k];
       b.t_atoms[k] = c->d_t_atoms[k]; b.t_term[k] = c->d_t_term[k];
       b.t_k[k] = c->d_t_k[k]; b.t_n[k] = c->d_t_n[k]; b.t_phase[k] = c->d_t_phase[k];
       b.do_tors[k] = do_tors[k] ? 1 : 0;
@@ -1421,31 +1422,37 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     b.want_virial = vir ? 1 : 0;
     b.want_energy = want_energy ? 1 : 0;
   }
+  // The bonded terms, one thread per term, on the first stream ahead of the
+  // lists; the second stream's forces go to an array of their own that the
+  // fold adds, so the two need no order.  (Evaluated per atom in the gather, a
+  // term ran once for each of its atoms, and the FP64 trigonometry held the
+  // gather to 185 VGPRs: 147 us of a 262 us step on a protein of 14,281 atoms.)
+  if (any_bonded) {
+    TimedScope ts(c, PM_T_BONDED);
+    pm_launch_bonded(s, c->box, b);
+  }
   // with one PME reciprocal term, the gather kernel's thread for an atom
-  // also adds that atom's correction and bonded forces (two launches fewer)
+  // also adds that atom's correction force (a launch fewer)
   PmAtomTail tail{};
-  const bool fuse = pme_launch.size() == 1;
+  const bool fuse = pme_launch.size() == 1 && c->forces[pme_launch[0].second].corr;
   if (fuse) {
     const ForceDesc& f = c->forces[pme_launch[0].second];
     tail.box = c->box;
-    if (f.corr) {
-      tail.corr = 1;
-      tail.pos = c->d_pos; tail.q = c->d_q;
-      tail.row = c->d_cx_row; tail.partner = c->d_cx_partner; tail.cls = c->d_cx_cls;
-      tail.alpha = f.alpha; tail.csf = c->csf;
-    }
-    if (any_bonded) {
-      tail.bonded = 1;
-      tail.b = b;
-    }
+    tail.pos = c->d_pos; tail.q = c->d_q;
+    tail.row = c->d_cx_row; tail.partner = c->d_cx_partner; tail.cls = c->d_cx_cls;
+    tail.alpha = f.alpha; tail.csf = c->csf;
   }
   for (auto& pl : pme_launch) {
     TimedScope ts(c, PM_T_PME, s2);
     pm_launch_pme_plans(s2, pl.first, c->plans, c->d_slot_pos64, c->precision, fuse ? &tail : nullptr);
   }
+  // (a correction without a reciprocal term is the array's first writer)
+  bool side_forces = !pme_launch.empty();
   for (auto& hr : pme_rec) {
     ForceDesc& f = c->forces[hr.first];
     if (!f.corr) continue;
+    if (!side_forces) pm_launch_zero_ll(s2, c->d_force_side, 3LL * n);
+    side_forces = true;
     const bool in_tail = fuse && hr.first == pme_launch[0].second;
     long long off = hr.second + (f.recip ? pm_pme_xpass_blocks(f.nx, f.ny, f.nz, c->precision, pme_plane(c, f)) : 0);
     int ntab = (int)c->tab_a.size();
@@ -1453,7 +1460,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     if (in_tail && !want_energy) continue;
     TimedScope ts(c, PM_T_CORR, s2);
     pm_launch_correction(s2, c->box, in_tail ? 0 : n, c->d_pos, c->d_q, c->d_cx_row, c->d_cx_partner, c->d_cx_cls,
-                         f.alpha, c->csf, vir ? 1 : 0, c->d_force, ntab, c->d_tab_a, c->d_tab_b, c->d_tab_c,
+                         f.alpha, c->csf, vir ? 1 : 0, c->d_force_side, ntab, c->d_tab_a, c->d_tab_b, c->d_tab_c,
                          c->d_epart + off * PM_NE, want_energy ? nblk : 0);
   }
   for (auto& hr : pme_rec) {
@@ -1465,12 +1472,6 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     pm_launch_ewald_lattice(s2, c->box, n, c->d_pos, c->d_q, c->d_xs_row, c->d_xs_part, c->d_lat, c->nlat,
                             f.rc * f.rc, f.alpha, c->csf, vir ? 1 : 0, c->d_force, c->d_epart + off * PM_NE,
                             lattice_blocks(n));
-  }
-  if (any_bonded && !(fuse && !want_energy)) {
-    PmBondedLaunch bl = b;
-    if (fuse) bl.n = 0;   // the forces came with the gather: energies only
-    TimedScope ts(c, PM_T_BONDED, s2);
-    pm_launch_bonded(s2, c->box, bl);
   }
   if (side) HIPCHECK(c, hipEventRecord(c->ev_join, s2));
 
@@ -1485,19 +1486,20 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       pm_launch_pair(s, c->box, pl.first, pl.second, c->precision);
     }
   }
-  // join, then the per-slot pair forces into the per-atom forces
+  // join, then the per-slot pair forces and the second stream's into the
+  // per-atom forces
   if (side) HIPCHECK(c, hipStreamWaitEvent(s, c->ev_join, 0));
-  if (!passes.empty()) {
+  if (!passes.empty() || side_forces) {
     TimedScope ts(c, PM_T_BIN);
     // with reuse also the end of the evaluation: the flag's readers all ran
-    pm_launch_fold_slots(s, c->nslot_max, c->d_counts, c->d_atom_of_slot, c->d_force_slot, c->d_force,
+    pm_launch_fold_slots(s, c->nslot_max, c->d_counts, c->d_atom_of_slot, c->d_force_slot,
+                         side_forces ? c->d_force_side : nullptr, c->d_force,
                          reuse ? c->d_rebuild : nullptr, c->d_stats + 2, 1);
   }
   if (want_energy) {
     TimedScope ts(c, PM_T_REDUCE);
     pm_launch_reduce_energy(s, c->d_epart, (int)rec, const_coul, const_vir, c->d_energy, 1, c->d_ered);
   }
-  (void)any_pme_recip;
   HIPCHECK(c, hipGetLastError());
   return PM_OK;
 }
@@ -1684,7 +1686,7 @@ void free_all(pm_context* c) {
   dfree(c->d_cx_row); dfree(c->d_cx_partner); dfree(c->d_cx_cls);
   dfree(c->d_tab_a); dfree(c->d_tab_b); dfree(c->d_tab_c);
   dfree(c->d_lj_f); dfree(c->d_lj_d);
-  dfree(c->d_pos); dfree(c->d_vel); dfree(c->d_force); dfree(c->d_energy); dfree(c->d_scratch3);
+  dfree(c->d_pos); dfree(c->d_vel); dfree(c->d_force); dfree(c->d_force_side); dfree(c->d_energy); dfree(c->d_scratch3);
   dfree(c->d_cell_of); dfree(c->d_key); dfree(c->d_cell_count); dfree(c->d_bin_count); dfree(c->d_cell_start); dfree(c->d_cell_slot);
   dfree(c->d_scan_aux);
   dfree(c->d_xbuild); dfree(c->d_rebuild); c->list_stale = true;
@@ -1700,12 +1702,12 @@ void free_all(pm_context* c) {
   dfree(c->d_lat);
   c->nlat = 0;
   dfree(c->d_bmod); dfree(c->d_expt); dfree(c->d_tw);
-  dfree(c->d_b_a); dfree(c->d_b_b); dfree(c->d_b_row); dfree(c->d_b_idx); dfree(c->d_b_k); dfree(c->d_b_r0);
-  dfree(c->d_a_a); dfree(c->d_a_b); dfree(c->d_a_c); dfree(c->d_a_row); dfree(c->d_a_idx);
+  dfree(c->d_b_a); dfree(c->d_b_b); dfree(c->d_b_k); dfree(c->d_b_r0);
+  dfree(c->d_a_a); dfree(c->d_a_b); dfree(c->d_a_c);
   dfree(c->d_a_k); dfree(c->d_a_t0); dfree(c->d_a_kub); dfree(c->d_a_rub);
   c->nbonds = c->nangles = 0;
   for (int k = 0; k < 2; k++) {
-    dfree(c->d_t_row[k]); dfree(c->d_t_idx[k]); dfree(c->d_t_term[k]); dfree(c->d_t_atoms[k]);
+    dfree(c->d_t_term[k]); dfree(c->d_t_atoms[k]);
     dfree(c->d_t_k[k]); dfree(c->d_t_phase[k]); dfree(c->d_t_n[k]);
     c->ntors[k] = 0;
   }
@@ -1956,6 +1958,7 @@ int pm_set_topology(pm_context* c, int n, const double* q, const int* type, int 
   if ((r = dalloc(c, &c->d_vel, 3 * (size_t)n))) return r;
   HIPCHECK(c, hipMemset(c->d_vel, 0, 3 * (size_t)n * sizeof(double)));
   if ((r = dalloc(c, &c->d_force, 3 * (size_t)n))) return r;
+  if ((r = dalloc(c, &c->d_force_side, 3 * (size_t)n))) return r;
   if ((r = dalloc(c, &c->d_scratch3, 3 * (size_t)n))) return r;
   if ((r = dalloc(c, &c->d_energy, PM_NE))) return r;
   HIPCHECK(c, hipMemset(c->d_energy, 0, PM_NE * sizeof(double)));
@@ -2022,22 +2025,8 @@ int pm_set_bonded(pm_context* c, int nb, const int* ba, const int* bb, const dou
     if (aa[k] < 0 || aa[k] >= n || ab[k] < 0 || ab[k] >= n || ac[k] < 0 || ac[k] >= n ||
         aa[k] == ab[k] || ab[k] == ac[k] || aa[k] == ac[k])
       return fail(c, PM_ERR_ARGUMENT, "angle %d (%d, %d, %d) out of range", k, aa[k], ab[k], ac[k]);
-  // per-atom CSR of the terms each atom belongs to
-  std::vector<int> brow(n + 1, 0), bidx(2 * (size_t)nb), arow(n + 1, 0), aidx(3 * (size_t)na);
-  for (int k = 0; k < nb; k++) { brow[ba[k] + 1]++; brow[bb[k] + 1]++; }
-  for (int k = 0; k < na; k++) { arow[aa[k] + 1]++; arow[ab[k] + 1]++; arow[ac[k] + 1]++; }
-  for (int i = 0; i < n; i++) { brow[i + 1] += brow[i]; arow[i + 1] += arow[i]; }
-  {
-    std::vector<int> fb(brow.begin(), brow.end() - 1), fa(arow.begin(), arow.end() - 1);
-    for (int k = 0; k < nb; k++) { bidx[fb[ba[k]]++] = k; bidx[fb[bb[k]]++] = k; }
-    for (int k = 0; k < na; k++) { aidx[fa[aa[k]]++] = k; aidx[fa[ab[k]]++] = k; aidx[fa[ac[k]]++] = k; }
-  }
   auto vi = [](const int* p, int m) { return std::vector<int>(p, p + m); };
   auto vd = [](const double* p, int m) { return std::vector<double>(p, p + m); };
-  if ((r = upload(c, &c->d_b_row, brow))) return r;
-  if ((r = upload(c, &c->d_b_idx, bidx))) return r;
-  if ((r = upload(c, &c->d_a_row, arow))) return r;
-  if ((r = upload(c, &c->d_a_idx, aidx))) return r;
   if ((r = upload(c, &c->d_b_a, vi(ba, nb)))) return r;
   if ((r = upload(c, &c->d_b_b, vi(bb, nb)))) return r;
   if ((r = upload(c, &c->d_b_k, vd(bk, nb)))) return r;
@@ -2080,20 +2069,8 @@ int pm_set_torsions(pm_context* c, int kind, int nt, const int* atoms, const int
       return fail(c, PM_ERR_ARGUMENT, "torsion %d has no term (term_row must increase)", t);
   }
   const int nterm = nt > 0 ? term_row[nt] : 0;
-  std::vector<int> row(n + 1, 0), idx(4 * (size_t)nt);
   std::vector<int4> at(nt);
-  for (int t = 0; t < nt; t++) {
-    at[t] = make_int4(atoms[4 * t], atoms[4 * t + 1], atoms[4 * t + 2], atoms[4 * t + 3]);
-    for (int j = 0; j < 4; j++) row[atoms[4 * t + j] + 1]++;
-  }
-  for (int i = 0; i < n; i++) row[i + 1] += row[i];
-  {
-    std::vector<int> fill(row.begin(), row.end() - 1);
-    for (int t = 0; t < nt; t++)
-      for (int j = 0; j < 4; j++) idx[fill[atoms[4 * t + j]]++] = t;
-  }
-  if ((r = upload(c, &c->d_t_row[kind], row))) return r;
-  if ((r = upload(c, &c->d_t_idx[kind], idx))) return r;
+  for (int t = 0; t < nt; t++) at[t] = make_int4(atoms[4 * t], atoms[4 * t + 1], atoms[4 * t + 2], atoms[4 * t + 3]);
   if ((r = upload(c, &c->d_t_atoms[kind], at))) return r;
   if ((r = upload(c, &c->d_t_term[kind], std::vector<int>(term_row, term_row + (nt > 0 ? nt + 1 : 0))))) return r;
   if ((r = upload(c, &c->d_t_k[kind], std::vector<double>(k, k + nterm)))) return r;

@@ -6,9 +6,7 @@
 // MTorsionSystemForce::calcTorsion (forces/MTorsionSystemForce.h:34-153) for
 // DihedralSystemForce and ImproperSystemForce.  Forces
 // are computed once per term and added to the atoms as 64-bit fixed-point
-// atomics (deterministic: integer sums do not depend on their order); the
-// PME gather's per-atom tail (pm_terms.h bonded_atom_force) is the other
-// route.  Energies and virials are summed per term in fixed-order block
+// atomics (deterministic: integer sums do not depend on their order).  Energies and virials are summed per term in fixed-order block
 // reductions.
 #include "pm_internal.h"
 #include "pm_terms.h"
@@ -22,8 +20,7 @@ namespace {
 // evaluated once, its forces go to its atoms as 64-bit fixed-point atomic
 // adds (integer addition is associative, so the sums do not depend on the
 // order of the atomics), and with want_energy the block writes one energy /
-// virial record.  a.n == 0 leaves the forces alone (the PME gather added
-// them per atom).
+// virial record.
 struct BondedBlocks { int off[5]; };
 __device__ inline void add_fix(long long* f, int i, const double* v, double sg, int* err) {
   for (int c = 0; c < 3; c++)
@@ -94,7 +91,7 @@ __device__ inline void bonded_terms_body(PmBox box, PmBondedLaunch a, BondedBloc
     }
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (a.n > 0) {   // uniform over the launch
+  {
     // the block's atom window
     int lo = 0x7fffffff, hi = -1;
     if (have)
@@ -189,13 +186,11 @@ void pm_launch_bonded(hipStream_t s, const PmBox& box, const PmBondedLaunch& a) 
   BondedBlocks bl;
   bl.off[0] = 0;
   for (int k = 0; k < 4; k++) bl.off[k + 1] = bl.off[k] + nblk[k];
-  // nothing to do when neither forces (a.n > 0) nor energies are wanted
-  const bool work = a.n > 0 || a.want_energy;
   const BondedTermArgs q{box, a, bl};
   const int groups[3] = {0, 2, 3};
   const int gblocks[3] = {nblk[0] + nblk[1], nblk[2], nblk[3]};
   for (int g = 0; g < 3; g++) {
-    const unsigned blocks = work ? (unsigned)gblocks[g] : 0u;
+    const unsigned blocks = (unsigned)gblocks[g];
     if (pm_recording()) {
       pm_record(PM_REC_BONDED_FORCE, groups[g], blocks, 256, 0, &q, sizeof(q));
       continue;

@@ -205,12 +205,12 @@ void pm_launch_check_disp(hipStream_t s, const PmBox& box, int n, const double* 
                           float lim2, int* flag, const int4* x_prune = nullptr, float lim2_in = 0.f);
 void pm_launch_set_flag(hipStream_t s, int* flag, int v);
 void pm_launch_invalidate_build(hipStream_t s, int n, int4* x_build);
-// force_fix[atom] += force_slot[slot] for every real slot (then the slot
-// cleared when `clear`); with `flag` (list reuse) also the end of the
+// force_fix[atom] += force_slot[slot] (+ force_pme[atom], may be null) for
+// every real slot (then the slot cleared when `clear`); with `flag` (list reuse) also the end of the
 // evaluation: builds[0] += (flag[0] != 0), builds[1] += (only flag[1] != 0:
 // an inner-list prune without a build), flag[0] = flag[1] = 0
 void pm_launch_fold_slots(hipStream_t s, int nslot_max, const int* counts, const int* atom_of_slot,
-                          long long* force_slot, long long* force_fix, int* flag,
+                          long long* force_slot, const long long* force_pme, long long* force_fix, int* flag,
                           unsigned long long* builds, int clear);
 // entries and issued lanes of the lists whose lengths are `jcount`
 void pm_launch_list_stats(hipStream_t s, const int* jcount, const int* counts, unsigned long long* out, int m,
@@ -255,7 +255,8 @@ struct PmPmeLaunch {
   double fac;                // pi^2/alpha^2
   double Lr[3];              // 1/L
   const double* tw;          // twiddles exp(-2 pi i m/n), interleaved re, im
-  long long* force_fix;
+  long long* force_fix;      // [3n] the gather writes every atom's force
+  int accumulate;            // 1: the gather adds to force_fix (a later term of several)
   double* epart;             // [pm_pme_xpass_blocks() * PM_NE]
   int want_virial;
   int want_energy;           // 0: no energy records (then neither is the virial wanted)
@@ -290,8 +291,8 @@ struct PmFftPlan {
   int tw;  // offset of this length's twiddles in the table (complex entries)
 };
 struct PmAtomTail;
-// spread, transforms and gather; tail (may be null) adds the correction and
-// bonded forces of each atom in the gather kernel's thread for that atom
+// spread, transforms and gather; tail (may be null) adds the correction force
+// of each atom in the gather kernel's thread for that atom
 bool pm_launch_pme_plans(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans,
                          const longlong4* pos64, int precision, const PmAtomTail* tail);
 // the lines along y (4, 2 or 1) of a k_spread_zfwd block whose 4 x ly z
@@ -414,22 +415,17 @@ bool pm_launch_constraints(hipStream_t s, const PmConstraints& c, int rattle, do
 int pm_scratch_init(int device);
 void* pm_scratch_address(int device);
 
-// Bonded terms (Bond / Angle system forces), per-atom gather formulation
+// Bonded terms (Bond, Angle, Dihedral and Improper system forces)
 struct PmBondedLaunch {
-  int n;
   const double* pos;
-  // per-atom CSR of the bonds and angles an atom belongs to
-  const int* b_row; const int* b_idx;     // bond index
-  const int* a_row; const int* a_idx;     // angle index
   int nb, na;
   const int* b_a; const int* b_b; const double* b_k; const double* b_r0;
   const int* a_a; const int* a_b; const int* a_c; const double* a_k; const double* a_t0;
   const double* a_kub; const double* a_rub;
   int do_bond, do_angle;
-  // torsions, kind 0 dihedrals and kind 1 impropers: per-atom CSR of the
-  // torsions an atom belongs to, the four atoms, and each torsion's terms
-  // term[t] .. term[t+1]-1 (force constant, periodicity, phase in radians)
-  const int* t_row[2]; const int* t_idx[2];
+  // torsions, kind 0 dihedrals and kind 1 impropers: the four atoms, and each
+  // torsion's terms term[t] .. term[t+1]-1 (force constant, periodicity, phase
+  // in radians)
   int nt[2];
   const int4* t_atoms[2]; const int* t_term[2];
   const double* t_k[2]; const int* t_n[2]; const double* t_phase[2];
@@ -443,18 +439,15 @@ struct PmBondedLaunch {
 void pm_bonded_blocks(const PmBondedLaunch& a, int nblk[4]);
 void pm_launch_bonded(hipStream_t s, const PmBox& box, const PmBondedLaunch& a);
 
-// Per-atom force terms that the PME gather kernel adds for its atoms, each
-// rounded to fixed point on its own as the separate kernels round it (the
-// integer sum is then the same as theirs).
+// The PME excluded-pair correction that the gather kernel adds for its atoms,
+// rounded to fixed point on its own as the separate kernel rounds it (the
+// integer sum is then the same).
 struct PmAtomTail {
   PmBox box;
-  int corr;                    // PME excluded-pair correction
   const double* pos;
   const double* q;
   const int* row; const int* partner; const int* cls;
   double alpha, csf;
-  int bonded;                  // bonded terms (b.do_bond / do_angle / do_tors)
-  PmBondedLaunch b;
 };
 
 // ------------------------------------------------- batched launch records

@@ -827,8 +827,9 @@ __global__ __launch_bounds__(256) void k_list_stats(const int* __restrict__ jcou
 
 // slot forces of the pair kernels into the per-atom fixed-point forces
 __device__ inline void fold_slots_body(const int* __restrict__ counts, const int* __restrict__ atom_of_slot,
-                             long long* __restrict__ force_slot, long long* __restrict__ force_fix,
-                             int* __restrict__ flag, unsigned long long* __restrict__ builds, int clear, int bx) {
+                             long long* __restrict__ force_slot, const long long* __restrict__ force_pme,
+                             long long* __restrict__ force_fix, int* __restrict__ flag,
+                             unsigned long long* __restrict__ builds, int clear, int bx) {
   if (flag && bx == 0 && threadIdx.x == 0) {
     // end of an evaluation that reuses lists (every reader of the flags ran
     // before): count a build or a prune of the inner lists, clear the flags
@@ -841,9 +842,15 @@ __device__ inline void fold_slots_body(const int* __restrict__ counts, const int
   if (sl >= counts[0]) return;
   const int at = atom_of_slot[sl];
   if (at < 0) return;
-  force_fix[3LL * at] += force_slot[3LL * sl];
-  force_fix[3LL * at + 1] += force_slot[3LL * sl + 1];
-  force_fix[3LL * at + 2] += force_slot[3LL * sl + 2];
+  long long f[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) f[k] = force_fix[3LL * at + k] + force_slot[3LL * sl + k];
+  if (force_pme) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) f[k] += force_pme[3LL * at + k];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; k++) force_fix[3LL * at + k] = f[k];
   if (clear) {
     // the next evaluation's pair kernels start from zero (only real slots
     // ever receive pair forces)
@@ -853,15 +860,16 @@ __device__ inline void fold_slots_body(const int* __restrict__ counts, const int
   }
 }
 __global__ void k_fold_slots(const int* __restrict__ counts, const int* __restrict__ atom_of_slot,
-                             long long* __restrict__ force_slot, long long* __restrict__ force_fix,
-                             int* __restrict__ flag, unsigned long long* __restrict__ builds, int clear) {
-  fold_slots_body(counts, atom_of_slot, force_slot, force_fix, flag, builds, clear, blockIdx.x);
+                             long long* __restrict__ force_slot, const long long* __restrict__ force_pme,
+                             long long* __restrict__ force_fix, int* __restrict__ flag,
+                             unsigned long long* __restrict__ builds, int clear) {
+  fold_slots_body(counts, atom_of_slot, force_slot, force_pme, force_fix, flag, builds, clear, blockIdx.x);
 }
-struct FoldSlotsArgs { const int* counts; const int* atom_of_slot; long long* force_slot; long long* force_fix; int* flag; unsigned long long* builds; int clear; };
+struct FoldSlotsArgs { const int* counts; const int* atom_of_slot; long long* force_slot; const long long* force_pme; long long* force_fix; int* flag; unsigned long long* builds; int clear; };
 __global__ void kb_fold_slots(const FoldSlotsArgs* __restrict__ t, const int* __restrict__ pre, int nrep) {
   const int r = pm_batch_replica(pre, nrep, blockIdx.x);
   const FoldSlotsArgs& q = t[r];
-  fold_slots_body(q.counts, q.atom_of_slot, q.force_slot, q.force_fix, q.flag, q.builds, q.clear, blockIdx.x - pre[r]);
+  fold_slots_body(q.counts, q.atom_of_slot, q.force_slot, q.force_pme, q.force_fix, q.flag, q.builds, q.clear, blockIdx.x - pre[r]);
 }
 
 
@@ -2158,16 +2166,16 @@ void pm_launch_invalidate_build(hipStream_t s, int n, int4* x_build) {
 }
 
 void pm_launch_fold_slots(hipStream_t s, int nslot_max, const int* counts, const int* atom_of_slot,
-                          long long* force_slot, long long* force_fix, int* flag,
+                          long long* force_slot, const long long* force_pme, long long* force_fix, int* flag,
                           unsigned long long* builds, int clear) {
   if (pm_recording()) {
-    const FoldSlotsArgs a{counts, atom_of_slot, force_slot, force_fix, flag, builds, clear};
+    const FoldSlotsArgs a{counts, atom_of_slot, force_slot, force_pme, force_fix, flag, builds, clear};
     pm_record(PM_REC_FOLD_SLOTS, 0, nslot_max > 0 ? (nslot_max + 255) / 256 : 0, 256, 0, &a, sizeof(a));
     return;
   }
   if (nslot_max > 0)
     hipLaunchKernelGGL(k_fold_slots, dim3((nslot_max + 255) / 256), dim3(256), 0, s, counts, atom_of_slot,
-                       force_slot, force_fix, flag, builds, clear);
+                       force_slot, force_pme, force_fix, flag, builds, clear);
 }
 
 void pm_launch_prune(hipStream_t s, const PmBox& box, const PmNbLaunch& a) {

@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256) void k_spread_tile(PmPmeLaunch a, const longlo
   }
 }
 
-// TAIL: the same thread also adds its atom's correction and bonded forces
+// TAIL: the same thread also adds its atom's correction force
 template <typename T, int P, bool TAIL>
 __global__ __launch_bounds__(256) void k_gather(PmPmeLaunch a, const longlong4* __restrict__ pos64, PmAtomTail tl) {
   pme_priority(a.prio);
@@ -482,18 +482,14 @@ __global__ __launch_bounds__(256) void k_gather(PmPmeLaunch a, const longlong4* 
                     pm_force_fix((double)fz * a.hr[2] * q, a.err)};
   if (TAIL) {
     double f[3];
-    if (tl.corr) {
-      corr_atom_force(tl.box, at, tl.pos, tl.q, tl.row, tl.partner, tl.cls, tl.alpha, tl.csf, f);
-      for (int k = 0; k < 3; k++) F[k] += pm_force_fix(f[k], a.err);
-    }
-    if (tl.bonded) {
-      bonded_atom_force(tl.box, tl.b, at, f);
-      for (int k = 0; k < 3; k++) F[k] += pm_force_fix(f[k], a.err);
-    }
+    corr_atom_force(tl.box, at, tl.pos, tl.q, tl.row, tl.partner, tl.cls, tl.alpha, tl.csf, f);
+    for (int k = 0; k < 3; k++) F[k] += pm_force_fix(f[k], a.err);
   }
-  a.force_fix[3 * at] += F[0];
-  a.force_fix[3 * at + 1] += F[1];
-  a.force_fix[3 * at + 2] += F[2];
+  if (a.accumulate)
+    for (int k = 0; k < 3; k++) F[k] += a.force_fix[3 * at + k];
+  a.force_fix[3 * at] = F[0];
+  a.force_fix[3 * at + 1] = F[1];
+  a.force_fix[3 * at + 2] = F[2];
 }
 
 // ---------------------------------------------------------- PME adjoint

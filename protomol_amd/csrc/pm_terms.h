@@ -184,38 +184,4 @@ __device__ inline void corr_atom_force(const PmBox& box, int i, const double* __
   }
 }
 
-// Bond and angle forces on atom i: each term it belongs to, its own share.
-__device__ inline void bonded_atom_force(const PmBox& box, const PmBondedLaunch& a, int i, double* f) {
-  f[0] = f[1] = f[2] = 0.0;
-  if (a.do_bond) {
-    for (int u = a.b_row[i]; u < a.b_row[i + 1]; u++) {
-      const int k = a.b_idx[u];
-      double f1[3], e, r12[3];
-      bond_term(box, a, k, f1, e, r12);
-      const double sg = (a.b_a[k] == i) ? 1.0 : -1.0;
-      f[0] += sg * f1[0]; f[1] += sg * f1[1]; f[2] += sg * f1[2];
-    }
-  }
-  if (a.do_angle) {
-    for (int u = a.a_row[i]; u < a.a_row[i + 1]; u++) {
-      const int k = a.a_idx[u];
-      double f1[3], f2[3], f3[3], e, r12[3], r32[3];
-      angle_term(box, a, k, f1, f2, f3, e, r12, r32);
-      const double* g = (a.a_a[k] == i) ? f1 : (a.a_b[k] == i) ? f2 : f3;
-      f[0] += g[0]; f[1] += g[1]; f[2] += g[2];
-    }
-  }
-  for (int kind = 0; kind < 2; kind++) {
-    if (!a.do_tors[kind]) continue;
-    for (int u = a.t_row[kind][i]; u < a.t_row[kind][i + 1]; u++) {
-      const int t = a.t_idx[kind][u];
-      double f1[3], f2[3], f3[3], e, r12[3], r23[3], r34[3];
-      torsion_term(box, a, kind, t, f1, f2, f3, e, r12, r23, r34);
-      const int4 at = a.t_atoms[kind][t];
-      for (int c = 0; c < 3; c++)
-        f[c] += (at.x == i) ? f1[c] : (at.y == i) ? f2[c] - f1[c] : (at.z == i) ? f3[c] - f2[c] : -f3[c];
-    }
-  }
-}
-
 }  // namespace
