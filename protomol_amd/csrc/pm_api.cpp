@@ -32,6 +32,8 @@
 // inner skin almost every step, and the prune pass costs more than the
 // 20-25 % of pair lanes it saves)
 #define PM_PRUNE_SKIN_AUTO 0.0
+// waves up to which a cluster's list is shared by several (pair_split)
+#define PM_SPLIT_WAVES 1024
 
 // launch recorder of the calling thread (replica batches)
 static thread_local std::vector<PmRecord>* g_recorder = nullptr;
@@ -151,6 +153,7 @@ struct pm_context {
   int *d_ex_row = nullptr, *d_ex_partner = nullptr, *d_ex_cls = nullptr;      // lookup CSR
   int *d_xs_row = nullptr, *d_xs_part = nullptr;   // resolved exclusions, both directions
   int xs_maxdeg = 0;
+  unsigned long long lj_types = 0;   // bit t: type t has Lennard-Jones parameters with some type
   int *d_cx_row = nullptr, *d_cx_partner = nullptr, *d_cx_cls = nullptr;      // correction CSR
   int *d_tab_a = nullptr, *d_tab_b = nullptr, *d_tab_c = nullptr;
   float4* d_lj_f = nullptr;
@@ -199,7 +202,7 @@ struct pm_context {
   std::map<double, std::pair<int4*, int>> half_stencils;
 
   // lists
-  int *d_jlist = nullptr, *d_jcount = nullptr, *d_overflow = nullptr;
+  int *d_jlist = nullptr, *d_jcount = nullptr, *d_jnear = nullptr, *d_overflow = nullptr;
   unsigned int* d_jmask = nullptr;     // per list entry: FULL / MODIFIED masks of flagged entries
   long long jlist_alloc = 0;
   int lcap = 0;
@@ -497,8 +500,47 @@ double prune_skin(const pm_context* c) {
 // option asks for rows (0) or its LDS (type table + four waves' areas) would
 // not fit a workgroup (FP64 with over 41 atom types)
 static int pair_lanes(const pm_context* c) {
-  const size_t tab = (size_t)(c->ntypes + 1) * (c->ntypes + 1) * (c->precision == PM_PRECISION_DOUBLE ? 32 : 16);
-  return c->pair_lanes_option && (tab + 15) / 16 * 16 + 4 * PM_JL_LDS <= (size_t)c->lds_max ? 1 : 0;
+  const bool dbl = c->precision == PM_PRECISION_DOUBLE;
+  const size_t tab = (size_t)(c->ntypes + 1) * (c->ntypes + 1) * (dbl ? 32 : 16);
+  const size_t area = dbl ? PM_JL_LDS(double) : PM_JL_LDS(float);
+  return c->pair_lanes_option && (tab + 15) / 16 * 16 + (dbl ? PM_JL_WAVES(double) : PM_JL_WAVES(float)) * area <= (size_t)c->lds_max ? 1 : 0;
+}
+
+// Whether the context's MD run is one that a batch can hold (Langevin, no
+// PME).  Replicas walk their lists unsorted with one wave per cluster, alone
+// as in a batch: their boxes share the chip, so that more waves only cost, and
+// a hot box amplifies a change of the summation order 20,000 times in 50
+// steps; this order gives the same trajectory alone and in a batch.
+static bool replica_form(const pm_context* c) {
+  if (c->md_handles.empty() || c->md_integrator != PM_INTEGRATOR_LANGEVIN) return false;
+  for (int h : c->md_handles)
+    if (c->forces[h].pme) return false;
+  return true;
+}
+
+// log2 of the waves per cluster of the lane-per-entry kernel: a box of few
+// clusters leaves the chip idle while each wave walks its list alone (648
+// atoms, 25 FP64 steps: 1.75 ms with one wave per cluster, 1.28 at most 512
+// waves, 1.20 at 1024 and at 4096; a batch of 64 replicas, 50 steps: 22.3 ms
+// with one, 22.4 at 512 waves, 22.7 at 1024 and 29 at 4096)
+static int pair_split(const pm_context* c) {
+  if (replica_form(c)) return 0;
+  int s = 0;
+  while (s < 3 && ((long long)c->ncl_max << (s + 1)) <= PM_SPLIT_WAVES) s++;
+  return s;
+}
+
+// The types with Lennard-Jones parameters, for the pair kernel to leave the
+// others' terms out.  With an uncharged atom every type counts: two atoms on
+// one point then still show as a force that is not finite.
+static void set_lj_types(pm_context* c) {
+  c->lj_types = 0;
+  const int T = c->ntypes;
+  for (int a = 0; a < T; a++)
+    for (int b = 0; b < T; b++)
+      for (int k : {a * T + b, b * T + a})
+        if (c->ljA[k] != 0.0 || c->ljB[k] != 0.0 || c->ljA14[k] != 0.0 || c->ljB14[k] != 0.0) c->lj_types |= 1ull << (a & 63);
+  if (std::find(c->q.begin(), c->q.end(), 0.0) != c->q.end()) c->lj_types = ~0ull;
 }
 
 // list skin in A: the option, or the automatic choice
@@ -577,6 +619,7 @@ int ensure_lists(pm_context* c, int lcap) {
   if ((r = dalloc(c, &c->d_jlist, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jmask, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jcount, c->ncl_max))) return r;
+  if ((r = dalloc(c, &c->d_jnear, c->ncl_max))) return r;
   c->jlist_alloc = need;
   c->lcap = lcap;
   return PM_OK;
@@ -1168,7 +1211,9 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   }
 
   // energy records: pair passes, PME x-pass blocks, correction blocks
-  long long rec = (long long)passes.size() * c->ncl_max;
+  const int slog = pair_split(c);
+  const long long pair_rec = (long long)c->ncl_max << (pair_lanes(c) ? slog : 0);
+  long long rec = (long long)passes.size() * pair_rec;
   std::vector<std::pair<int, long long>> pme_rec;   // (handle, offset)
   for (int h : handles) {
     ForceDesc& f = c->forces[h];
@@ -1240,6 +1285,9 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.xs_tcap = c->m * c->xs_maxdeg;
     a.m = c->m;
     a.jlanes = pair_lanes(c);
+    a.split_log = adj ? 0 : slog;
+    a.near_margin = replica_form(c) ? PM_NEAR_ALL : PM_NEAR_MARGIN;
+    a.lj_types = c->lj_types;
     a.molecule = c->d_mol;
     a.ex_row = c->d_ex_row;
     a.ex_partner = c->d_ex_partner;
@@ -1251,7 +1299,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.atom_lj_d = c->d_atom_lj_d;
     a.force_fix = c->d_force;
     a.force_slot = c->d_force_slot;
-    a.epart = c->d_epart + (long long)pi * c->ncl_max * PM_NE;
+    a.epart = c->d_epart + (long long)pi * pair_rec * PM_NE;
     a.want_virial = vir ? 1 : 0;
     a.want_energy = want_energy ? 1 : 0;
   }
@@ -1260,6 +1308,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     pl.first.jlist = c->d_jlist;
     pl.first.jmask = c->d_jmask;
     pl.first.jcount = c->d_jcount;
+    pl.first.jnear = c->d_jnear;
     pl.first.lcap = c->lcap;
     if (inner) {
       // the pair cutoff + the inner skin, padded as the list cutoff is
@@ -1693,7 +1742,7 @@ void free_all(pm_context* c) {
   dfree(c->d_xprune); dfree(c->d_ilist); dfree(c->d_imask); dfree(c->d_icount); c->ilist_alloc = 0;
   dfree(c->d_cell_rank); dfree(c->d_force_slot); dfree(c->d_cell_atoms); dfree(c->d_cluster_cell); dfree(c->d_counts);
   dfree(c->d_slot_pos); dfree(c->d_slot_pos64); dfree(c->d_slot_meta); dfree(c->d_atom_of_slot);
-  dfree(c->d_jlist); dfree(c->d_jcount); dfree(c->d_stats); dfree(c->d_epart); dfree(c->d_ered);
+  dfree(c->d_jlist); dfree(c->d_jcount); dfree(c->d_jnear); dfree(c->d_stats); dfree(c->d_epart); dfree(c->d_ered);
   dfree(c->d_grid_fix);
   if (c->d_grid_r) hipFree(c->d_grid_r);
   if (c->d_grid_c) hipFree(c->d_grid_c);
@@ -1929,6 +1978,7 @@ int pm_set_topology(pm_context* c, int n, const double* q, const int* type, int 
     }
   }
   // LJ tables with one extra all-zero type for padding slots
+  set_lj_types(c);
   int t1 = ntypes + 1;
   std::vector<float4> ljf(t1 * t1, make_float4(0, 0, 0, 0));
   std::vector<double4> ljd(t1 * t1, make_double4(0, 0, 0, 0));
@@ -2829,6 +2879,9 @@ int pm_set_charges(pm_context* c, const double* q) {
   for (int i = 0; i < c->n; i++)
     if (!std::isfinite(q[i])) return fail(c, PM_ERR_ARGUMENT, "charge %d is not finite", i);
   c->q.assign(q, q + c->n);
+  const unsigned long long types = c->lj_types;
+  set_lj_types(c);
+  if (c->lj_types != types) c->gen++;   // a kernel argument of captured MD steps
   // same size: the copy keeps the device address, so captured MD steps stay valid
   HIPCHECK(c, hipMemcpy(c->d_q, c->q.data(), c->q.size() * sizeof(double), hipMemcpyHostToDevice));
   c->md_forces_valid = false;

@@ -49,9 +49,19 @@
 #define PM_E_VIR 7
 #define PM_NE 16
 // LDS bytes per wave of the lane-per-entry pair kernel (k_pair_jl), after
-// the block's LJ type table: small, so that the kernel leaves most of a CU's
-// LDS to the PME kernels that run beside it on the other stream
-#define PM_JL_LDS 2048
+// the block's LJ type table (the 64 entries' j forces and slots of an
+// iteration, the cluster's box): small, so that the kernel leaves most of a
+// CU's LDS to the PME kernels that run beside it on the other stream
+#define PM_JL_LDS(T) (3 * 64 * sizeof(T) + 64 * sizeof(int) + 8 * sizeof(T))
+// Waves per block of k_pair_jl at most, and the launches (waves) that take them
+#define PM_JL_WAVES(T) (sizeof(T) == 4 ? 8 : 4)
+#define PM_JL_WIDE_MAX 32768
+// List entries within the pair cutoff + this many A of the cluster at the
+// build are near ones: the motion between two builds rarely takes a pair
+// beyond it (98k water: a hydrogen moves 0.2-0.3 A over the nine steps)
+#define PM_NEAR_MARGIN 0.5
+// lists in one group, in the order of the cells
+#define PM_NEAR_ALL 1e9
 
 // Error flags the kernels raise in the context's flag word (atomicOr); the
 // host reads and clears the word after each evaluation or MD run and turns a
@@ -127,6 +137,8 @@ struct PmNbLaunch {
   // lists
   int* jlist;
   int* jcount;
+  double near_margin;        // a near entry is within the pair cutoff + this much of the cluster
+  int* jnear;                // how many of a list's entries are near ones (they come first)
   int lcap;
   int* overflow;
   int bbox_filter;
@@ -137,6 +149,8 @@ struct PmNbLaunch {
   int xs_tcap;               // LDS entries per cluster: M * largest partner count
   unsigned int* jmask;       // per list entry (flagged entries): FULL bit ii, MODIFIED bit 16 + ii
   int m;                     // atoms per cluster (4 or 8)
+  int split_log;             // log2 of the waves per cluster of k_pair_jl and k_adjoint
+  unsigned long long lj_types;  // bit t % 64: type t has Lennard-Jones parameters with some type
   int jlanes;                // pair kernel: 1 one lane per list entry (k_pair_jl), 0 rows of m lanes (k_pair)
   // topology
   const int* molecule;

@@ -10,6 +10,7 @@
 #include "pm_step.h"
 
 #include <math.h>
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -516,11 +517,20 @@ __device__ inline int wrap_cell(int c, int d, int n) {
 // kernel keeps a pair only when the j slot follows the i slot, so every
 // unordered pair within the cutoff is listed exactly once.  Bit 31 marks an
 // entry that some cluster atom excludes or modifies; its masks (FULL bit ii,
-// MODIFIED bit 16 + ii) go to jmask.  BB: 1 the bounding-box test, 0 the
+// MODIFIED bit 16 + ii) go to jmask.  The cluster's own slots carry FULL bits
+// for the atoms from themselves on, which states the half-list rule for them
+// (all other entries lie after the whole cluster).
+// The entries stand in two groups: the near ones (within cut2_near of the
+// cluster at the build) from the list's start, the far ones, which only the
+// skin keeps, from its end backwards (list_at).  A far entry comes within
+// the cutoff only after some tenths of an Angstrom of motion, so the pair
+// kernel drops nearly every iteration of them after one box test; mixed into
+// one order they shared their iterations with pairs within the cutoff and
+// cost as much.  BB: 1 the bounding-box test, 0 the
 // exact per-atom test, 2 the one a.bbox_filter names (batched launches, whose
 // replicas may differ)
 template <int M, int BB>
-__device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, int bx) {
+__device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, float cut2_near, int bx) {
   const bool bbox = BB == 2 ? a.bbox_filter != 0 : BB == 1;
   if (a.rebuild && *a.rebuild == 0) return;   // lists kept from the last build
   extern __shared__ int s_dyn[];
@@ -705,7 +715,7 @@ __device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, int b
 
   int* out = a.jlist + (long long)cl * a.lcap;
   unsigned int* outm = a.jmask + (long long)cl * a.lcap;
-  int count = 0;
+  int count = 0, far = 0;   // near and far entries so far (uniform)
   // candidates beyond PM_CAND_FACTOR * lcap mean a degenerate cell layout:
   // stop scanning and report it as a list overflow
   const int scan = min(total, PM_CAND_FACTOR * a.lcap);
@@ -718,7 +728,7 @@ __device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, int b
     int s = scur;
     for (int t = scur + 1; t < nact && s_pref[t] <= k0 + 63; t++)
       if (k >= s_pref[t]) s = t;
-    bool pass = false;
+    bool pass = false, near = true;
     int sj = 0, o = 0;
     if (k < scan) {
       sj = s_start[s] + (k - s_pref[s]);
@@ -731,20 +741,24 @@ __device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, int b
         const float gx = fmaxf(0.f, fmaxf(lox - dx, dx - hix));
         const float gy = fmaxf(0.f, fmaxf(loy - dy, dy - hiy));
         const float gz = fmaxf(0.f, fmaxf(loz - dz, dz - hiz));
-        pass = loose || gx * gx + gy * gy + gz * gz < cut2_list;
+        const float g2 = gx * gx + gy * gy + gz * gz;
+        pass = loose || g2 < cut2_list;
+        near = g2 < cut2_near;
       } else {
         // box too small for the bounding-box test: keep the entry when one
         // of the cluster's atoms lies within the list cutoff, by the pair
         // kernel's own minimal-image difference (the cluster's positions
         // are wave-uniform loads)
-        pass = false;
+        float g2 = 3.0e38f;
 #pragma unroll
         for (int ii = 0; ii < M; ii++) {
           const float dx = (float)(int)(p.x - qx[ii]) * fx;
           const float dy = (float)(int)(p.y - qy[ii]) * fy;
           const float dz = (float)(int)(p.z - qz[ii]) * fz;
-          pass = pass || (((qreal >> ii) & 1u) && dx * dx + dy * dy + dz * dz < cut2_list);
+          if ((qreal >> ii) & 1u) g2 = fminf(g2, dx * dx + dy * dy + dz * dz);
         }
+        pass = g2 < cut2_list;
+        near = g2 < cut2_near;
       }
       o = (a.slot_meta[sj] >> 8) & 0x7fffff;
     }
@@ -768,28 +782,45 @@ __device__ inline void list_body(PmBox box, PmNbLaunch a, float cut2_list, int b
         }
       }
     }
-    const unsigned long long bal = __ballot(pass);
-    const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
-    const int idx = count + before;
-    if (pass && idx < a.lcap) {
+    // half-list rule within the cluster: atom ii pairs with later slots only
+    const int d = sj - first;
+    if (pass && d < M) {
+      const int own = ((1 << M) - 1) & ~((1 << d) - 1);
+      xm = (xm & ~(own << 16)) | own;
+    }
+    const unsigned long long bn = __ballot(pass && near), bf = __ballot(pass && !near);
+    const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(bn >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bn, 0));
+    const int fbefore = __builtin_amdgcn_mbcnt_hi((unsigned)(bf >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bf, 0));
+    const int pos = near ? count + before : far + fbefore;   // place in its group
+    if (pass && pos < a.lcap) {
+      const int idx = near ? pos : a.lcap - 1 - pos;
       out[idx] = sj | (xm != 0 ? (int)0x80000000 : 0);
       if (xm != 0) outm[idx] = (unsigned int)xm;
     }
-    count += __popcll(bal);
+    count += __popcll(bn);
+    far += __popcll(bf);
   }
   if (lane == 0) {
-    if (count > a.lcap) { atomicOr(a.overflow, PM_FLAG_CAPACITY); count = a.lcap; }
-    a.jcount[cl] = count;
+    if (count + far > a.lcap) {
+      atomicOr(a.overflow, PM_FLAG_CAPACITY);
+      count = min(count, a.lcap);
+      far = a.lcap - count;
+    }
+    a.jcount[cl] = count + far;
+    a.jnear[cl] = count;
   }
 }
+// Place in the list's storage of entry p of a list of which the first `near`
+// entries are the near ones.
+__device__ inline int list_at(int p, int near, int lcap) { return p < near ? p : lcap - 1 - (p - near); }
 template <int M, int BB>
-__global__ __launch_bounds__(256) void k_list(PmBox box, PmNbLaunch a, float cut2_list) { list_body<M, BB>(box, a, cut2_list, blockIdx.x); }
-struct ListArgs { PmBox box; PmNbLaunch a; float cut2_list; };
+__global__ __launch_bounds__(256) void k_list(PmBox box, PmNbLaunch a, float cut2_list, float cut2_near) { list_body<M, BB>(box, a, cut2_list, cut2_near, blockIdx.x); }
+struct ListArgs { PmBox box; PmNbLaunch a; float cut2_list; float cut2_near; };
 template <int M>
 __global__ __launch_bounds__(256) void kb_list(const ListArgs* __restrict__ t, const int* __restrict__ pre, int nrep) {
   const int r = pm_batch_replica(pre, nrep, blockIdx.x);
   const ListArgs& q = t[r];
-  list_body<M, 2>(q.box, q.a, q.cut2_list, blockIdx.x - pre[r]);
+  list_body<M, 2>(q.box, q.a, q.cut2_list, q.cut2_near, blockIdx.x - pre[r]);
 }
 
 
@@ -898,11 +929,11 @@ __device__ inline void prune_body(const PmBox& box, const PmNbLaunch& a, int bx)
   const float sx = (float)box.fix_to_A[0], sy = (float)box.fix_to_A[1], sz = (float)box.fix_to_A[2];
   const long long lbase = (long long)cl * a.lcap;
   const int* __restrict__ lst = a.jlist + lbase;
-  const int cnt = a.jcount[cl];
+  const int cnt = a.jcount[cl], near = a.jnear[cl];
   int icnt = 0;   // wave-uniform
   for (int base = 0; base < cnt; base += JW) {
-    const int k = base + js;
-    const bool valid = k < cnt;
+    const bool valid = base + js < cnt;
+    const int k = list_at(base + js, near, a.lcap);
     const int e = valid ? lst[k] : a.dummy_slot;
     const int sj = e & 0x7fffffff;
     const int4 pj = a.slot_pos[sj];
@@ -1153,6 +1184,7 @@ __device__ inline void pair_cluster(const PmBox& box, const PmNbLaunch& a, const
   const int* __restrict__ lst = (a.inner ? a.ilist : a.jlist) + lbase;
   const unsigned int* __restrict__ msk = (a.inner ? a.imask : a.jmask) + lbase;
   const int cnt = a.inner ? a.icount[cl] : a.jcount[cl];
+  const int near = a.inner ? cnt : a.jnear[cl];
   const int last = cnt > 0 ? cnt - 1 : 0;
   const bool vir = WE && a.want_virial != 0;
   long long* __restrict__ ff = a.force_slot;
@@ -1163,8 +1195,8 @@ __device__ inline void pair_cluster(const PmBox& box, const PmNbLaunch& a, const
   // in flight, and the other way round, so no register copies carry values
   // across the loop; the trip's two rows share one atomic instruction.  Loads
   // past the list's end re-read its last entry (masked), so no load branches.
-  int eA = cnt > 0 ? lst[min(js, last)] : a.dummy_slot;
-  int eB = cnt > 0 ? lst[min(js + JW, last)] : a.dummy_slot;
+  int eA = cnt > 0 ? lst[list_at(min(js, last), near, a.lcap)] : a.dummy_slot;
+  int eB = cnt > 0 ? lst[list_at(min(js + JW, last), near, a.lcap)] : a.dummy_slot;
   P4 pA = spos[eA & 0x7fffffff];
   int mA = a.slot_meta[eA & 0x7fffffff];
   P4 pB;
@@ -1193,7 +1225,7 @@ __device__ inline void pair_cluster(const PmBox& box, const PmNbLaunch& a, const
     bool modified = false, any_mod = false;
     if (__ballot(flagged) != 0ull) {
       if (flagged && mask) {
-        const int xm = (int)msk[k];
+        const int xm = (int)msk[list_at(k, near, a.lcap)];
         if ((xm >> ii) & 1) mask = false;
         else modified = ((xm >> (16 + ii)) & 1) != 0;
       }
@@ -1299,14 +1331,14 @@ __device__ inline void pair_cluster(const PmBox& box, const PmNbLaunch& a, const
     const int eA_now = eA;
     pB = spos[eB & 0x7fffffff];
     mB = a.slot_meta[eB & 0x7fffffff];
-    eA = lst[min(kA + 2 * JW, last)];
+    eA = lst[list_at(min(kA + 2 * JW, last), near, a.lcap)];
     int sA;
     const T vA = row(kA, eA_now, pA, mA, sA);
     // row B; prefetch the j atom of the next row A and the entry of the next row B
     const int eB_now = eB;
     pA = spos[eA & 0x7fffffff];
     mA = a.slot_meta[eA & 0x7fffffff];
-    eB = lst[min(kB + 2 * JW, last)];
+    eB = lst[list_at(min(kB + 2 * JW, last), near, a.lcap)];
     int sB;
     const T vB = row(kB, eB_now, pB, mB, sB);
     if constexpr (M >= 8) {
@@ -1403,23 +1435,32 @@ __device__ inline long long uni(long long v) {
 }
 __device__ inline double uni(double v) { return __longlong_as_double(uni(__double_as_longlong(v))); }
 
-// PM_JL_LDS (pm_internal.h) bytes per wave: an iteration's j forces (3 x 64
-// values and 64 slots), later the i-force reduction, PM_JL_NV(T) values of
-// the 64 lanes per pass.
-#define PM_JL_NV(T) (PM_JL_LDS / 64 / (int)sizeof(T))
+// the minimal-image difference a - b of two periodic fixed-point coordinates
+__device__ inline float min_image(int a, int b) { return (float)(int)((unsigned int)a - (unsigned int)b); }
+__device__ inline double min_image(long long a, long long b) {
+  return (double)(long long)((unsigned long long)a - (unsigned long long)b);
+}
 
-// Half-list pair kernel with one lane per list entry: one wave per i-cluster
-// of M atoms, whose positions, charges and types sit in scalar registers; a
-// lane takes one entry (64 per iteration) and evaluates it against the M i
-// atoms in turn.  The j force of an entry is then whole in its lane and is
-// added with one 64-bit integer atomic per component, with no cross-lane
-// sums; the i forces accumulate per lane in FP32 (one term per iteration and
-// i atom; FP64 in the FP64 kernel) and are summed over the lanes in FP64 at
-// the end, through LDS, in lane order.  Same pair arithmetic and the same
-// half-list rule as pair_cluster; only the order in which FP32 partial sums
-// are formed differs.
+// Half-list pair kernel with one lane per list entry: a.split waves per
+// i-cluster of M atoms, whose positions, charges and types sit in scalar
+// registers; a lane takes one entry (64 per iteration) and evaluates it
+// against the M i atoms in turn.  Wave `part` of a cluster takes the
+// iterations part, part + split, ...  The j force of an entry is then whole
+// in its lane and is added with one 64-bit integer atomic per component, with
+// no cross-lane sums; the i forces accumulate per lane in FP32 (one term per
+// iteration and i atom; FP64 in the FP64 kernel) and are summed over the
+// lanes in FP64 at the end, through LDS, in lane order.  Same pair arithmetic
+// and the same half-list rule as pair_cluster; only the order in which FP32
+// partial sums are formed differs.
+// VALU issue bounds it in boxes that fill the chip, so it leaves out what a
+// wave-uniform test can: the iterations of far entries whose 64 entries all
+// lie beyond the cutoff of the cluster's bounding box, the exclusion test of
+// iterations without a flagged entry, the pair arithmetic of an i atom none
+// of whose 64 pairs is within the cutoff, and the Lennard-Jones terms of an
+// i atom whose type has none with any type (the hydrogens of water models).
 template <typename T, int LJSWF, int CK, int CSWF, bool WE, int M, bool PA>
-__device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, const PmPairParams& pp, const int cl) {
+__device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, const PmPairParams& pp, const int wid) {
+  const int cl = wid >> a.split_log, part = wid & ((1 << a.split_log) - 1);
   extern __shared__ unsigned char s_lj_raw[];
   typedef typename std::conditional<sizeof(T) == 4, float4, double4>::type LJ4;
   const LJ4* s_lj = reinterpret_cast<const LJ4*>(s_lj_raw);
@@ -1427,7 +1468,12 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
   const int lane = threadIdx.x & 63;
   const int ncl = a.counts[1];
   if (cl >= ncl) {
-    if (WE && cl < a.ncl_max && lane < PM_NE) a.epart[(long long)cl * PM_NE + lane] = 0.0;
+    if (WE && cl < a.ncl_max && lane < PM_NE) a.epart[(long long)wid * PM_NE + lane] = 0.0;
+    return;
+  }
+  const int cnt = a.inner ? a.icount[cl] : a.jcount[cl];
+  if (64 * part >= cnt) {   // no iteration of this wave's
+    if (WE && lane < PM_NE) a.epart[(long long)wid * PM_NE + lane] = 0.0;
     return;
   }
   typedef typename std::conditional<sizeof(T) == 4, int4, longlong4>::type P4;
@@ -1438,8 +1484,9 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
   // the cluster's atoms, wave-uniform
   PI ipx[M], ipy[M], ipz[M];
   T iq[M];
-  int ity[M], ioi[M];
-  unsigned int ireal = 0;
+  int ioi[M];
+  unsigned long long ity = 0;   // types, 8 bits each
+  unsigned int ireal = 0, ilj = 0;   // atoms that are real, that have Lennard-Jones terms
 #pragma unroll
   for (int ii = 0; ii < M; ii++) {
     const P4 p = spos[c0 + ii];
@@ -1448,9 +1495,11 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
     ipy[ii] = uni(p.y);
     ipz[ii] = uni(p.z);
     if constexpr (sizeof(T) == 4) iq[ii] = __int_as_float(uni(p.w)); else iq[ii] = __longlong_as_double(uni(p.w));
-    ity[ii] = m & 0xff;
+    ity |= (unsigned long long)(m & 0xff) << (8 * ii);
     ioi[ii] = (m >> 8) & 0x7fffff;
     if (ioi[ii] != 0x7fffff) ireal |= 1u << ii;
+    // (padding slots carry the type after the last and are skipped)
+    if (PA || CK == PM_COUL_NONE || ((a.lj_types >> (m & 0x3f)) & 1ull)) ilj |= 1u << ii;
   }
   const T sx = sizeof(T) == 4 ? (T)box.fix_to_A[0] : (T)(box.fix_to_A[0] * 2.3283064365386963e-10);
   const T sy = sizeof(T) == 4 ? (T)box.fix_to_A[1] : (T)(box.fix_to_A[1] * 2.3283064365386963e-10);
@@ -1475,73 +1524,111 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
   const long long lbase = (long long)cl * a.lcap;
   const int* __restrict__ lst = (a.inner ? a.ilist : a.jlist) + lbase;
   const unsigned int* __restrict__ msk = (a.inner ? a.imask : a.jmask) + lbase;
-  const int cnt = a.inner ? a.icount[cl] : a.jcount[cl];
-  const int last = cnt > 0 ? cnt - 1 : 0;
+  const int near = a.inner ? cnt : a.jnear[cl];
+  const int last = cnt - 1;
   const bool vir = WE && a.want_virial != 0;
   long long* __restrict__ ff = a.force_slot;
   bool range_bad = false;
   // this wave's LDS area (after the LJ table): the j forces of an iteration
-  // (3 x 64 values and 64 slots), then the i-force reduction
-  constexpr int NV = PM_JL_NV(T);
+  // (3 x 64 values and 64 slots)
   const size_t tbytes = LJSWF != PM_SWF_NONE ? ((size_t)nt1 * nt1 * sizeof(LJ4) + 15) / 16 * 16 : 0;
-  T* s_red = reinterpret_cast<T*>(s_lj_raw + tbytes) + (threadIdx.x >> 6) * 64 * NV;
-  T* s_jf = s_red;
-  int* s_js = reinterpret_cast<int*>(s_red + 3 * 64);
+  T* s_jf = reinterpret_cast<T*>(s_lj_raw + tbytes + (threadIdx.x >> 6) * PM_JL_LDS(T));
+  int* s_js = reinterpret_cast<int*>(s_jf + 3 * 64);
+
+  // the cluster's bounding box relative to its first atom, for the far
+  // entries' test: valid while every atom's minimal image of an entry within
+  // the cutoff is also the first atom's.  Kept in LDS: the loop's scalar
+  // registers hold the cluster
+  T* s_box = reinterpret_cast<T*>(s_js + 64);
+  int far0 = 0x7fffffff;   // iterations from here on are tested
+  {
+    T lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+#pragma unroll
+    for (int ii = 1; ii < M; ii++) {
+      if (!((ireal >> ii) & 1u)) continue;
+      const T d[3] = {min_image(ipx[ii], ipx[0]) * sx, min_image(ipy[ii], ipy[0]) * sy, min_image(ipz[ii], ipz[0]) * sz};
+#pragma unroll
+      for (int c = 0; c < 3; c++) { lo[c] = min(lo[c], d[c]); hi[c] = max(hi[c], d[c]); }
+    }
+    const T reach = (T)(sqrt(pp.cut2) + 1e-3);   // padded for the test's rounding
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      ok = ok && reach + max(-lo[c], hi[c]) < (T)(0.499 * box.L[c]);
+      s_box[c] = lo[c];
+      s_box[3 + c] = hi[c];
+    }
+    s_box[6] = reach * reach;
+    if (uni((int)ok)) far0 = near;
+  }
+  wave_lds_sync();
 
   // the entry and j atom of this iteration, and the entry of the next, in
   // flight while the previous iteration computes; loads past the list's end
   // re-read its last entry (masked)
-  int e = cnt > 0 ? lst[min(lane, last)] : a.dummy_slot;
+  const int step = 64 << a.split_log;
+  const int first = 64 * part;
+  int e = lst[list_at(min(first + lane, last), near, a.lcap)];
   P4 pj = spos[e & 0x7fffffff];
   int mj = a.slot_meta[e & 0x7fffffff];
-  int en = cnt > 0 ? lst[min(lane + 64, last)] : a.dummy_slot;
-  for (int base = 0; base < cnt; base += 64) {
+  int en = lst[list_at(min(first + step + lane, last), near, a.lcap)];
+  for (int base = first; base < cnt; base += step) {
     const P4 pn = spos[en & 0x7fffffff];
     const int mn = a.slot_meta[en & 0x7fffffff];
-    const int enn = lst[min(base + 128 + lane, last)];
+    const int enn = lst[list_at(min(base + 2 * step + lane, last), near, a.lcap)];
     const int k = base + lane;
-    const bool valid = k < cnt;
     const int sj = e & 0x7fffffff;
-    // exclusions: only entries the list flagged hold an excluded pair
-    const bool flagged = valid && e < 0;
+    // the atom masks as scalars of this iteration: hoisted out of the loop,
+    // their bits would become sixteen lane masks and spill
+    unsigned int rm = (unsigned int)uni((int)ireal), lm = (unsigned int)uni((int)ilj);
+    asm volatile("" : "+s"(rm), "+s"(lm));
+    if (base >= far0) {
+      const T dx = min_image(pj.x, ipx[0]) * sx, dy = min_image(pj.y, ipy[0]) * sy, dz = min_image(pj.z, ipz[0]) * sz;
+      const T gx = max(max(s_box[0] - dx, dx - s_box[3]), T(0)), gy = max(max(s_box[1] - dy, dy - s_box[4]), T(0)),
+              gz = max(max(s_box[2] - dz, dz - s_box[5]), T(0));
+      if (__ballot(gx * gx + gy * gy + gz * gz <= s_box[6]) == 0ull) {
+        e = en;
+        pj = pn;
+        mj = mn;
+        en = enn;
+        continue;
+      }
+    }
+    // exclusions: only entries the list flagged hold an excluded pair; lanes
+    // past the list's end mask every pair
+    const bool flagged = k >= cnt || e < 0;
     unsigned int xm = 0;
     const bool anyflag = __ballot(flagged) != 0ull;
-    if (anyflag && flagged) xm = msk[k];
+    if (anyflag && flagged) xm = k >= cnt ? 0xffffu : msk[list_at(k, near, a.lcap)];
     const bool any_mod = anyflag && __ballot((xm >> 16) != 0u) != 0ull;
     T qj;
     if constexpr (sizeof(T) == 4) qj = __int_as_float(pj.w); else qj = __longlong_as_double(pj.w);
     const int tj = mj & 0xff;
     T fjx = 0, fjy = 0, fjz = 0;
-    // the pair of this lane's entry with cluster atom ii: MOD false for the
-    // ordinary pairs (excluded and modified ones masked; xm is 0 for entries
-    // the list did not flag), true for the modified (1-4) pairs, with the
-    // 1-4 LJ parameters and the Coulomb scaling
-    auto pair_ii = [&](const int ii, auto mod) {
-      constexpr bool MOD = decltype(mod)::value;
-      T dx, dy, dz;
-      if constexpr (sizeof(T) == 4) {
-        dx = (T)(int)(pj.x - ipx[ii]) * sx;
-        dy = (T)(int)(pj.y - ipy[ii]) * sy;
-        dz = (T)(int)(pj.z - ipz[ii]) * sz;
-      } else {
-        dx = (T)(long long)((unsigned long long)pj.x - (unsigned long long)ipx[ii]) * sx;
-        dy = (T)(long long)((unsigned long long)pj.y - (unsigned long long)ipy[ii]) * sy;
-        dz = (T)(long long)((unsigned long long)pj.z - (unsigned long long)ipz[ii]) * sz;
-      }
+    // the pair of this lane's entry with cluster atom ii: FL 0 for iterations
+    // without flagged entries, 1 for the ordinary pairs of the others (FULL
+    // and modified ones masked; xm is 0 for entries the list did not flag), 2
+    // for the modified (1-4) pairs, with the 1-4 LJ parameters and the
+    // Coulomb scaling
+    auto pair_ii = [&](const int ii, auto fl) {
+      constexpr int FL = decltype(fl)::value;
+      constexpr bool MOD = FL == 2;
+      const T dx = min_image(pj.x, ipx[ii]) * sx, dy = min_image(pj.y, ipy[ii]) * sy, dz = min_image(pj.z, ipz[ii]) * sz;
       const T r2 = dx * dx + dy * dy + dz * dz;
-      const bool mask = valid && sj > c0 + ii && (r2 <= cut2) &&
-                        (MOD ? (xm & (65536u << ii)) != 0u : (xm & (65537u << ii)) == 0u);
+      bool mask = r2 <= cut2;
+      if constexpr (FL == 1) mask = mask && (xm & (65537u << ii)) == 0u;
+      if constexpr (FL == 2) mask = mask && (xm & (65536u << ii)) != 0u;
       if (__ballot(mask) == 0ull) return;   // no lane's pair with atom ii counts
       T rr2, rinv;
       if constexpr (sizeof(T) == 4) { rinv = Prec<T>::rsq(r2); rr2 = rinv * rinv; }
       else { rr2 = T(1) / r2; rinv = sqrt(rr2); }
-      T F, E1 = 0, E2 = 0;
-      if constexpr (LJSWF != PM_SWF_NONE) {
+      T F = 0, E1 = 0, E2 = 0;
+      if (LJSWF != PM_SWF_NONE && ((lm >> ii) & 1u)) {
         T A, B;
         if constexpr (PA) {
-          lj_ab<T>(a, s_lj, ity[ii], mj, nt1, ioi[ii], MOD ? PM_EXCL_MODIFIED : PM_EXCL_NONE, A, B);
+          lj_ab<T>(a, s_lj, (int)((ity >> (8 * ii)) & 0xff), mj, nt1, ioi[ii], MOD ? PM_EXCL_MODIFIED : PM_EXCL_NONE, A, B);
         } else {
-          const LJ4 ab = s_lj[ity[ii] * nt1 + tj];
+          const LJ4 ab = s_lj[(int)((ity >> (8 * ii)) & 0xff) * nt1 + tj];
           // A14, B14 for modified pairs (LennardJonesForce.h:55-60)
           A = MOD ? (T)ab.z : (T)ab.x;
           B = MOD ? (T)ab.w : (T)ab.y;
@@ -1598,7 +1685,7 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
           if (modify)
             apply_switch<T, CSWF>(r2, r2 * rinv, c_cut2, c_on2, c_sw1, c_sw2, c_sw3, c_c15_1, c_c05_3, c_c15_3, f2, e2);
         }
-        if constexpr (LJSWF != PM_SWF_NONE) F += f2; else F = f2;
+        F += f2;
         E2 = e2;
       }
       F = mask ? F : T(0);
@@ -1619,13 +1706,14 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
         }
       }
     };
+    // (padding slots skipped: uniform)
 #pragma unroll
     for (int ii = 0; ii < M; ii++)
-      if ((ireal >> ii) & 1u) pair_ii(ii, std::false_type{});   // padding slots skipped (uniform)
+      if ((rm >> ii) & 1u) pair_ii(ii, std::integral_constant<int, 1>{});
     if (any_mod) {
 #pragma unroll
       for (int ii = 0; ii < M; ii++)
-        if ((ireal >> ii) & 1u) pair_ii(ii, std::true_type{});
+        if ((rm >> ii) & 1u) pair_ii(ii, std::integral_constant<int, 2>{});
     }
     // j forces: the 64 entries' x, y, z regrouped through LDS so that lane
     // v of round r adds component v % 3 of entry v / 3 (v = 64 r + lane):
@@ -1651,34 +1739,34 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
     mj = mn;
     en = enn;
   }
-  // i forces: per pass, every lane's partial sums of NV values into LDS;
-  // lane L adds value L % NV over the G = 64 / NV lane segments' share
-  // L / NV in FP64, then the G segment sums of each value are added over the
-  // lanes (the same order on every run).  The cluster's slots are
-  // consecutive, so value c is component c % 3 of slot c0 + c / 3.
+  // i forces: the 3 M sums over the 64 lanes by halving in FP64, the same
+  // order on every run: lanes l and l ^ 32 keep one half of the values each
+  // and add the other's share, then l ^ 16, ..., until a lane holds 3 values,
+  // one atom's, summed over all but the last lane bits
   {
-    constexpr int G = 64 / NV, SEG = 64 / G;
-    static_assert(NV * sizeof(T) * 64 == PM_JL_LDS && 3 * 64 * sizeof(T) + 64 * sizeof(int) <= PM_JL_LDS, "LDS area");
+    double v[3 * M];
 #pragma unroll
-    for (int pass = 0; pass < (3 * M + NV - 1) / NV; pass++) {
+    for (int ii = 0; ii < M; ii++) { v[3 * ii] = fix[ii]; v[3 * ii + 1] = fiy[ii]; v[3 * ii + 2] = fiz[ii]; }
+    int at = 0;   // the atom whose sums this lane keeps
 #pragma unroll
-      for (int v = 0; v < NV; v++) {
-        const int c = pass * NV + v, ii = c / 3, comp = c % 3;
-        if (c < 3 * M) s_red[v * 64 + lane] = comp == 0 ? fix[ii] : (comp == 1 ? fiy[ii] : fiz[ii]);
+    for (int half = M / 2, bit = 32; half >= 1; half /= 2, bit /= 2) {
+      const bool up = (lane & bit) != 0;
+#pragma unroll
+      for (int u = 0; u < 3 * half; u++) {
+        const double keep = up ? v[3 * half + u] : v[u], send = up ? v[u] : v[3 * half + u];
+        v[u] = keep + __shfl_xor(send, bit, 64);
       }
-      wave_lds_sync();
-      const int v = lane % NV, g = lane / NV;
-      double acc = 0.0;
+      at += up ? half : 0;
+    }
 #pragma unroll
-      for (int t = 0; t < SEG; t++) acc += (double)s_red[v * 64 + g * SEG + t];
+    for (int bit = 32 / M; bit > 0; bit /= 2)
 #pragma unroll
-      for (int off = NV; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
-      const int c = pass * NV + v;
-      if (lane < NV && c < 3 * M && ((ireal >> (c / 3)) & 1u)) {
-        range_bad |= !(__builtin_fabs(acc) < PM_FORCE_LIMIT);
-        atomicAdd((unsigned long long*)(ff + 3LL * c0 + c), (unsigned long long)__double2ll_rn(acc * PM_FORCE_FIX));
-      }
-      wave_lds_sync();
+      for (int u = 0; u < 3; u++) v[u] += __shfl_xor(v[u], bit, 64);
+    const int u = lane & (64 / M - 1);   // of an atom's 64 / M lanes, 0, 1, 2 add x, y, z
+    const double acc = u == 0 ? v[0] : u == 1 ? v[1] : v[2];
+    if (u < 3 && ((ireal >> at) & 1u)) {
+      range_bad |= !(__builtin_fabs(acc) < PM_FORCE_LIMIT);
+      atomicAdd((unsigned long long*)(ff + 3LL * (c0 + at) + u), (unsigned long long)__double2ll_rn(acc * PM_FORCE_FIX));
     }
   }
   if (__ballot(range_bad) != 0ull && lane == 0) pm_raise(box.err, PM_FLAG_FORCE_RANGE);
@@ -1694,7 +1782,7 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
       r[u] = v;
     }
     if (lane == 0) {
-      double* ep = a.epart + (long long)cl * PM_NE;
+      double* ep = a.epart + (long long)wid * PM_NE;
       ep[PM_E_COUL] = r[0];
       ep[PM_E_LJ] = r[1];
       for (int u = 2; u < PM_E_VIR; u++) ep[u] = 0.0;
@@ -1708,10 +1796,14 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
     }
   }
 }
+// Measured (98k water, rc 10): 122 us in mixed precision with or without the
+// 48 % of the instructions left out (the j-force atomics bound it: 78 us with
+// them taken out), FP64 264 -> 245 us; a million atoms beside PME 1525 -> 1385
+// us; 648 atoms FP64 35 -> 12 us with 8 waves per cluster.
 template <typename T, int LJSWF, int CK, int CSWF, bool WE, int M, bool PA>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 6 : 1) void k_pair_jl(PmBox box, PmNbLaunch a, PmPairParams pp) {
+__global__ __launch_bounds__(64 * PM_JL_WAVES(T), sizeof(T) == 4 ? 6 : 1) void k_pair_jl(PmBox box, PmNbLaunch a, PmPairParams pp) {
   pair_load_table<T, LJSWF>(a);
-  pair_cluster_jl<T, LJSWF, CK, CSWF, WE, M, PA>(box, a, pp, uni((int)(blockIdx.x * 4 + (threadIdx.x >> 6))));
+  pair_cluster_jl<T, LJSWF, CK, CSWF, WE, M, PA>(box, a, pp, uni((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6))));
 }
 struct PairArgs { PmBox box; PmNbLaunch a; PmPairParams pp; };
 // batched launches: JL selects the kernel layout (one lane per entry or a row per entry)
@@ -1762,7 +1854,8 @@ __global__ __launch_bounds__(256) void k_adjoint(PmBox box, PmNbLaunch a, PmPair
     __syncthreads();
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int cl = blockIdx.x * 4 + wave;
+  // 1 << a.split_log waves walk a cluster's list, one row of 8 entries each in turn
+  const int wid = blockIdx.x * 4 + wave, cl = wid >> a.split_log, part = wid & ((1 << a.split_log) - 1);
   if (cl >= a.counts[1]) return;
   const int ii = lane % M, js = lane / M;
   const int si = cl * M + ii;
@@ -1796,12 +1889,13 @@ __global__ __launch_bounds__(256) void k_adjoint(PmBox box, PmNbLaunch a, PmPair
   }
   double ax = 0, ay = 0, az = 0;
   const int* __restrict__ lst = a.jlist + (long long)cl * a.lcap;
-  const int cnt = a.jcount[cl];
+  const int cnt = a.jcount[cl], near = a.jnear[cl];
   const int comp = ii;   // lanes ii = 0, 1, 2 add the x, y, z component of a row
 
-  for (int base = 0; base < cnt; base += JW) {
-    const int k = base + js;
-    const bool valid = k < cnt;
+  if (JW * part >= cnt) return;
+  for (int base = JW * part; base < cnt; base += JW << a.split_log) {
+    const bool valid = base + js < cnt;
+    const int k = list_at(base + js, near, a.lcap);
     const int e = valid ? lst[k] : a.dummy_slot;
     const bool flagged = e < 0;
     const int sj = e & 0x7fffffff;
@@ -2198,41 +2292,51 @@ void pm_launch_list_stats(hipStream_t s, const int* jcount, const int* counts, u
 void pm_launch_list(hipStream_t s, const PmBox& box, const PmNbLaunch& a, const PmPairParams& p) {
   double cut = sqrt(p.cut2) + a.skin;
   float c = (float)(cut * (1.0 + 1e-5) + 1e-4);
+  const float cn = (float)(sqrt(p.cut2) + a.near_margin);
   size_t lds = 4 * (6 * a.nstencil + 1 + 2 * a.xs_tcap) * sizeof(int);
   if (pm_recording()) {
-    const ListArgs q{box, a, c * c};
+    const ListArgs q{box, a, c * c, cn * cn};
     pm_record(PM_REC_LIST, a.m, (a.ncl_max + 3) / 4, 256, (unsigned)lds, &q, sizeof(q));
     return;
   }
   const dim3 g((a.ncl_max + 3) / 4), b(256);
   if (a.m == 4) {
-    if (a.bbox_filter) hipLaunchKernelGGL((k_list<4, 1>), g, b, lds, s, box, a, c * c);
-    else hipLaunchKernelGGL((k_list<4, 0>), g, b, lds, s, box, a, c * c);
+    if (a.bbox_filter) hipLaunchKernelGGL((k_list<4, 1>), g, b, lds, s, box, a, c * c, cn * cn);
+    else hipLaunchKernelGGL((k_list<4, 0>), g, b, lds, s, box, a, c * c, cn * cn);
   } else {
-    if (a.bbox_filter) hipLaunchKernelGGL((k_list<8, 1>), g, b, lds, s, box, a, c * c);
-    else hipLaunchKernelGGL((k_list<8, 0>), g, b, lds, s, box, a, c * c);
+    if (a.bbox_filter) hipLaunchKernelGGL((k_list<8, 1>), g, b, lds, s, box, a, c * c, cn * cn);
+    else hipLaunchKernelGGL((k_list<8, 0>), g, b, lds, s, box, a, c * c, cn * cn);
   }
 }
 
 template <typename T, int LJ, int CK, int CS>
 static void launch_pair_t(hipStream_t s, const PmBox& box, const PmNbLaunch& a, const PmPairParams& p) {
   size_t lds = (LJ != PM_SWF_NONE) ? (size_t)a.ntypes1 * a.ntypes1 * (sizeof(T) == 4 ? 16 : 32) : 0;
-  // one block per four clusters (batched launches: per replica)
-  const dim3 gb((a.ncl_max + 3) / 4), b(256);
-  const dim3 g = gb;
+  // four waves per block: 1 << a.split_log waves per cluster, or one (rows)
+  const long long waves = (long long)a.ncl_max << (a.jlanes ? a.split_log : 0);
+  const dim3 g((waves + 3) / 4), b(256);
   const bool pa = LJ != PM_SWF_NONE && (sizeof(T) == 4 ? a.atom_lj_f != nullptr : a.atom_lj_d != nullptr);
-  // one lane per entry: the LJ table, then each wave's i-force reduction area
-  const size_t ljl = (lds + 15) / 16 * 16 + (size_t)4 * PM_JL_LDS;
+  // one lane per entry: the LJ table, then each wave's area
+  const size_t tab = (lds + 15) / 16 * 16;
   if (pm_recording()) {
     // per-atom LJ parameters have no batched kernel: the record is marked
     // unsupported and the batch runs its replicas as chains
     const PairArgs q{box, a, p};
     pm_record(pa ? -1 : PM_REC_PAIR,
-              pair_variant(sizeof(T) == 8, LJ, CK, CS, a.want_energy != 0, a.m, a.jlanes != 0), gb.x, 256,
-              (unsigned)(a.jlanes ? ljl : lds), &q, sizeof(q));
+              pair_variant(sizeof(T) == 8, LJ, CK, CS, a.want_energy != 0, a.m, a.jlanes != 0), g.x, 256,
+              (unsigned)(a.jlanes ? tab + 4 * PM_JL_LDS(T) : lds), &q, sizeof(q));
     return;
   }
   if (a.jlanes) {
+    // Blocks of 8 waves in mixed precision where the launch is a few rounds
+    // of the chip: a CU then frees two waves per SIMD at a time, and the PME
+    // kernels of the second stream find room for a block sooner (98k water,
+    // 50 steps with PME: 11.40 ms with 8, 12.17 with 4, 12.2 / 11.7 / 12.0
+    // with 10 / 12 / 16).  In larger boxes the pair kernel bounds the step
+    // and 4 are better (a million atoms, 16 steps: 37.2 ms with 4, 38.9 with 8)
+    const int W = sizeof(T) == 4 && waves <= PM_JL_WIDE_MAX ? PM_JL_WAVES(T) : 4;
+    const size_t ljl = tab + (size_t)W * PM_JL_LDS(T);
+    const dim3 g((waves + W - 1) / W), b(64 * W);
     if constexpr (LJ != PM_SWF_NONE) {
       if (pa) {
         if (a.want_energy) hipLaunchKernelGGL((k_pair_jl<T, LJ, CK, CS, true, 8, true>), g, b, ljl, s, box, a, p);
@@ -2294,7 +2398,7 @@ template <typename T, int LJ, int CK, int CS>
 static void launch_adjoint_t(hipStream_t s, const PmBox& box, const PmNbLaunch& a, const PmPairParams& p, int mode,
                              const double4* sv, long long* out) {
   size_t lds = (LJ != PM_SWF_NONE) ? (size_t)a.ntypes1 * a.ntypes1 * (sizeof(T) == 4 ? 16 : 32) : 0;
-  const dim3 g((a.ncl_max + 3) / 4), b(256);
+  const dim3 g((((long long)a.ncl_max << a.split_log) + 3) / 4), b(256);
   if (mode == 1) hipLaunchKernelGGL((k_adjoint<T, LJ, CK, CS, 1>), g, b, lds, s, box, a, p, sv, out);
   else hipLaunchKernelGGL((k_adjoint<T, LJ, CK, CS, 2>), g, b, lds, s, box, a, p, sv, out);
 }

@@ -1,0 +1,57 @@
+"""Where the lane-per-entry pair kernel's launch changes (waves per cluster,
+waves per block) and where its list groups and skipped terms can go wrong:
+forces and energies against the oracle, at fresh positions and, with the kept
+lists, after moves that bring far entries within the cutoff.  Tolerances: the
+mixed-precision force bar (5e-6 RMS relative, FP32 pair arithmetic) and FP64
+round-off of sums of ~300 terms (1e-11)."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from protomol_amd import water
+from tests.cases import exclusion_mix, gpu_forces_c1, rms_rel
+
+pytestmark = pytest.mark.gpu
+TOL = {"mixed": 5e-6, "double": 1e-11}
+
+
+def reference(port, s, x):
+    t = s.copy()
+    t.pos = x
+    a = port.cutoff(t, [po.term(po.POT_LJ, po.SWF_C2, 8.0, 7.0)], 8.0, 4.0)
+    b = port.cutoff(t, [po.term(po.POT_COULOMB, po.SWF_C2, 8.0, 7.0)], 8.0, 4.0)
+    return a["forces"] + b["forces"], a["energies"] + b["energies"]
+
+
+# molecules: 8, 4, 2 and 1 waves per cluster, and a launch on each side of a
+# change (about 1,024 waves)
+@pytest.mark.parametrize("molecules", [150, 217, 600, 1301, 2600])
+@pytest.mark.parametrize("kind", ["water", "exclusions", "uncharged"])
+@pytest.mark.parametrize("precision", ["mixed", "double"])
+def test_pair_forces_over_launch_shapes(gpu_ctx_factory, port, molecules, kind, precision):
+    print("case: pair split", molecules, kind, precision, flush=True)
+    s = water.water_box(molecules, (molecules / 0.0334) ** (1.0 / 3.0), seed=molecules, jitter=0.3)
+    if kind == "exclusions":
+        s = exclusion_mix(s)          # hydrogens with Lennard-Jones, 1-4 pairs
+    if kind == "uncharged":
+        s.q = np.where(np.arange(s.n) % 7 == 3, 0.0, s.q)
+    c = gpu_ctx_factory(precision)
+    c.set_topology(s)
+    c.set_boundary(s.box, s.origin, 4.0)
+    hs = gpu_forces_c1(c)
+    rng = np.random.default_rng(molecules)
+    builds = None
+    # the second move keeps the lists (half the skin is 1.1 A mixed, 0.5 FP64)
+    # and carries pairs from outside the near margin (0.5 A) into the cutoff
+    for step in (0.0, 0.45):
+        d = rng.standard_normal((molecules, 3))
+        x = s.pos + step * np.repeat(d / np.linalg.norm(d, axis=1)[:, None], 3, axis=0)
+        f, e = c.evaluate(hs, x)
+        if builds is not None:
+            assert c.stats()["list_builds"] == builds
+        builds = c.stats()["list_builds"]
+        fr, er = reference(port, s, x)
+        err = rms_rel(f, fr)
+        print("rms rel force", err, flush=True)
+        assert err < TOL[precision]
+        np.testing.assert_allclose(e[:2], er[:2], rtol=10 * TOL[precision], atol=1e-6 * np.abs(er[:2]).max())
