@@ -34,6 +34,8 @@
 #define PM_PRUNE_SKIN_AUTO 0.0
 // waves up to which a cluster's list is shared by several (pair_split)
 #define PM_SPLIT_WAVES 1024
+// work space that a context keeps between pm_lanczos calls
+#define PM_LANCZOS_KEEP_BYTES (256u << 20)
 
 // launch recorder of the calling thread (replica batches)
 static thread_local std::vector<PmRecord>* g_recorder = nullptr;
@@ -170,6 +172,11 @@ struct pm_context {
   long long* d_adj_fix = nullptr;       // [3 adj_n] per-atom fixed point
   double* d_adj_v = nullptr;            // [3 adj_n] direction
   double* d_adj_out = nullptr;          // [3 adj_n] FP64 parts
+  double* d_lanczos = nullptr;          // work space of pm_lanczos
+  size_t lanczos_alloc = 0;
+  // two PME grids of the adjoint (the charges' and the direction's)
+  void *d_adj_grid_r = nullptr, *d_adj_grid_c = nullptr;
+  size_t adj_grid_bytes = 0;
   long long adj_nslot = 0;
   int adj_n = 0;
 
@@ -530,6 +537,15 @@ static int pair_split(const pm_context* c) {
   return s;
 }
 
+// log2 of the waves per cluster of the adjoint kernel, whose rows take only 8
+// entries per iteration (8,100 atoms, mixed: 67 us with one wave per cluster,
+// 1,013 waves)
+static int adjoint_split(const pm_context* c) {
+  int s = 0;
+  while (s < 4 && ((long long)c->ncl_max << (s + 1)) <= 16384) s++;
+  return s;
+}
+
 // The types with Lennard-Jones parameters, for the pair kernel to leave the
 // others' terms out.  With an uncharged atom every type counts: two atoms on
 // one point then still show as a force that is not finite.
@@ -642,6 +658,19 @@ int ensure_epart(pm_context* c, long long records) {
   int r = dalloc(c, &c->d_epart, (size_t)records * PM_NE);
   if (r) return r;
   c->epart_alloc = records;
+  return PM_OK;
+}
+
+// the adjoint's complex and real grids, `bytes` each
+int ensure_adj_grids(pm_context* c, size_t bytes) {
+  if (bytes <= c->adj_grid_bytes) return PM_OK;
+  if (c->d_adj_grid_r) hipFree(c->d_adj_grid_r);
+  if (c->d_adj_grid_c) hipFree(c->d_adj_grid_c);
+  c->d_adj_grid_r = c->d_adj_grid_c = nullptr;
+  c->adj_grid_bytes = 0;
+  HIPCHECK(c, hipMalloc(&c->d_adj_grid_r, bytes));
+  HIPCHECK(c, hipMalloc(&c->d_adj_grid_c, bytes));
+  c->adj_grid_bytes = bytes;
   return PM_OK;
 }
 
@@ -1074,6 +1103,8 @@ struct AdjointSpec {
   double4* slot_v = nullptr;   // [nslot_max + 1]
   long long* slot = nullptr;   // [3 (nslot_max + 1)] per-slot fixed point
   long long* fix = nullptr;    // [3n] per-atom fixed point
+  bool kept = false;           // the positions are those of the previous pass of this
+                               // call: its layout, lists and potential still hold
   double* hv = nullptr;        // [3n] mode 1 (PME and correction parts, FP64)
   double* dq = nullptr;        // [n] mode 2 (PME, correction and self parts, FP64)
 };
@@ -1178,7 +1209,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   const int* rb = reuse ? c->d_rebuild : nullptr;
   const bool inner = reuse && inner_lists(c);
   c->inner_last = inner;
-  {
+  if (!adj || !adj->kept) {
   TimedScope ts(c, PM_T_BIN);
   if (reuse && c->list_stale) {
     pm_launch_invalidate_build(s, n, c->d_xbuild);
@@ -1194,7 +1225,9 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   // (the MD position update may have binned the atoms and cleared the forces
   // already, for the layout in place; the last fold cleared the slot forces)
   const bool binned = prebinned && c->prebin_gen == c->layout_gen;
-  if (!binned) {
+  if (adj) {
+    pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, rb);
+  } else if (!binned) {
     pm_launch_zero_force_cells(s, rb, c->d_force, 3LL * n, c->d_force_slot,
                                passes.empty() && !any_pme ? 0 : 3LL * c->nslot_max, nullptr, 0);
     pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, rb);
@@ -1285,7 +1318,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.xs_tcap = c->m * c->xs_maxdeg;
     a.m = c->m;
     a.jlanes = pair_lanes(c);
-    a.split_log = adj ? 0 : slog;
+    a.split_log = adj ? adjoint_split(c) : slog;
     a.near_margin = replica_form(c) ? PM_NEAR_ALL : PM_NEAR_MARGIN;
     a.lj_types = c->lj_types;
     a.molecule = c->d_mol;
@@ -1388,12 +1421,22 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       // rebuilds the layout), padded for the float displacement test
       const double drift_A = (reuse ? 0.5 * skin * (1.0 + 1e-3) : 0.0) + 1e-3;
       for (int d = 0; d < 3; d++) a.drift_u[d] = drift_A * ng[d] / c->box.L[d] + 0.01;
-      a.spread_zfwd = !adj && c->pme_spread_option != 0 ? pm_pme_spread_zfwd_fits(a, c->precision) : 0;
+      if (adj) {
+        // two grids of its own, so that the charges' potential outlives the
+        // direction's convolution; line-major, with theta from the table
+        const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+        if ((r = ensure_adj_grids(c, 2 * er * (size_t)a.nx * a.ny * a.nzc * 2))) return r;
+        a.grid_r = c->d_adj_grid_r;
+        a.grid_c = c->d_adj_grid_c;
+        a.plane = 0;
+        a.want_energy = a.want_virial = 0;
+      }
+      a.spread_zfwd = c->pme_spread_option != 0 ? pm_pme_spread_zfwd_fits(a, c->precision) : 0;
       if (!a.spread_zfwd && (size_t)a.tile[0] * a.tile[1] * a.tile[2] * 8 > 64 * 1024)
         return fail(c, PM_ERR_UNSUPPORTED, "PME grid too fine for the cell size: spread tile exceeds 64 KB of LDS (use a smaller cellsize)");
       pme_launch.push_back(std::make_pair(a, hr.first));
     }
-    if (f.corr) {
+    if (f.corr && !adj) {
       // point self energy and charged-system term (:604-628)
       double q2 = 0.0, qs = 0.0;
       for (int i = 0; i < n; i++) q2 += c->q[i] * c->q[i];
@@ -1412,28 +1455,37 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     return r;
 
   if (adj) {
-    // adjoint kernels, all on the first stream
-    pm_launch_slot_vec(s, c->d_counts, c->d_atom_of_slot, adj->mode == 1 ? adj->v : c->d_scratch3, adj->slot_v,
-                       c->nslot_max);
-    pm_launch_zero_ll(s, adj->slot, 3LL * (c->nslot_max + 1));
-    pm_launch_zero_ll(s, adj->fix, 3LL * n);
-    if (adj->mode == 1) pm_launch_zero_d(s, adj->hv, 3LL * n);
-    else pm_launch_zero_d(s, adj->dq, n);
+    // pairs on the first stream, PME and correction on the second: they write
+    // different arrays (fixed point, FP64)
+    hipStream_t s2 = pme_rec.empty() ? s : c->stream2;
+    double* out = adj->mode == 1 ? adj->hv : adj->dq;
+    if (adj->mode == 1) pm_launch_slot_vec(s, c->d_counts, c->d_atom_of_slot, adj->v, adj->slot_v, c->nslot_max);
+    if (s2 != s) {
+      HIPCHECK(c, hipEventRecord(c->ev_fork, s));
+      HIPCHECK(c, hipStreamWaitEvent(s2, c->ev_fork, 0));
+    }
+    pm_launch_zero_force_cells(s, nullptr, adj->slot, 3LL * (c->nslot_max + 1), adj->fix, 3LL * n, nullptr, 0);
     for (auto& pl : pair_launch) {
-      pm_launch_list(s, c->box, pl.first, pl.second);
+      // (one pass keeps its lists between the passes of a call)
+      if (!adj->kept || pair_launch.size() > 1) pm_launch_list(s, c->box, pl.first, pl.second);
       pm_launch_adjoint(s, c->box, pl.first, pl.second, c->precision, adj->mode, adj->slot_v, adj->slot);
     }
     if (!pair_launch.empty())
       pm_launch_fold_slots(s, c->nslot_max, c->d_counts, c->d_atom_of_slot, adj->slot, nullptr, adj->fix, nullptr,
                            nullptr, 0);
+    if (pme_launch.empty()) pm_launch_zero_d(s2, out, adj->mode == 1 ? 3LL * n : n);
     for (auto& pl : pme_launch)
-      pm_launch_pme_adjoint(s, pl.first, c->plans, c->d_slot_pos64, c->precision, adj->mode == 1 ? 1 : 0,
-                            adj->slot_v, adj->mode == 1 ? adj->hv : adj->dq);
+      pm_launch_pme_adjoint(s2, pl.first, c->plans, c->d_slot_pos64, c->precision, adj->mode == 1 ? 1 : 0,
+                            adj->kept && pme_launch.size() == 1, adj->slot_v, out);
     for (auto& hr : pme_rec) {
       ForceDesc& f = c->forces[hr.first];
       if (!f.corr) continue;
-      pm_launch_corr_adjoint(s, c->box, n, c->d_pos, c->d_q, c->d_cx_row, c->d_cx_partner, c->d_cx_cls, f.alpha,
-                             c->csf, adj->mode == 1 ? 1 : 0, adj->v, adj->mode == 1 ? adj->hv : adj->dq);
+      pm_launch_corr_adjoint(s2, c->box, n, c->d_pos, c->d_q, c->d_cx_row, c->d_cx_partner, c->d_cx_cls, f.alpha,
+                             c->csf, adj->mode == 1 ? 1 : 0, adj->v, out);
+    }
+    if (s2 != s) {
+      HIPCHECK(c, hipEventRecord(c->ev_join, s2));
+      HIPCHECK(c, hipStreamWaitEvent(s, c->ev_join, 0));
     }
     HIPCHECK(c, hipGetLastError());
     return PM_OK;
@@ -1730,7 +1782,12 @@ void free_all(pm_context* c) {
   dfree(c->d_xs_row); dfree(c->d_xs_part); dfree(c->d_jmask);
   dfree(c->d_atom_lj_f); dfree(c->d_atom_lj_d);
   c->lj_R.clear(); c->lj_e.clear();
-  dfree(c->d_adj_sv); dfree(c->d_adj_slot); dfree(c->d_adj_fix); dfree(c->d_adj_v); dfree(c->d_adj_out);
+  dfree(c->d_adj_sv); dfree(c->d_adj_slot); dfree(c->d_adj_fix); dfree(c->d_adj_v); dfree(c->d_adj_out); dfree(c->d_lanczos);
+  c->lanczos_alloc = 0;
+  if (c->d_adj_grid_r) hipFree(c->d_adj_grid_r);
+  if (c->d_adj_grid_c) hipFree(c->d_adj_grid_c);
+  c->d_adj_grid_r = c->d_adj_grid_c = nullptr;
+  c->adj_grid_bytes = 0;
   c->adj_nslot = 0; c->adj_n = 0;
   dfree(c->d_cx_row); dfree(c->d_cx_partner); dfree(c->d_cx_cls);
   dfree(c->d_tab_a); dfree(c->d_tab_b); dfree(c->d_tab_c);
@@ -2808,35 +2865,30 @@ static int adjoint_check(pm_context* c, const int* handles, int nh) {
 // one adjoint pass over the positions already in d_pos: mode 1 H v with the
 // direction in d_adj_v, mode 2 parameter gradients; results in d_adj_fix
 // (fixed point) and d_adj_out (FP64 parts)
-static int adjoint_pass(pm_context* c, const int* handles, int nh, int mode) {
+static int adjoint_pass(pm_context* c, const int* handles, int nh, int mode, bool kept = false) {
   AdjointSpec a;
   a.mode = mode;
+  a.kept = kept;
   a.slot_v = c->d_adj_sv; a.slot = c->d_adj_slot; a.fix = c->d_adj_fix; a.v = c->d_adj_v;
   if (mode == 1) a.hv = c->d_adj_out; else a.dq = c->d_adj_out;
   std::vector<int> hs(handles, handles + nh);
   return evaluate_group(c, hs, 0, false, &a);
 }
 
-static int adjoint_run(pm_context* c, const int* handles, int nh, const double* positions, const double* v,
-                       int mode, std::vector<long long>& fix, std::vector<double>& dbl) {
+// one adjoint pass over host positions (and, mode 1, a host direction); the
+// results stay on the device
+static int adjoint_run(pm_context* c, const int* handles, int nh, const double* positions, const double* v, int mode) {
   int r;
   if (!positions) return fail(c, PM_ERR_ARGUMENT, "positions required");
   if ((r = adjoint_check(c, handles, nh))) return r;
-  const int n = c->n;
   hipStream_t s = c->stream;
-  const size_t bytes = 3 * (size_t)n * sizeof(double);
+  const size_t bytes = 3 * (size_t)c->n * sizeof(double);
   hipError_t e = hipMemcpyAsync(c->d_pos, positions, bytes, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(c->d_adj_v, v ? v : positions, bytes, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess && v) e = hipMemcpyAsync(c->d_adj_v, v, bytes, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return fail(c, PM_ERR_DEVICE, "HIP error %s copying the inputs", hipGetErrorString(e));
   c->md_forces_valid = false;
   if ((r = adjoint_pass(c, handles, nh, mode))) { hipStreamSynchronize(s); return r; }
-  fix.assign(3 * (size_t)n, 0);
-  dbl.assign(mode == 1 ? 3 * (size_t)n : (size_t)n, 0.0);
-  e = hipMemcpyAsync(fix.data(), c->d_adj_fix, fix.size() * sizeof(long long), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(dbl.data(), c->d_adj_out, dbl.size() * sizeof(double), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess) return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
-  return check_overflow(c);
+  return PM_OK;
 }
 
 int pm_hessian_vec(pm_context* c, const int* handles, int nh, const double* positions, const double* v,
@@ -2844,11 +2896,17 @@ int pm_hessian_vec(pm_context* c, const int* handles, int nh, const double* posi
   if (!c || !v || !hv) return PM_ERR_ARGUMENT;
   int r;
   if ((r = set_device(c))) return r;
-  std::vector<long long> fix;
-  std::vector<double> dbl;
-  if ((r = adjoint_run(c, handles, nh, positions, v, 1, fix, dbl))) return r;
-  for (size_t k = 0; k < fix.size(); k++) hv[k] = (double)fix[k] * PM_FORCE_UNFIX + dbl[k];
-  return PM_OK;
+  if ((r = adjoint_run(c, handles, nh, positions, v, 1))) return r;
+  const int n3 = 3 * c->n;
+  pm_launch_fix_combine(c->stream, n3, c->d_adj_fix, c->d_adj_out, nullptr, c->d_scratch3);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(hv, c->d_scratch3, (size_t)n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  if (e != hipSuccess) {
+    hipStreamSynchronize(c->stream);
+    return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
+  }
+  return check_overflow(c);
 }
 
 int pm_param_gradients(pm_context* c, const int* handles, int nh, const double* positions, double* dE_dq,
@@ -2858,17 +2916,21 @@ int pm_param_gradients(pm_context* c, const int* handles, int nh, const double* 
   if ((r = set_device(c))) return r;
   if ((dE_dsigma || dE_depsilon) && c->lj_R.empty())
     return fail(c, PM_ERR_STATE, "gradients with respect to sigma and epsilon need per-atom LJ parameters (pm_set_lj_per_atom)");
-  std::vector<long long> fix;
-  std::vector<double> dbl;
-  if ((r = adjoint_run(c, handles, nh, positions, nullptr, 2, fix, dbl))) return r;
-  const double rfac = std::pow(2.0, -5.0 / 6.0);   // dR/dsigma
-  for (int i = 0; i < c->n; i++) {
-    if (dE_dq) dE_dq[i] = (double)fix[3 * i] * PM_FORCE_UNFIX + dbl[i];
-    if (dE_dsigma) dE_dsigma[i] = (double)fix[3 * i + 1] * PM_FORCE_UNFIX * rfac;
-    // de/deps = 1/(2 sqrt(eps)): no finite derivative at eps = 0 (reported 0)
-    if (dE_depsilon) dE_depsilon[i] = c->lj_e[i] > 0 ? (double)fix[3 * i + 2] * PM_FORCE_UNFIX / (2.0 * c->lj_e[i]) : 0.0;
+  if ((r = adjoint_run(c, handles, nh, positions, nullptr, 2))) return r;
+  const int n = c->n;
+  // dE/dq, dE/dsigma = dE/dR dR/dsigma, dE/deps = dE/de / (2 e) one after the other
+  pm_launch_param_out(c->stream, n, c->d_adj_fix, c->d_adj_out, c->d_atom_lj_d, std::pow(2.0, -5.0 / 6.0), c->d_scratch3);
+  hipError_t e = hipGetLastError();
+  double* host[3] = {dE_dq, dE_dsigma, dE_depsilon};
+  for (int k = 0; k < 3; k++)
+    if (host[k] && e == hipSuccess)
+      e = hipMemcpyAsync(host[k], c->d_scratch3 + (size_t)k * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost,
+                         c->stream);
+  if (e != hipSuccess) {
+    hipStreamSynchronize(c->stream);
+    return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
   }
-  return PM_OK;
+  return check_overflow(c);
 }
 
 int pm_set_charges(pm_context* c, const double* q) {
@@ -2956,16 +3018,25 @@ int pm_lanczos(pm_context* c, const int* handles, int nh, const double* position
   const int m = steps;
   // device work space: basis V [m + 1][n3], w, 1/sqrt(mass), partial sums,
   // coefficients [2][m + 1], alpha [m], beta [m], tridiagonal eigenvectors
-  double *V = nullptr, *w = nullptr, *wt = nullptr, *part = nullptr, *coef = nullptr, *ab = nullptr, *S = nullptr,
-         *Y = nullptr;
-  auto cleanup = [&]() { dfree(V); dfree(w); dfree(wt); dfree(part); dfree(coef); dfree(ab); dfree(S); dfree(Y); };
-  if ((r = dalloc(c, &V, (size_t)(m + 1) * n3)) || (r = dalloc(c, &w, (size_t)n3)) ||
-      (r = dalloc(c, &wt, (size_t)n)) || (r = dalloc(c, &part, (size_t)(m + 1) * nblk)) ||
-      (r = dalloc(c, &coef, 2 * (size_t)(m + 1))) || (r = dalloc(c, &ab, 2 * (size_t)m)) ||
-      (r = dalloc(c, &S, (size_t)std::max(1, nvec) * m)) || (r = dalloc(c, &Y, nvec > 0 ? (size_t)nvec * n3 : 1))) {
-    cleanup();
-    return r;
+  // in one array that the context keeps for the next call while it is small
+  // (eight allocations and frees a call took 1 ms otherwise)
+  const size_t parts[8] = {(size_t)(m + 1) * n3, (size_t)n3, (size_t)n, (size_t)(m + 1) * nblk, 2 * (size_t)(m + 1),
+                           2 * (size_t)m, (size_t)std::max(1, nvec) * m, nvec > 0 ? (size_t)nvec * n3 : 1};
+  size_t total = 0, at[8];
+  for (int k = 0; k < 8; k++) { at[k] = total; total += (parts[k] + 31) / 32 * 32; }
+  if (c->lanczos_alloc < total) {
+    c->lanczos_alloc = 0;
+    if ((r = dalloc(c, &c->d_lanczos, total))) return r;
+    c->lanczos_alloc = total;
   }
+  double* const base = c->d_lanczos;
+  double *V = base + at[0], *w = base + at[1], *wt = base + at[2], *part = base + at[3], *coef = base + at[4],
+         *ab = base + at[5], *S = base + at[6], *Y = base + at[7];
+  auto cleanup = [&]() {
+    if (c->lanczos_alloc * sizeof(double) <= PM_LANCZOS_KEEP_BYTES) return;
+    dfree(c->d_lanczos);
+    c->lanczos_alloc = 0;
+  };
   std::vector<double> h(n3);
   const double inv0 = 1.0 / std::sqrt(nrm0);
   for (int k = 0; k < n3; k++) h[k] = v0[k] * inv0;
@@ -2984,7 +3055,7 @@ int pm_lanczos(pm_context* c, const int* handles, int nh, const double* position
     double* vj = V + (size_t)j * n3;
     // w = M^-1/2 H M^-1/2 v_j (M = 1 without mass weighting)
     pm_launch_scale_copy(s, n3, vj, mw, c->d_adj_v);
-    if ((r = adjoint_pass(c, handles, nh, 1))) { hipStreamSynchronize(s); cleanup(); return r; }
+    if ((r = adjoint_pass(c, handles, nh, 1, j > 0))) { hipStreamSynchronize(s); cleanup(); return r; }
     pm_launch_fix_combine(s, n3, c->d_adj_fix, c->d_adj_out, mw, w);
     // two classical Gram-Schmidt passes against v_0..v_j; alpha_j = v_j . w
     // collects the v_j coefficients of both passes

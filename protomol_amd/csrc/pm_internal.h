@@ -271,6 +271,7 @@ struct PmPmeLaunch {
   const double* tw;          // twiddles exp(-2 pi i m/n), interleaved re, im
   long long* force_fix;      // [3n] the gather writes every atom's force
   int accumulate;            // 1: the gather adds to force_fix (a later term of several)
+  int grid0;                 // the first grid of a launch over several (adjoint), else 0
   double* epart;             // [pm_pme_xpass_blocks() * PM_NE]
   int want_virial;
   int want_energy;           // 0: no energy records (then neither is the virial wanted)
@@ -320,10 +321,12 @@ void pm_launch_pme_theta(hipStream_t s, const PmPmeLaunch& a, int precision);
 int pm_pme_xpass_blocks(int nx, int ny, int nz, int precision, int plane);
 // 1 when a kz plane of an nx x ny grid fits the plane kernel's LDS
 int pm_pme_plane_fits(int nx, int ny, int precision, int lds_max);
-// PME adjoint: mode 0 out[n] += dE/dq (reciprocal potential), mode 1
-// out[3n] += (H v) of the reciprocal energy; slot_v = v in slot order
+// PME adjoint: mode 0 out[n] = dE/dq (reciprocal potential), mode 1 out[3n] =
+// (H v) of the reciprocal energy (added with a.accumulate); slot_v = v in slot
+// order.  grid_r and grid_c hold two grids, the charges' and the direction's;
+// kept: the first still holds the potential of these positions
 bool pm_launch_pme_adjoint(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, const longlong4* pos64,
-                           int precision, int mode, const double4* slot_v, double* out);
+                           int precision, int mode, bool kept, const double4* slot_v, double* out);
 
 // PME real-space term with lattice images, for boxes no wider than twice the
 // cutoff: lat = 3 * nlat lattice vectors ((0,0,0) first, nlat <= 1024), one
@@ -348,6 +351,11 @@ int pm_krylov_dot_blocks(int n3);
 void pm_launch_scale_copy(hipStream_t s, int n3, const double* in, const double* w, double* out);
 void pm_launch_fix_combine(hipStream_t s, int n3, const long long* fix, const double* dbl, const double* w,
                            double* out);
+// per atom: out[i] = dE/dq (fix[3i] + dq[i]), out[n + i] = rfac fix[3i + 1],
+// out[2n + i] = fix[3i + 2] / (2 e) with e = lj[i].y (0 where e is 0: no finite
+// derivative there); the last two only with per-atom LJ parameters
+void pm_launch_param_out(hipStream_t s, int n, const long long* fix, const double* dq, const double4* lj, double rfac,
+                         double* out);
 void pm_launch_dots(hipStream_t s, int n3, int nv, const double* V, const double* x, double* partial, double* out,
                     int acc_row, double* acc, int acc_set, int take_sqrt);
 void pm_launch_gs_update(hipStream_t s, int n3, int nv, const double* V, const double* c, double* w);

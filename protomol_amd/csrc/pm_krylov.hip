@@ -45,6 +45,17 @@ __global__ void k_fix_combine(int n3, const long long* __restrict__ fix, const d
   out[k] = w ? v * w[k / 3] : v;
 }
 
+__global__ void k_param_out(int n, const long long* __restrict__ fix, const double* __restrict__ dq,
+                            const double4* __restrict__ lj, double rfac, double* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  out[i] = (double)fix[3 * i] * PM_FORCE_UNFIX + dq[i];
+  if (!lj) return;
+  const double e = lj[i].y;
+  out[n + i] = (double)fix[3 * i + 1] * PM_FORCE_UNFIX * rfac;
+  out[2 * n + i] = e > 0 ? (double)fix[3 * i + 2] * PM_FORCE_UNFIX / (2.0 * e) : 0.0;
+}
+
 // partial[j][b] = sum over block b's chunk of V[j][k] x[k]; grid (nblk, nv)
 __global__ __launch_bounds__(KB) void k_dots_partial(int n3, const double* __restrict__ V, const double* __restrict__ x,
                                                      double* __restrict__ partial) {
@@ -119,6 +130,11 @@ void pm_launch_scale_copy(hipStream_t s, int n3, const double* in, const double*
 void pm_launch_fix_combine(hipStream_t s, int n3, const long long* fix, const double* dbl, const double* w,
                            double* out) {
   if (n3 > 0) hipLaunchKernelGGL(k_fix_combine, blocks_for(n3), dim3(KB), 0, s, n3, fix, dbl, w, out);
+}
+
+void pm_launch_param_out(hipStream_t s, int n, const long long* fix, const double* dq, const double4* lj, double rfac,
+                         double* out) {
+  if (n > 0) hipLaunchKernelGGL(k_param_out, blocks_for(n), dim3(KB), 0, s, n, fix, dq, lj, rfac, out);
 }
 
 void pm_launch_dots(hipStream_t s, int n3, int nv, const double* V, const double* x, double* partial, double* out,

@@ -188,6 +188,16 @@ __device__ T2* fft_lines(T2* b0, T2* b1, int nl, const PmFftPlan& p, const T2* t
   return in;
 }
 
+// The complex and real grids of this block: an adjoint launch transforms
+// several grids, one after the other in memory (a.grid0 + blockIdx.y), every
+// other launch one.
+template <typename T2> __device__ inline T2* grid_c_of(const PmPmeLaunch& a) {
+  return reinterpret_cast<T2*>(a.grid_c) + (long long)(a.grid0 + blockIdx.y) * a.nx * a.ny * a.nzc;
+}
+template <typename T> __device__ inline T* grid_r_of(const PmPmeLaunch& a) {
+  return reinterpret_cast<T*>(a.grid_r) + (long long)(a.grid0 + blockIdx.y) * a.nx * a.ny * a.nz;
+}
+
 // stage the twiddles of one transform length into LDS (followed by a barrier
 // in the caller's first __syncthreads)
 template <typename T2>
@@ -600,9 +610,9 @@ __global__ __launch_bounds__(256) void k_spread_dir(PmPmeLaunch a, const longlon
   }
 }
 
-// MODE 0: out[at] += phi(x_at) (dE/dq of the reciprocal energy)
-// MODE 1: out[3 at + c] += q (grad grad W . v)_c summed against phi
-// MODE 2: out[3 at + c] += q (grad W)_c summed against dphi (the grid holds it)
+// MODE 0: out[at] (+)= phi(x_at) (dE/dq of the reciprocal energy)
+// MODE 1: out[3 at + c] (+)= q (grad grad W . v)_c summed against phi (grid 0)
+// and q (grad W)_c summed against dphi (grid 1)
 template <typename T, int P, int MODE>
 __global__ __launch_bounds__(256) void k_gather_adj(PmPmeLaunch a, const longlong4* __restrict__ pos64,
                                                     const double4* __restrict__ slot_v, double* __restrict__ out) {
@@ -622,7 +632,8 @@ __global__ __launch_bounds__(256) void k_gather_adj(PmPmeLaunch a, const longlon
   const T vx = (T)v.x, vy = (T)v.y, vz = (T)v.z;
   const int off = -(P - 1) / 2;
   const T* g = reinterpret_cast<const T*>(a.grid_r);
-  T r0 = 0, r1 = 0, r2 = 0;
+  const long long second = (long long)a.nx * a.ny * a.nz;   // to the direction's potential
+  T r0 = 0, r1 = 0, r2 = 0, d0 = 0, d1 = 0, d2 = 0;
 #pragma unroll
   for (int i = 0; i < P; i++) {
     const int gx = wrap_grid(ix + off + i, a.nx);
@@ -636,8 +647,9 @@ __global__ __launch_bounds__(256) void k_gather_adj(PmPmeLaunch a, const longlon
         const T phi = row[gz];
         if constexpr (MODE == 0) {
           r0 += phi * tx[i] * ty[j] * tz[k];
-        } else if constexpr (MODE == 1) {
-          // Hessian of W(g - x) with respect to x, applied to v
+        } else {
+          // Hessian of W(g - x) with respect to x, applied to v, on the
+          // charges' potential; the gradient of W on the direction's
           const T hxx = h0 * h0 * ex[i] * ty[j] * tz[k], hyy = h1 * h1 * tx[i] * ey[j] * tz[k];
           const T hzz = h2 * h2 * tx[i] * ty[j] * ez[k];
           const T hxy = h0 * h1 * dx[i] * dy[j] * tz[k], hxz = h0 * h2 * dx[i] * ty[j] * dz[k];
@@ -645,21 +657,22 @@ __global__ __launch_bounds__(256) void k_gather_adj(PmPmeLaunch a, const longlon
           r0 += phi * (hxx * vx + hxy * vy + hxz * vz);
           r1 += phi * (hxy * vx + hyy * vy + hyz * vz);
           r2 += phi * (hxz * vx + hyz * vy + hzz * vz);
-        } else {
-          r0 += phi * h0 * dx[i] * ty[j] * tz[k];
-          r1 += phi * h1 * tx[i] * dy[j] * tz[k];
-          r2 += phi * h2 * tx[i] * ty[j] * dz[k];
+          const T dphi = row[second + gz];
+          d0 += dphi * h0 * dx[i] * ty[j] * tz[k];
+          d1 += dphi * h1 * tx[i] * dy[j] * tz[k];
+          d2 += dphi * h2 * tx[i] * ty[j] * dz[k];
         }
       }
     }
   }
+  // the first term of several writes, the others add
   if constexpr (MODE == 0) {
-    out[at] += (double)r0;
+    out[at] = a.accumulate ? out[at] + (double)r0 : (double)r0;
   } else {
     const double q = a.q[at];
-    out[3 * at] += q * (double)r0;
-    out[3 * at + 1] += q * (double)r1;
-    out[3 * at + 2] += q * (double)r2;
+    double t[3] = {q * (double)r0 + q * (double)d0, q * (double)r1 + q * (double)d1, q * (double)r2 + q * (double)d2};
+#pragma unroll
+    for (int k = 0; k < 3; k++) out[3 * at + k] = a.accumulate ? out[3 * at + k] + t[k] : t[k];
   }
 }
 
@@ -696,7 +709,7 @@ __global__ __launch_bounds__(256) void k_fft_z_fwd(PmPmeLaunch a, PmFftPlan p, i
   }
   __syncthreads();
   T2* r = fft_lines<T, T2>(b0, b1, TL, p, tws, -1, ls);
-  T2* gc = reinterpret_cast<T2*>(a.grid_c);
+  T2* gc = grid_c_of<T2>(a);
   if (a.plane) {
     for (int e = threadIdx.x; e < TL * nzc; e += blockDim.x) {
       const int k = e / TL, l = e - k * TL;
@@ -724,8 +737,11 @@ __global__ __launch_bounds__(256) void k_fft_z_fwd(PmPmeLaunch a, PmFftPlan p, i
 // to clear.
 #define PM_SZ_LX 4
 #define PM_SZ_MAXCOL 256
-template <typename T, int P>
-__global__ __launch_bounds__(256) void k_spread_zfwd(PmPmeLaunch a, PmFftPlan p, const longlong4* __restrict__ pos64) {
+// ADJ: grid 0 takes the charges, grid 1 their derivative along the direction
+// slot_v, q v . grad W (k_spread_dir)
+template <typename T, int P, bool ADJ>
+__global__ __launch_bounds__(256) void k_spread_zfwd(PmPmeLaunch a, PmFftPlan p, const longlong4* __restrict__ pos64,
+                                                     const double4* __restrict__ slot_v) {
   pme_priority(a.prio);
   typedef typename Cx<T>::t T2;
   constexpr int LX = PM_SZ_LX;
@@ -833,6 +849,14 @@ __global__ __launch_bounds__(256) void k_spread_zfwd(PmPmeLaunch a, PmFftPlan p,
     bspline<T, P>(wy, ty, dy);
     bspline<T, P>(wz, tz, dz);
     const T q = (T)a.q[at];
+    const bool dir = ADJ && a.grid0 + blockIdx.y == 1;   // uniform over the block
+    T vx = 0, vy = 0, vz = 0;
+    if (dir) {
+      const double4 v = slot_v[sl];
+      vx = (T)(v.x * a.hr[0]) * q;
+      vy = (T)(v.y * a.hr[1]) * q;
+      vz = (T)(v.z * a.hr[2]) * q;
+    }
     int gzs[P];
 #pragma unroll
     for (int k = 0; k < P; k++) gzs[k] = wrap_grid(iz + off + k, a.nz);
@@ -844,12 +868,14 @@ __global__ __launch_bounds__(256) void k_spread_zfwd(PmPmeLaunch a, PmFftPlan p,
       for (int j = 0; j < P; j++) {
         if (!((my >> j) & 1u)) continue;
         const T qab = qa * ty[j];
+        const T cxy = vx * dx[i] * ty[j] + vy * tx[i] * dy[j], cz = vz * tx[i] * ty[j];
         unsigned long long* line = acc + (lxs[i] * LY + lys[j]) * n;
 #pragma unroll
         for (int k = 0; k < P; k++) {
+          const T val = dir ? cxy * tz[k] + cz * dz[k] : qab * tz[k];
           long long v;
-          if constexpr (sizeof(T) == 4) v = __float2ll_rn(qab * tz[k] * scale);
-          else v = __double2ll_rn(qab * tz[k] * scale);
+          if constexpr (sizeof(T) == 4) v = __float2ll_rn(val * scale);
+          else v = __double2ll_rn(val * scale);
           atomicAdd(line + gzs[k], (unsigned long long)v);
         }
       }
@@ -866,7 +892,7 @@ __global__ __launch_bounds__(256) void k_spread_zfwd(PmPmeLaunch a, PmFftPlan p,
   }
   __syncthreads();
   T2* r = fft_lines<T, T2>(b0, b1, TL, p, tws, -1, ls);
-  T2* gc = reinterpret_cast<T2*>(a.grid_c);
+  T2* gc = grid_c_of<T2>(a);
   const int nl_tot = a.nx * a.ny;
   for (int e = threadIdx.x; e < TL * nzc; e += blockDim.x) {
     int l, k;
@@ -992,7 +1018,7 @@ __global__ __launch_bounds__(256) void k_fft_y(PmPmeLaunch a, PmFftPlan p, int T
     s_off[threadIdx.x] = line < nl ? (long long)x * a.ny * a.nzc + kz : -1;
   }
   __syncthreads();
-  T2* gc = reinterpret_cast<T2*>(a.grid_c);
+  T2* gc = grid_c_of<T2>(a);
   for (int e = threadIdx.x; e < TL * n; e += blockDim.x) {
     const int y = e / TL, l = e - y * TL;
     const long long o = s_off[l];
@@ -1033,7 +1059,7 @@ __global__ __launch_bounds__(256) void k_fft_x_conv(PmPmeLaunch a, PmFftPlan p, 
   }
   __syncthreads();
   const long long xs = (long long)a.ny * a.nzc;   // grid stride of x
-  T2* gc = reinterpret_cast<T2*>(a.grid_c);
+  T2* gc = grid_c_of<T2>(a);
   for (int e = threadIdx.x; e < TL * n; e += blockDim.x) {
     const int x = e / TL, l = e - x * TL;
     const int y = s_y[l];
@@ -1124,7 +1150,7 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(PmPmeLaunch a, PmFftPlan p, i
   T2* tws = b1 + TL * ls;
   load_twiddles(tws, p, a.tw);
   const int line0 = blockIdx.x * TL;
-  const T2* gc = reinterpret_cast<const T2*>(a.grid_c);
+  const T2* gc = grid_c_of<T2>(a);
   if (a.plane) {
     for (int e = threadIdx.x; e < TL * n; e += blockDim.x) {
       const int k = e / TL, l = e - k * TL;
@@ -1150,7 +1176,7 @@ __global__ __launch_bounds__(256) void k_fft_z_inv(PmPmeLaunch a, PmFftPlan p, i
   }
   __syncthreads();
   T2* r = fft_lines<T, T2>(b0, b1, TL, p, tws, +1, ls);
-  T* g = reinterpret_cast<T*>(a.grid_r);
+  T* g = grid_r_of<T>(a);
   for (int e = threadIdx.x; e < TL * n; e += blockDim.x) {
     const int l = e / n, k = e - l * n;
     const int line = line0 + l;
@@ -1208,13 +1234,14 @@ static int plane_threads(const PmFftPlan& px, const PmFftPlan& py) {
 // them in one kernel per kz plane, then z inverse: the fixed-point charge
 // grid to the real potential grid
 template <typename T>
-static void launch_fft_chain(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, bool z_done = false) {
+static void launch_fft_chain(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, bool z_done = false,
+                             int ngrid = 1) {
   const size_t el = sizeof(typename Cx<T>::t);
   const int nthreads = 256;
   if (!z_done) {
     const int tl = lines_per_block(a.nz, el);
     const int nb = (a.nx * a.ny + tl - 1) / tl;
-    hipLaunchKernelGGL(k_fft_z_fwd<T>, dim3(nb), dim3(nthreads), zpass_lds(a.nz, tl, el), s, a, plans[2], tl);
+    hipLaunchKernelGGL(k_fft_z_fwd<T>, dim3(nb, ngrid), dim3(nthreads), zpass_lds(a.nz, tl, el), s, a, plans[2], tl);
   }
   if (a.plane) {
     hipLaunchKernelGGL(k_fft_plane<T>, dim3(a.nzc), dim3(plane_threads(plans[0], plans[1])),
@@ -1223,23 +1250,23 @@ static void launch_fft_chain(hipStream_t s, const PmPmeLaunch& a, const PmFftPla
     {
       const int tl = lines_per_block(a.ny, el);
       const int nb = (a.nx * a.nzc + tl - 1) / tl;
-      hipLaunchKernelGGL(k_fft_y<T>, dim3(nb), dim3(nthreads), line_lds(a.ny, tl, el), s, a, plans[1], tl, -1);
+      hipLaunchKernelGGL(k_fft_y<T>, dim3(nb, ngrid), dim3(nthreads), line_lds(a.ny, tl, el), s, a, plans[1], tl, -1);
     }
     {
       const int tl = lines_per_block(a.nx, el);
       const int nb = (a.ny * a.nzc + tl - 1) / tl;
-      hipLaunchKernelGGL(k_fft_x_conv<T>, dim3(nb), dim3(nthreads), line_lds(a.nx, tl, el), s, a, plans[0], tl);
+      hipLaunchKernelGGL(k_fft_x_conv<T>, dim3(nb, ngrid), dim3(nthreads), line_lds(a.nx, tl, el), s, a, plans[0], tl);
     }
     {
       const int tl = lines_per_block(a.ny, el);
       const int nb = (a.nx * a.nzc + tl - 1) / tl;
-      hipLaunchKernelGGL(k_fft_y<T>, dim3(nb), dim3(nthreads), line_lds(a.ny, tl, el), s, a, plans[1], tl, +1);
+      hipLaunchKernelGGL(k_fft_y<T>, dim3(nb, ngrid), dim3(nthreads), line_lds(a.ny, tl, el), s, a, plans[1], tl, +1);
     }
   }
   {
     const int tl = lines_per_block(a.nz, el);
     const int nb = (a.nx * a.ny + tl - 1) / tl;
-    hipLaunchKernelGGL(k_fft_z_inv<T>, dim3(nb), dim3(nthreads), zpass_lds(a.nz, tl, el), s, a, plans[2], tl);
+    hipLaunchKernelGGL(k_fft_z_inv<T>, dim3(nb, ngrid), dim3(nthreads), zpass_lds(a.nz, tl, el), s, a, plans[2], tl);
   }
 }
 
@@ -1257,8 +1284,8 @@ static void launch_pme_t(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* p
     const size_t el = sizeof(typename Cx<T>::t);
     const int ly = a.spread_zfwd;
     const int nb = ((a.nx + PM_SZ_LX - 1) / PM_SZ_LX) * ((a.ny + ly - 1) / ly);
-    hipLaunchKernelGGL((k_spread_zfwd<T, P>), dim3(nb), dim3(256), zpass_lds(a.nz, PM_SZ_LX * ly, el), s, a,
-                       plans[2], pos64);
+    hipLaunchKernelGGL((k_spread_zfwd<T, P, false>), dim3(nb), dim3(256), zpass_lds(a.nz, PM_SZ_LX * ly, el), s, a,
+                       plans[2], pos64, nullptr);
     launch_fft_chain<T>(s, a, plans, true);
   } else {
     launch_spread_tile<T, P>(s, a, pos64);
@@ -1270,22 +1297,38 @@ static void launch_pme_t(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* p
 }
 
 // adjoint: mode 0 the reciprocal potential at every atom (dE/dq), mode 1 the
-// reciprocal H v (the gather of grad grad W against phi, then the spread of
-// the directional charge derivative, its potential and the gather of grad W)
+// reciprocal H v: the gather of grad grad W against the charges' potential
+// (grid 0) and of grad W against that of the charges' derivative along the
+// direction (grid 1).  The two convolutions run as one chain of launches;
+// with `kept` grid 0 still holds the potential of these positions and only
+// grid 1 is transformed.
 template <typename T, int P>
-static void launch_pme_adj_t(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, const longlong4* pos64,
-                             int mode, const double4* slot_v, double* out) {
+static void launch_pme_adj_t(hipStream_t s, const PmPmeLaunch& a0, const PmFftPlan* plans, const longlong4* pos64,
+                             int mode, bool kept, const double4* slot_v, double* out) {
+  PmPmeLaunch a = a0;
   const dim3 g((a.nslot_max + 255) / 256), b(256);
-  launch_spread_tile<T, P>(s, a, pos64);
-  launch_fft_chain<T>(s, a, plans);
-  if (mode == 0) {
-    hipLaunchKernelGGL((k_gather_adj<T, P, 0>), g, b, 0, s, a, pos64, slot_v, out);
-    return;
+  a.grid0 = mode == 1 && kept ? 1 : 0;
+  const int ngrid = mode == 1 && !kept ? 2 : 1;
+  const size_t el = sizeof(typename Cx<T>::t);
+  if (a.spread_zfwd) {
+    const int ly = a.spread_zfwd;
+    const int nb = ((a.nx + PM_SZ_LX - 1) / PM_SZ_LX) * ((a.ny + ly - 1) / ly);
+    hipLaunchKernelGGL((k_spread_zfwd<T, P, true>), dim3(nb, ngrid), dim3(256), zpass_lds(a.nz, PM_SZ_LX * ly, el), s,
+                       a, plans[2], pos64, slot_v);
+  } else {
+    const int tl = lines_per_block(a.nz, el);
+    const int nb = (a.nx * a.ny + tl - 1) / tl;
+    for (int k = a.grid0; k < a.grid0 + ngrid; k++) {
+      PmPmeLaunch z = a;
+      z.grid0 = k;
+      if (k == 0) launch_spread_tile<T, P>(s, z, pos64);
+      else hipLaunchKernelGGL((k_spread_dir<T, P>), g, b, 0, s, z, pos64, slot_v);
+      hipLaunchKernelGGL(k_fft_z_fwd<T>, dim3(nb), dim3(256), zpass_lds(a.nz, tl, el), s, z, plans[2], tl);
+    }
   }
-  hipLaunchKernelGGL((k_gather_adj<T, P, 1>), g, b, 0, s, a, pos64, slot_v, out);
-  hipLaunchKernelGGL((k_spread_dir<T, P>), g, b, 0, s, a, pos64, slot_v);
-  launch_fft_chain<T>(s, a, plans);
-  hipLaunchKernelGGL((k_gather_adj<T, P, 2>), g, b, 0, s, a, pos64, slot_v, out);
+  launch_fft_chain<T>(s, a, plans, true, ngrid);
+  if (mode == 0) hipLaunchKernelGGL((k_gather_adj<T, P, 0>), g, b, 0, s, a, pos64, slot_v, out);
+  else hipLaunchKernelGGL((k_gather_adj<T, P, 1>), g, b, 0, s, a, pos64, slot_v, out);
 }
 
 int pm_pme_spread_zfwd_fits(const PmPmeLaunch& a, int precision) {
@@ -1329,22 +1372,22 @@ static bool launch_pme_p(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* p
 
 template <typename T>
 static bool launch_pme_adj_p(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, const longlong4* pos64,
-                             int mode, const double4* sv, double* out) {
+                             int mode, bool kept, const double4* sv, double* out) {
   switch (a.order) {
-    case 2: launch_pme_adj_t<T, 2>(s, a, plans, pos64, mode, sv, out); return true;
-    case 4: launch_pme_adj_t<T, 4>(s, a, plans, pos64, mode, sv, out); return true;
-    case 6: launch_pme_adj_t<T, 6>(s, a, plans, pos64, mode, sv, out); return true;
-    case 8: launch_pme_adj_t<T, 8>(s, a, plans, pos64, mode, sv, out); return true;
-    case 10: launch_pme_adj_t<T, 10>(s, a, plans, pos64, mode, sv, out); return true;
-    case 12: launch_pme_adj_t<T, 12>(s, a, plans, pos64, mode, sv, out); return true;
+    case 2: launch_pme_adj_t<T, 2>(s, a, plans, pos64, mode, kept, sv, out); return true;
+    case 4: launch_pme_adj_t<T, 4>(s, a, plans, pos64, mode, kept, sv, out); return true;
+    case 6: launch_pme_adj_t<T, 6>(s, a, plans, pos64, mode, kept, sv, out); return true;
+    case 8: launch_pme_adj_t<T, 8>(s, a, plans, pos64, mode, kept, sv, out); return true;
+    case 10: launch_pme_adj_t<T, 10>(s, a, plans, pos64, mode, kept, sv, out); return true;
+    case 12: launch_pme_adj_t<T, 12>(s, a, plans, pos64, mode, kept, sv, out); return true;
     default: return false;
   }
 }
 
 bool pm_launch_pme_adjoint(hipStream_t s, const PmPmeLaunch& a, const PmFftPlan* plans, const longlong4* pos64,
-                           int precision, int mode, const double4* slot_v, double* out) {
-  if (precision == 1) return launch_pme_adj_p<double>(s, a, plans, pos64, mode, slot_v, out);
-  return launch_pme_adj_p<float>(s, a, plans, pos64, mode, slot_v, out);
+                           int precision, int mode, bool kept, const double4* slot_v, double* out) {
+  if (precision == 1) return launch_pme_adj_p<double>(s, a, plans, pos64, mode, kept, slot_v, out);
+  return launch_pme_adj_p<float>(s, a, plans, pos64, mode, kept, slot_v, out);
 }
 
 void pm_launch_pme_theta(hipStream_t s, const PmPmeLaunch& a, int precision) {
