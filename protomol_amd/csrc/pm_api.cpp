@@ -34,6 +34,8 @@
 #define PM_PRUNE_SKIN_AUTO 0.0
 // waves up to which a cluster's list is shared by several (pair_split)
 #define PM_SPLIT_WAVES 1024
+// values of x or v up to which pm_md_get_state copies through pinned memory
+#define PM_STAGE_STATE 65536
 // work space that a context keeps between pm_lanczos calls
 #define PM_LANCZOS_KEEP_BYTES (256u << 20)
 
@@ -155,6 +157,9 @@ struct pm_context {
   int *d_ex_row = nullptr, *d_ex_partner = nullptr, *d_ex_cls = nullptr;      // lookup CSR
   int *d_xs_row = nullptr, *d_xs_part = nullptr;   // resolved exclusions, both directions
   int xs_maxdeg = 0;
+  double q_sum = 0, q2_sum = 0;      // of the charges and their squares
+  double* h_stage = nullptr;         // pinned host memory for results (host_stage)
+  size_t h_stage_n = 0;
   unsigned long long lj_types = 0;   // bit t: type t has Lennard-Jones parameters with some type
   int *d_cx_row = nullptr, *d_cx_partner = nullptr, *d_cx_cls = nullptr;      // correction CSR
   int *d_tab_a = nullptr, *d_tab_b = nullptr, *d_tab_c = nullptr;
@@ -546,10 +551,12 @@ static int adjoint_split(const pm_context* c) {
   return s;
 }
 
-// The types with Lennard-Jones parameters, for the pair kernel to leave the
-// others' terms out.  With an uncharged atom every type counts: two atoms on
+// What the passes need of the charges: their sums, and the types with
+// Lennard-Jones parameters, for the pair kernel to leave the others' terms out.  With an uncharged atom every type counts: two atoms on
 // one point then still show as a force that is not finite.
-static void set_lj_types(pm_context* c) {
+static void set_charge_data(pm_context* c) {
+  c->q2_sum = c->q_sum = 0.0;
+  for (double q : c->q) { c->q2_sum += q * q; c->q_sum += q; }
   c->lj_types = 0;
   const int T = c->ntypes;
   for (int a = 0; a < T; a++)
@@ -1438,9 +1445,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     }
     if (f.corr && !adj) {
       // point self energy and charged-system term (:604-628)
-      double q2 = 0.0, qs = 0.0;
-      for (int i = 0; i < n; i++) q2 += c->q[i] * c->q[i];
-      for (int i = 0; i < n; i++) qs += c->q[i];
+      const double q2 = c->q2_sum, qs = c->q_sum;
       const_coul += -q2 * f.alpha / std::sqrt(kPi);
       if (std::fabs(qs * 0.00268283) > 1.0e-5) {
         double V = c->box.L[0] * c->box.L[1] * c->box.L[2];
@@ -1605,11 +1610,33 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   return PM_OK;
 }
 
-int check_overflow(pm_context* c) {
+// pinned host memory for `count` doubles, kept for the context's next calls: a
+// copy into pageable memory makes the host wait for the stream each time
+double* host_stage(pm_context* c, size_t count) {
+  if (count <= c->h_stage_n) return c->h_stage;
+  if (c->h_stage) (void)hipHostFree(c->h_stage);
+  c->h_stage = nullptr;
+  c->h_stage_n = 0;
+  void* p = nullptr;
+  if (hipHostMalloc(&p, count * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  c->h_stage = static_cast<double*>(p);
+  c->h_stage_n = count;
+  return c->h_stage;
+}
+
+// what the kernels flagged, as read from the device (`word`, or nullptr: read it)
+int check_overflow(pm_context* c, const int* word = nullptr) {
   if (!c->d_overflow) return PM_OK;
   int ov = 0;
-  HIPCHECK(c, hipMemcpyAsync(&ov, c->d_overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  if (word) {
+    ov = *word;
+  } else {
+    HIPCHECK(c, hipMemcpyAsync(&ov, c->d_overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+  }
   if (ov) {
     HIPCHECK(c, hipMemset(c->d_overflow, 0, sizeof(int)));
     if (ov & PM_FLAG_NONFINITE)
@@ -1777,6 +1804,9 @@ PmConstraints constraint_launch(pm_context* c, double eps, int max_iter, double 
 }
 
 void free_all(pm_context* c) {
+  if (c->h_stage) (void)hipHostFree(c->h_stage);
+  c->h_stage = nullptr;
+  c->h_stage_n = 0;
   dfree(c->d_q); dfree(c->d_mass); dfree(c->d_type); dfree(c->d_mol);
   dfree(c->d_ex_row); dfree(c->d_ex_partner); dfree(c->d_ex_cls);
   dfree(c->d_xs_row); dfree(c->d_xs_part); dfree(c->d_jmask);
@@ -2035,7 +2065,7 @@ int pm_set_topology(pm_context* c, int n, const double* q, const int* type, int 
     }
   }
   // LJ tables with one extra all-zero type for padding slots
-  set_lj_types(c);
+  set_charge_data(c);
   int t1 = ntypes + 1;
   std::vector<float4> ljf(t1 * t1, make_float4(0, 0, 0, 0));
   std::vector<double4> ljd(t1 * t1, make_double4(0, 0, 0, 0));
@@ -2067,6 +2097,7 @@ int pm_set_topology(pm_context* c, int n, const double* q, const int* type, int 
   if ((r = dalloc(c, &c->d_force, 3 * (size_t)n))) return r;
   if ((r = dalloc(c, &c->d_force_side, 3 * (size_t)n))) return r;
   if ((r = dalloc(c, &c->d_scratch3, 3 * (size_t)n))) return r;
+  host_stage(c, (3 * (size_t)n <= PM_STAGE_STATE ? 6 : 3) * (size_t)n + PM_NE + 1);   // (calls go without where there is none)
   if ((r = dalloc(c, &c->d_energy, PM_NE))) return r;
   HIPCHECK(c, hipMemset(c->d_energy, 0, PM_NE * sizeof(double)));
   for (auto& f : c->forces) f.cached = false;
@@ -2296,12 +2327,25 @@ int pm_evaluate(pm_context* c, const int* handles, int nh, const double* positio
   std::vector<int> hv(handles, handles + nh);
   if ((r = evaluate_group(c, hv, flags))) return r;
   pm_launch_fix_to_double(c->stream, 3 * n, c->d_force, c->d_scratch3);
-  std::vector<double> f(3 * (size_t)n), e(PM_NE);
-  HIPCHECK(c, hipMemcpyAsync(f.data(), c->d_scratch3, 3 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipMemcpyAsync(e.data(), c->d_energy, PM_NE * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  if ((r = check_overflow(c))) return r;
-  for (size_t k = 0; k < f.size(); k++) forces[k] += f[k];
+  // energies, the error word and the forces through pinned memory, one wait
+  // (pageable where none is to be had)
+  const size_t n3 = 3 * (size_t)n;
+  std::vector<double> pageable;
+  double* h = host_stage(c, n3 + PM_NE + 1);
+  if (!h) {
+    pageable.resize(n3 + PM_NE + 1);
+    h = pageable.data();
+  }
+  double *e = h, *f = h + PM_NE + 1;
+  int* word = c->d_overflow ? reinterpret_cast<int*>(h + PM_NE) : nullptr;
+  hipError_t he = hipMemcpyAsync(f, c->d_scratch3, n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  if (he == hipSuccess) he = hipMemcpyAsync(e, c->d_energy, PM_NE * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  if (he == hipSuccess && word) he = hipMemcpyAsync(word, c->d_overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+  const hipError_t hs = hipStreamSynchronize(c->stream);
+  HIPCHECK(c, he);
+  HIPCHECK(c, hs);
+  if ((r = check_overflow(c, word))) return r;
+  for (size_t k = 0; k < n3; k++) forces[k] += f[k];
   for (int k = 0; k < PM_NE; k++) energies[k] += e[k];
   c->md_forces_valid = false;
   c->gen++;
@@ -2795,12 +2839,33 @@ int pm_md_get_state(pm_context* c, double* x, double* v, double* energies) {
   if (!c) return PM_ERR_ARGUMENT;
   int r;
   if ((r = set_device(c))) return r;
-  const size_t bytes = 3 * (size_t)c->n * sizeof(double);
-  if (x) HIPCHECK(c, hipMemcpyAsync(x, c->d_pos, bytes, hipMemcpyDeviceToHost, c->stream));
-  if (v) HIPCHECK(c, hipMemcpyAsync(v, c->d_vel, bytes, hipMemcpyDeviceToHost, c->stream));
-  if (energies) HIPCHECK(c, hipMemcpyAsync(energies, c->d_energy, PM_NE * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
-  return check_overflow(c);
+  // small boxes: all results through pinned memory with one wait; large arrays
+  // go straight to the caller, whose copy would take longer than the wait
+  const size_t n3 = 3 * (size_t)c->n;
+  const bool staged = n3 <= PM_STAGE_STATE;
+  double* h = host_stage(c, (staged ? 2 * n3 : 0) + PM_NE + 1);
+  std::vector<double> pageable;
+  if (!h) {
+    pageable.resize((staged ? 2 * n3 : 0) + PM_NE + 1);
+    h = pageable.data();
+  }
+  int* word = c->d_overflow ? reinterpret_cast<int*>(h + PM_NE) : nullptr;
+  double *hx = staged ? h + PM_NE + 1 : x, *hv = staged ? hx + n3 : v;
+  hipError_t he = hipSuccess;
+  auto get = [&](void* dst, const void* src, size_t bytes) {
+    if (he == hipSuccess) he = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
+  };
+  if (x) get(hx, c->d_pos, n3 * sizeof(double));
+  if (v) get(hv, c->d_vel, n3 * sizeof(double));
+  if (energies) get(h, c->d_energy, PM_NE * sizeof(double));
+  if (word) get(word, c->d_overflow, sizeof(int));
+  const hipError_t hs = hipStreamSynchronize(c->stream);
+  HIPCHECK(c, he);
+  HIPCHECK(c, hs);
+  if (staged && x) std::copy(hx, hx + n3, x);
+  if (staged && v) std::copy(hv, hv + n3, v);
+  if (energies) std::copy(h, h + PM_NE, energies);
+  return check_overflow(c, word);
 }
 
 int pm_last_stats(pm_context* c, long long* stats, int nstats) {
@@ -2942,7 +3007,7 @@ int pm_set_charges(pm_context* c, const double* q) {
     if (!std::isfinite(q[i])) return fail(c, PM_ERR_ARGUMENT, "charge %d is not finite", i);
   c->q.assign(q, q + c->n);
   const unsigned long long types = c->lj_types;
-  set_lj_types(c);
+  set_charge_data(c);
   if (c->lj_types != types) c->gen++;   // a kernel argument of captured MD steps
   // same size: the copy keeps the device address, so captured MD steps stay valid
   HIPCHECK(c, hipMemcpy(c->d_q, c->q.data(), c->q.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -3611,14 +3676,21 @@ int pm_batch_exchange(pm_batch* b, int attempt, unsigned long long seed, int* ac
   if (hipSetDevice(b->ctx[0]->device) != hipSuccess) return bfail(b, PM_ERR_DEVICE, "hipSetDevice failed");
   // potential energy of every replica at its last step (ScalarStructure::potentialEnergy)
   std::vector<double> epot(R, 0.0);
+  // (all copies are queued, into pinned memory, before the first is waited for)
+  bool ok = true;
+  std::vector<std::array<double, PM_NE>> pageable(R);
+  std::vector<double*> e(R);
   for (int k = 0; k < R; k++) {
     pm_context* c = b->ctx[k];
-    double e[PM_NE];
-    if (hipMemcpyAsync(e, c->d_energy, sizeof(e), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-        hipStreamSynchronize(c->stream) != hipSuccess)
-      return bfail(b, PM_ERR_DEVICE, "energy copy failed");
-    for (int u = 0; u < PM_E_VIR; u++) epot[k] += e[u];
+    e[k] = host_stage(c, PM_NE);
+    if (!e[k]) e[k] = pageable[k].data();
+    ok = hipMemcpyAsync(e[k], c->d_energy, PM_NE * sizeof(double), hipMemcpyDeviceToHost, c->stream) == hipSuccess && ok;
   }
+  for (int k = 0; k < R; k++) {
+    ok = hipStreamSynchronize(b->ctx[k]->stream) == hipSuccess && ok;
+    for (int u = 0; ok && u < PM_E_VIR; u++) epot[k] += e[k][u];
+  }
+  if (!ok) return bfail(b, PM_ERR_DEVICE, "energy copy failed");
   // neighbour pairs (k, k+1) of the ladder with k of the attempt's parity
   // (getNextAddress, applications/rem-app/rem.cpp:949-957); the Metropolis
   // test on calcDelta (:941-946, canDoEvenSwitch :841-880) swaps the two
@@ -3646,9 +3718,10 @@ int pm_batch_exchange(pm_batch* b, int attempt, unsigned long long seed, int* ac
         return bfail(b, PM_ERR_DEVICE, "temperature copy failed");
       if (b->exchange_velocities == PM_EXCHANGE_RESCALE)
         pm_launch_scale(c->stream, 3 * c->n, std::sqrt(tnew[u] / told[u]), c->d_vel);
-      if (hipStreamSynchronize(c->stream) != hipSuccess) return bfail(b, PM_ERR_DEVICE, "exchange failed");
     }
   }
+  for (pm_context* c : b->ctx) ok = hipStreamSynchronize(c->stream) == hipSuccess && ok;
+  if (!ok) return bfail(b, PM_ERR_DEVICE, "exchange failed");
   return PM_OK;
 }
 
