@@ -11,17 +11,33 @@
 // atoms, so a sweep over the whole list is, group by group, a sweep over each
 // group's constraints in their list order: one thread per group repeats the
 // reference's FP64 operations (no contraction) exactly.  Only the number of
-// sweeps is global.  A probe kernel records the error after 0 .. maxIter
-// sweeps (on copies of the positions or velocities), summed per block; every
-// block of the apply kernel sums those parts in the same fixed order into the
-// mean error, finds the first sweep count whose mean is within epsilon and
-// runs that many sweeps on the real positions and velocities.  Groups of up
-// to 4 atoms (waters, methyl groups) keep their atoms in registers.
+// sweeps is global.  A probe kernel records the error after 0 ..
+// PM_PROBE_FIRST sweeps (on copies of the positions or velocities), summed per
+// wave; a second launch sums those parts in a fixed order into the mean errors
+// and, where none is within epsilon, records the errors up to maxIter sweeps.
+// Every block of the apply kernel finds the first sweep count whose mean is
+// within epsilon in the same way and runs that many sweeps on the real
+// positions and velocities.  Groups of up to 4 atoms (waters, methyl groups)
+// keep their atoms in registers.
+//
+// Each group is one serial FP64 chain, and 98k water atoms are only 512 waves:
+// latency bounds both kernels.  Hence the short first probe (the steps of a
+// run need far fewer sweeps than maxIter allows), loads that wait for no
+// branch, and blocks of one wave while that spreads them over more CUs.  98k
+// water: probe 41 us, apply 45 us with 30 probed sweeps, blocks of four waves
+// and the groups loaded after the sums; 24 + 8 (the second launch) + 26 us now.
 #include "pm_internal.h"
 
 #include <math.h>
 
 #include <mutex>
+
+// Sweeps whose errors the first probe records: water at 2 fs and epsilon 1e-5
+// needs 12 or 13, a sweep of the probe takes 1 us, and a count beyond the first
+// probe repeats it (98k water, 25 steps: 9.02 ms at 16, 9.13 at 30, 9.64 at 12)
+#define PM_PROBE_FIRST 16
+// waves up to which a block is one wave
+#define PM_CONS_WAVE_BLOCKS 1024
 
 namespace {
 
@@ -154,7 +170,11 @@ __device__ inline void rload(Reg4& r, const double* src, int4 at) {
 #pragma unroll
   for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int d = 0; d < 3; d++) r.p[i][d] = a[i] >= 0 ? src[3 * a[i] + d] : 0.0;
+    for (int d = 0; d < 3; d++) {
+      // (a slot that is not used reads the first atom: no load waits for a branch)
+      const double t = src[3 * (a[i] >= 0 ? a[i] : a[0]) + d];
+      r.p[i][d] = a[i] >= 0 ? t : 0.0;
+    }
 }
 __device__ inline void rstore(const Reg4& r, double* dst, int4 at) {
   const int a[4] = {at.x, at.y, at.z, at.w};
@@ -381,13 +401,54 @@ __device__ inline void wave_part(double e, double* part, long long at) {
   if ((threadIdx.x & 63) == 0) part[at] = e;
 }
 
-// probe: every group's error after 0 .. maxit sweeps, summed per wave into
+// the first sweep count up to `upto` whose mean error, the sum of the nw wave
+// parts (lanes in a fixed order) over the constraints, is within eps; -1 if
+// none is.  Called by whole blocks; the first wave sums
+__device__ inline int find_sweeps(const PmConstraints& c, int nw, int upto) {
+  __shared__ int s_found;
+  if (threadIdx.x < 64) {
+    int found = -1;
+    // eight counts at a time, 32 loads in flight: each load takes most of a
+    // microsecond
+    constexpr int Q = 8, U = 4;
+    for (int s0 = 0; s0 <= upto && found < 0; s0 += Q) {
+      double t[Q];
+#pragma unroll
+      for (int q = 0; q < Q; q++) t[q] = 0.0;
+      for (int u0 = threadIdx.x; u0 < nw; u0 += 64 * U) {
+        double e[U][Q];
+#pragma unroll
+        for (int k = 0; k < U; k++)
+#pragma unroll
+          for (int q = 0; q < Q; q++) e[k][q] = c.err[(long long)min(s0 + q, upto) * nw + min(u0 + 64 * k, nw - 1)];
+#pragma unroll
+        for (int k = 0; k < U; k++)
+#pragma unroll
+          for (int q = 0; q < Q; q++) t[q] += u0 + 64 * k < nw ? e[k][q] : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) t[q] += __shfl_down(t[q], off, 64);
+        const double mean = __shfl(t[q], 0, 64) / c.ncons;
+        if (found < 0 && s0 + q <= upto && !(mean > c.eps)) found = s0 + q;
+      }
+    }
+    if (threadIdx.x == 0) s_found = found;
+  }
+  __syncthreads();
+  return s_found;
+}
+
+// probe: every group's error after from .. to sweeps, summed per wave into
 // part[s * waves + wave]; small groups in registers, larger ones on a
-// scratch copy of their atoms' positions (SHAKE) or velocities (RATTLE)
+// scratch copy of their atoms' positions (SHAKE) or velocities (RATTLE).
+// Nothing to do when a count below `from` is within eps already.
 template <bool RATTLE>
 __global__ __launch_bounds__(256) void k_constraint_probe(PmConstraints c, const double* __restrict__ x,
                                                           const double* __restrict__ v,
-                                                          const double* __restrict__ xl) {
+                                                          const double* __restrict__ xl, int from, int to) {
+  if (from > 0 && find_sweeps(c, gridDim.x * (blockDim.x >> 6), from - 1) >= 0) return;
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int nw = gridDim.x * (blockDim.x >> 6), gw = g >> 6;
   const bool valid = g < c.ngroup;
@@ -415,14 +476,16 @@ __global__ __launch_bounds__(256) void k_constraint_probe(PmConstraints c, const
     }
   }
   for (int it = 0;; it++) {
-    double e = 0.0;
-    if (small) {
-      e = error_r<RATTLE>(q, water, X, V);
-    } else if (valid) {
-      for (int k = k0; k < k1; k++) e += RATTLE ? rattle_err(c, x, c.scratch, k) : shake_err(c, c.scratch, k);
+    if (it >= from) {
+      double e = 0.0;
+      if (small) {
+        e = error_r<RATTLE>(q, water, X, V);
+      } else if (valid) {
+        for (int k = k0; k < k1; k++) e += RATTLE ? rattle_err(c, x, c.scratch, k) : shake_err(c, c.scratch, k);
+      }
+      wave_part(e, c.err, (long long)it * nw + gw);
     }
-    wave_part(e, c.err, (long long)it * nw + gw);
-    if (it == c.maxit) break;
+    if (it == to) break;
     if (small) {
       sweep_r<RATTLE, false>(q, water, c.dt, X, V, XL);
     } else if (valid) {
@@ -434,49 +497,30 @@ __global__ __launch_bounds__(256) void k_constraint_probe(PmConstraints c, const
   }
 }
 
-// apply: every block sums the probe's wave parts in the same fixed order to
-// the mean error after s sweeps (four sweep counts at a time, one per wave)
-// and takes the reference's sweep count (the first s with mean <= eps, or
-// maxit + 1); then that many sweeps on x and v, and SHAKE records x as the
-// next reference positions
+// apply: the reference's sweep count (the first s with mean <= eps, or
+// maxit + 1) from the probe's parts; then that many sweeps on x and v, and
+// SHAKE records x as the next reference positions
 template <bool RATTLE>
 __global__ __launch_bounds__(256) void k_constraint_apply(PmConstraints c, double* __restrict__ x,
                                                           double* __restrict__ v, double* __restrict__ xl) {
-  __shared__ double s_mean[4];
-  __shared__ int s_sweeps;
-  const int nw = gridDim.x * (blockDim.x >> 6);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (threadIdx.x == 0) s_sweeps = -1;
-  for (int s0 = 0; s0 <= c.maxit; s0 += 4) {
-    const int s = s0 + w;
-    double t = 0.0;
-    if (s <= c.maxit)
-      for (int u = lane; u < nw; u += 64) t += c.err[(long long)s * nw + u];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
-    if (lane == 0) s_mean[w] = t / c.ncons;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int u = 0; u < 4 && s0 + u <= c.maxit; u++)
-        if (!(s_mean[u] > c.eps)) { s_sweeps = s0 + u; break; }
-    __syncthreads();
-    if (s_sweeps >= 0) break;
-  }
-  if (s_sweeps < 0) s_sweeps = c.maxit + 1;   // every thread writes the same value
-  __syncthreads();
-  const int sweeps = s_sweeps;
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g == 0 && c.sweeps) c.sweeps[0] = sweeps;
-  if (g >= c.ngroup) return;
-  const int k0 = c.gstart[g], k1 = c.gstart[g + 1];
-  const int4 at = c.gatom[g];
-  if (at.x >= 0) {
-    Reg4 X, V, XL;
-    Cons6 q;
+  const bool valid = g < c.ngroup;
+  const int k0 = valid ? c.gstart[g] : 0, k1 = valid ? c.gstart[g + 1] : 0;
+  const int4 at = valid ? c.gatom[g] : make_int4(-1, -1, -1, -1);
+  const bool small = valid && at.x >= 0;
+  // the group's data in flight while the error parts are summed
+  Reg4 X, V, XL;
+  Cons6 q;
+  if (small) {
     load_cons(c, k0, k1, q);
     rload(X, x, at);
     rload(V, v, at);
     if (!RATTLE) rload(XL, xl, at);
+  }
+  const int found = find_sweeps(c, gridDim.x * (blockDim.x >> 6), c.maxit);
+  const int sweeps = found >= 0 ? found : c.maxit + 1;
+  if (g == 0 && c.sweeps) c.sweeps[0] = sweeps;
+  if (small) {
     const bool water = at.w == PM_CONS_WATER;
     for (int it = 0; it < sweeps; it++) sweep_r<RATTLE, true>(q, water, c.dt, X, V, XL);
     if (!RATTLE) {
@@ -539,12 +583,17 @@ bool pm_launch_constraints(hipStream_t s, const PmConstraints& c, int rattle, do
     return true;
   }
   if (c.ngroup <= 0) return true;
-  const dim3 g((c.ngroup + 255) / 256), b(256);
+  // blocks of one wave while a CU holds a few of them
+  const int threads = c.ngroup <= PM_CONS_WAVE_BLOCKS * 64 ? 64 : 256;
+  const dim3 g((c.ngroup + threads - 1) / threads), b(threads);
+  const int first = c.maxit < PM_PROBE_FIRST ? c.maxit : PM_PROBE_FIRST;
   if (rattle) {
-    hipLaunchKernelGGL(k_constraint_probe<true>, g, b, 0, s, c, x, v, xl);
+    hipLaunchKernelGGL(k_constraint_probe<true>, g, b, 0, s, c, x, v, xl, 0, first);
+    if (first < c.maxit) hipLaunchKernelGGL(k_constraint_probe<true>, g, b, 0, s, c, x, v, xl, first + 1, c.maxit);
     hipLaunchKernelGGL(k_constraint_apply<true>, g, b, 0, s, c, x, v, xl);
   } else {
-    hipLaunchKernelGGL(k_constraint_probe<false>, g, b, 0, s, c, x, v, xl);
+    hipLaunchKernelGGL(k_constraint_probe<false>, g, b, 0, s, c, x, v, xl, 0, first);
+    if (first < c.maxit) hipLaunchKernelGGL(k_constraint_probe<false>, g, b, 0, s, c, x, v, xl, first + 1, c.maxit);
     hipLaunchKernelGGL(k_constraint_apply<false>, g, b, 0, s, c, x, v, xl);
   }
   return true;
