@@ -2625,6 +2625,7 @@ int md_unit(pm_context* c, int kind, bool energy) {
   int r;
   PmStepWork w{};
   const bool shake = md_shake(c), rattle = md_rattle(c);
+  bool sw = false;
   if (kind == 0) {
     {
       TimedScope ts(c, PM_T_INTEGRATE);
@@ -2635,15 +2636,17 @@ int md_unit(pm_context* c, int kind, bool energy) {
         const double hh = 0.5 * c->md_dt * kInvTimeFactor;
         pm_launch_kick(s, n, 2, hh, c->d_mass, c->d_force, c->d_vel, c->d_pos);
         md_rattle_step(c);
-        pm_launch_kick(s, n, 2, hh, c->d_mass, c->d_force, c->d_vel, c->d_pos);
-        pm_launch_drift(s, n, h, c->d_vel, c->d_pos);
+        sw = md_step_work(c, &w);
+        pm_launch_kick(s, n, 2, hh, c->d_mass, c->d_force, c->d_vel, c->d_pos, nullptr, sw ? 1 : 0);
+        pm_launch_drift(s, n, h, c->d_vel, c->d_pos, sw && !shake ? &w : nullptr);
       } else {
-        // the displacement test and binning need the final positions: not
-        // in the update when SHAKE moves them afterwards
-        const bool sw = !shake && md_step_work(c, &w);
-        pm_launch_kick(s, n, 1, h, c->d_mass, c->d_force, c->d_vel, c->d_pos, sw ? &w : nullptr, sw ? 1 : 0);
+        sw = md_step_work(c, &w);
+        pm_launch_kick(s, n, 1, h, c->d_mass, c->d_force, c->d_vel, c->d_pos, sw && !shake ? &w : nullptr, sw ? 1 : 0);
       }
+      // the displacement test and binning need the final positions: in the
+      // update, or after SHAKE
       if (shake) md_shake_step(c);
+      if (shake && sw) pm_launch_step_work(s, n, c->d_pos, w);
     }
     if ((r = evaluate_group(c, c->md_handles, 0, energy))) md_step_failed(c);
     return r;
@@ -2651,10 +2654,11 @@ int md_unit(pm_context* c, int kind, bool energy) {
   const double g = c->md_gamma / (1000 * kInvTimeFactor);
   {
     TimedScope ts(c, PM_T_INTEGRATE);
-    const bool sw = !shake && md_step_work(c, &w);
+    sw = md_step_work(c, &w);
     pm_launch_langevin_kick(s, n, h, g, c->d_mass, c->d_force, c->d_vel, c->md_seed, c->d_md, 0, sw ? 1 : 0);
-    pm_launch_drift(s, n, h, c->d_vel, c->d_pos, sw ? &w : nullptr);
+    pm_launch_drift(s, n, h, c->d_vel, c->d_pos, sw && !shake ? &w : nullptr);
     if (shake) md_shake_step(c);   // postDriftOrNextModify (STSIntegrator.cpp:42-47)
+    if (shake && sw) pm_launch_step_work(s, n, c->d_pos, w);
   }
   if ((r = evaluate_group(c, c->md_handles, 0, energy))) {
     md_step_failed(c);

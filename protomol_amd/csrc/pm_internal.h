@@ -389,6 +389,8 @@ struct PmStepWork {
 // next evaluation then needs no clearing of its own)
 void pm_launch_kick(hipStream_t s, int n, int mode, double h, const double* mass, long long* f,
                     double* v, double* x, const PmStepWork* w = nullptr, int zero_f = 0);
+// PmStepWork on positions that a constraint moved after the update
+void pm_launch_step_work(hipStream_t s, int n, const double* x, const PmStepWork& w);
 // MD state the integrator kernels read from device memory
 struct PmMdDevice {
   unsigned long long counter;   // Langevin noise counter (2 per step)

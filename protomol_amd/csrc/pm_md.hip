@@ -421,6 +421,16 @@ __device__ inline void drift_body(const DriftArgs& a, int bx) {
 }
 __global__ void k_drift(DriftArgs a) { drift_body(a, blockIdx.x); }
 
+// The displacement test and binning at positions that SHAKE has moved: one
+// launch bound by its boundary and latency (98k atoms: 5 us) instead of the
+// test, the clearing of the forces and the binning one after the other (17 us)
+__global__ void k_step_work(int n, const double* __restrict__ x, PmStepWork w) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double xn[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
+  step_work(w, i, xn);
+}
+
 // batched launches over replicas (argument tables in device memory)
 __global__ void kb_kick_drift(const KickArgs* __restrict__ t, const int* __restrict__ pre, int nrep) {
   const int r = pm_batch_replica(pre, nrep, blockIdx.x);
@@ -568,6 +578,14 @@ void pm_launch_drift(hipStream_t s, int n, double h, const double* v, double* x,
     return;
   }
   if (n > 0) hipLaunchKernelGGL(k_drift, grid_for(n, 256), dim3(256), 0, s, a);
+}
+
+void pm_launch_step_work(hipStream_t s, int n, const double* x, const PmStepWork& w) {
+  if (pm_recording()) {   // follows constraints, which have no batched form
+    pm_record(-1, 0, 0, 0, 0, nullptr, 0);
+    return;
+  }
+  if (n > 0) hipLaunchKernelGGL(k_step_work, grid_for(n, 256), dim3(256), 0, s, n, x, w);
 }
 
 bool pm_launch_batched_md(hipStream_t s, int kind, int variant, const void* t, const int* pre, int nrep,
