@@ -1240,8 +1240,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, rb);
   }
   pm_launch_scan_cells(s, nc, c->box.n[2], c->d_bin_count, c->d_cell_count, c->d_cell_start, c->d_cell_slot, c->d_counts,
-                       c->d_cluster_cell, c->ncl_max, c->m, rb, c->d_scan_aux);
-  pm_launch_scatter(s, n, c->d_cell_of, c->d_cell_rank, c->d_cell_start, c->d_cell_atoms, rb);
+                       c->d_cluster_cell, c->ncl_max, c->m, rb, c->d_scan_aux, n, c->d_cell_of, c->d_cell_rank, c->d_cell_atoms);
   pm_launch_fill_slots(s, c->box, nc, c->d_pos, c->d_q, c->d_type, c->d_cell_count, c->d_cell_start,
                        c->d_cell_slot, c->d_cell_atoms, c->d_key, c->d_slot_pos,
                        c->precision == PM_PRECISION_DOUBLE ? c->d_slot_pos64 : nullptr, c->d_slot_meta,
@@ -2368,8 +2367,7 @@ int pm_cell_diagnostics(pm_context* c, const double* positions, double algorithm
   pm_launch_zero_i(s, c->d_bin_count, nc);
   pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, nullptr);
   pm_launch_scan_cells(s, nc, c->box.n[2], c->d_bin_count, c->d_cell_count, c->d_cell_start, c->d_cell_slot, c->d_counts,
-                       c->d_cluster_cell, c->ncl_max, c->m, nullptr, c->d_scan_aux);
-  pm_launch_scatter(s, n, c->d_cell_of, c->d_cell_rank, c->d_cell_start, c->d_cell_atoms, nullptr);
+                       c->d_cluster_cell, c->ncl_max, c->m, nullptr, c->d_scan_aux, n, c->d_cell_of, c->d_cell_rank, c->d_cell_atoms);
   std::vector<int> cell(n), cnt(nc), start(nc), atoms(n);
   HIPCHECK(c, hipMemcpyAsync(cell.data(), c->d_cell_of, n * sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHECK(c, hipMemcpyAsync(cnt.data(), c->d_cell_count, nc * sizeof(int), hipMemcpyDeviceToHost, s));

@@ -197,12 +197,11 @@ void pm_launch_bin(hipStream_t s, const PmBox& box, int n, const double* pos, in
 // after its last cell (nz <= 8192).  aux: 2 ints per chunk of whole columns
 // of at most 8192 cells (at most 2 (ncells / 4096 + 2) in all); with more
 // than two chunks (and not recording) the scan runs over many blocks,
-// otherwise in one
+// otherwise in one.  Then the scatter of the n atoms into their cells
+// (cell_atoms), in the same launch for small boxes
 void pm_launch_scan_cells(hipStream_t s, int ncells, int nz, int* bin_count, int* cell_count, int* cell_start,
                           int* cell_slot, int* counts, int* cluster_cell, int ncl_max, int m, const int* rebuild,
-                          int* aux);
-void pm_launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank, const int* cell_start,
-                       int* cell_atoms, const int* rebuild);
+                          int* aux, int n, const int* cell_of, const int* rank, int* cell_atoms);
 // x_prune (may be null): the positions of the last inner-list prune, written
 // on builds and, on kept layouts, when the prune flag rebuild[1] is set
 void pm_launch_fill_slots(hipStream_t s, const PmBox& box, int ncells, const double* pos,

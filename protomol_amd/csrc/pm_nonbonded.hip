@@ -167,7 +167,16 @@ __device__ inline void scan_cells_body(int ncells, int nz, int* __restrict__ cnt
 __global__ __launch_bounds__(1024) void k_scan_cells(int ncells, int nz, int* __restrict__ cnt, int* __restrict__ cnt_out,
                                                      int* __restrict__ start, int* __restrict__ slot,
                                                      int* __restrict__ counts, int* __restrict__ cluster_cell,
-                                                     int ncl_max, int m_cl, const int* __restrict__ rebuild) { scan_cells_body(ncells, nz, cnt, cnt_out, start, slot, counts, cluster_cell, ncl_max, m_cl, rebuild, blockIdx.x); }
+                                                     int ncl_max, int m_cl, const int* __restrict__ rebuild,
+                                                     int n, const int* __restrict__ cell_of, const int* __restrict__ rank,
+                                                     int* __restrict__ cell_atoms) {
+  scan_cells_body(ncells, nz, cnt, cnt_out, start, slot, counts, cluster_cell, ncl_max, m_cl, rebuild, blockIdx.x);
+  if (n == 0 || (rebuild && *rebuild == 0)) return;
+  // the scatter of a small box (n > 0) by the block that wrote the starts
+  __syncthreads();
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 1024) cell_atoms[start[cell_of[i]] + rank[i]] = i;
+}
 struct ScanCellsArgs { int ncells; int nz; int* cnt; int* cnt_out; int* start; int* slot; int* counts; int* cluster_cell; int ncl_max; int m_cl; const int* rebuild; };
 __global__ __launch_bounds__(1024) void kb_scan_cells(const ScanCellsArgs* __restrict__ t, const int* __restrict__ pre, int nrep) {
   const int r = pm_batch_replica(pre, nrep, blockIdx.x);
@@ -2185,30 +2194,9 @@ void pm_launch_bin(hipStream_t s, const PmBox& box, int n, const double* pos, in
                        rebuild);
 }
 
-void pm_launch_scan_cells(hipStream_t s, int ncells, int nz, int* bin_count, int* cell_count, int* cell_start,
-                          int* cell_slot, int* counts, int* cluster_cell, int ncl_max, int m, const int* rebuild,
-                          int* aux) {
-  const int ch = scan_chunk_cells(nz);
-  const int nchunks = (ncells + ch - 1) / ch;
-  if (!pm_recording() && aux && nchunks > 2) {
-    hipLaunchKernelGGL(k_scan_chunks, dim3(nchunks), dim3(1024), 0, s, ncells, nz, bin_count, cell_count, m, aux,
-                       rebuild);
-    hipLaunchKernelGGL(k_scan_finish, dim3(nchunks), dim3(1024), 0, s, ncells, nz, cell_count, cell_start,
-                       cell_slot, counts, cluster_cell, ncl_max, m, aux, rebuild);
-    return;
-  }
-  if (pm_recording()) {
-    const ScanCellsArgs a{ncells, nz, bin_count, cell_count, cell_start, cell_slot, counts, cluster_cell, ncl_max, m,
-                          rebuild};
-    pm_record(PM_REC_SCAN_CELLS, 0, 1, 1024, 0, &a, sizeof(a));
-    return;
-  }
-  hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(1024), 0, s, ncells, nz, bin_count, cell_count, cell_start,
-                     cell_slot, counts, cluster_cell, ncl_max, m, rebuild);
-}
-
-void pm_launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank, const int* cell_start,
-                       int* cell_atoms, const int* rebuild) {
+#define PM_SCAN_SCATTER 16384
+static void launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank, const int* cell_start,
+                           int* cell_atoms, const int* rebuild) {
   if (pm_recording()) {
     const ScatterArgs a{n, cell_of, rank, cell_start, cell_atoms, rebuild};
     pm_record(PM_REC_SCATTER, 0, n > 0 ? (n + 255) / 256 : 0, 256, 0, &a, sizeof(a));
@@ -2217,6 +2205,35 @@ void pm_launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank
   if (n > 0)
     hipLaunchKernelGGL(k_scatter, dim3((n + 255) / 256), dim3(256), 0, s, n, cell_of, rank, cell_start,
                        cell_atoms, rebuild);
+}
+
+void pm_launch_scan_cells(hipStream_t s, int ncells, int nz, int* bin_count, int* cell_count, int* cell_start,
+                          int* cell_slot, int* counts, int* cluster_cell, int ncl_max, int m, const int* rebuild,
+                          int* aux, int n, const int* cell_of, const int* rank, int* cell_atoms) {
+  const int ch = scan_chunk_cells(nz);
+  const int nchunks = (ncells + ch - 1) / ch;
+  if (!pm_recording() && aux && nchunks > 2) {
+    hipLaunchKernelGGL(k_scan_chunks, dim3(nchunks), dim3(1024), 0, s, ncells, nz, bin_count, cell_count, m, aux,
+                       rebuild);
+    hipLaunchKernelGGL(k_scan_finish, dim3(nchunks), dim3(1024), 0, s, ncells, nz, cell_count, cell_start,
+                       cell_slot, counts, cluster_cell, ncl_max, m, aux, rebuild);
+    launch_scatter(s, n, cell_of, rank, cell_start, cell_atoms, rebuild);
+    return;
+  }
+  if (pm_recording()) {
+    const ScanCellsArgs a{ncells, nz, bin_count, cell_count, cell_start, cell_slot, counts, cluster_cell, ncl_max, m,
+                          rebuild};
+    pm_record(PM_REC_SCAN_CELLS, 0, 1, 1024, 0, &a, sizeof(a));
+    launch_scatter(s, n, cell_of, rank, cell_start, cell_atoms, rebuild);
+    return;
+  }
+  // Up to PM_SCAN_SCATTER atoms the scan's block also scatters (16 rounds at
+  // most, on build steps only): a launch less on every step, and a launch that
+  // returns at once still costs its boundary, about 4.5 us
+  const bool merged = n <= PM_SCAN_SCATTER;
+  hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(1024), 0, s, ncells, nz, bin_count, cell_count, cell_start,
+                     cell_slot, counts, cluster_cell, ncl_max, m, rebuild, merged ? n : 0, cell_of, rank, cell_atoms);
+  if (!merged) launch_scatter(s, n, cell_of, rank, cell_start, cell_atoms, rebuild);
 }
 
 void pm_launch_fill_slots(hipStream_t s, const PmBox& box, int ncells, const double* pos,

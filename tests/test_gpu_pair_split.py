@@ -55,3 +55,15 @@ def test_pair_forces_over_launch_shapes(gpu_ctx_factory, port, molecules, kind, 
         print("rms rel force", err, flush=True)
         assert err < TOL[precision]
         np.testing.assert_allclose(e[:2], er[:2], rtol=10 * TOL[precision], atol=1e-6 * np.abs(er[:2]).max())
+
+
+# the scan of up to 16,384 atoms also scatters them: a box on each side
+@pytest.mark.parametrize("molecules", [5461, 5462])
+def test_forces_over_layout_launches(gpu_ctx_factory, port, molecules):
+    print("case: layout launches", molecules, flush=True)
+    s = water.water_box(molecules, (molecules / 0.0334) ** (1.0 / 3.0), seed=molecules, jitter=0.3)
+    c = gpu_ctx_factory("double")
+    c.set_topology(s)
+    c.set_boundary(s.box, s.origin, 4.0)
+    f, _ = c.evaluate(gpu_forces_c1(c), s.pos)
+    assert rms_rel(f, reference(port, s, s.pos)[0]) < TOL["double"]
