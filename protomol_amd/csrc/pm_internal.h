@@ -427,7 +427,7 @@ struct PmConstraints {
   double* scratch;           // [3n] probe copy of positions (SHAKE) or velocities (RATTLE)
 };
 // SHAKE (rattle 0: x, v corrected, xl the reference positions, then set to
-// x) or RATTLE (rattle 1: v corrected); two launches
+// x) or RATTLE (rattle 1: v corrected); two launches, three with maxit > 16
 bool pm_launch_constraints(hipStream_t s, const PmConstraints& c, int rattle, double* x, double* v, double* xl);
 // The allocation-free entry point's work space: a file-scope device array of
 // PM_NOALLOC_SCRATCH_BYTES in pm_shake.hip.  pm_scratch_init (with `device`

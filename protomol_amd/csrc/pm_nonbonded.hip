@@ -1450,15 +1450,15 @@ __device__ inline double min_image(long long a, long long b) {
   return (double)(long long)((unsigned long long)a - (unsigned long long)b);
 }
 
-// Half-list pair kernel with one lane per list entry: a.split waves per
+// Half-list pair kernel with one lane per list entry: 1 << a.split_log waves per
 // i-cluster of M atoms, whose positions, charges and types sit in scalar
 // registers; a lane takes one entry (64 per iteration) and evaluates it
 // against the M i atoms in turn.  Wave `part` of a cluster takes the
-// iterations part, part + split, ...  The j force of an entry is then whole
+// iterations part, part + (1 << a.split_log), ...  The j force of an entry is then whole
 // in its lane and is added with one 64-bit integer atomic per component, with
 // no cross-lane sums; the i forces accumulate per lane in FP32 (one term per
 // iteration and i atom; FP64 in the FP64 kernel) and are summed over the
-// lanes in FP64 at the end, through LDS, in lane order.  Same pair arithmetic
+// lanes in FP64 at the end, by halving shuffles in a fixed order.  Same pair arithmetic
 // and the same half-list rule as pair_cluster; only the order in which FP32
 // partial sums are formed differs.
 // VALU issue bounds it in boxes that fill the chip, so it leaves out what a
