@@ -236,7 +236,8 @@ struct pm_context {
   double lat_key[4] = {0, 0, 0, 0};   // rc and box edges d_lat was built for
   double *d_bmod = nullptr, *d_expt = nullptr, *d_tw = nullptr;
   PmFftPlan plans[3];
-  double pme_alpha_tables = -1;
+  double pme_alpha_tables = -1;   // what d_bmod, d_expt and d_theta were made for
+  int pme_order_tables = 0;
 
   // MD
   std::vector<int> md_handles;
@@ -790,8 +791,9 @@ int ensure_pme(pm_context* c, ForceDesc& f) {
     c->pme_nx = nx; c->pme_ny = ny; c->pme_nz = nz; c->pme_prec = c->precision;
     c->pme_alpha_tables = -1;
   }
-  if (c->pme_alpha_tables != f.alpha) {
-    // Grid::initialize (base/Grid.h:557-648)
+  if (c->pme_alpha_tables != f.alpha || c->pme_order_tables != f.order) {
+    // Grid::initialize (base/Grid.h:557-648); bmod follows from the order
+    c->pme_alpha_tables = -1;
     const double lx = c->box.L[0], ly = c->box.L[1], lz = c->box.L[2];
     const double fac = kPi * kPi / (f.alpha * f.alpha);
     std::vector<double> bm(nx + ny + nz), ex(nx + ny + nzc);
@@ -818,6 +820,7 @@ int ensure_pme(pm_context* c, ForceDesc& f) {
     pm_launch_pme_theta(c->stream, t, c->precision);
     HIPCHECK(c, hipGetLastError());
     c->pme_alpha_tables = f.alpha;
+    c->pme_order_tables = f.order;
   }
   return PM_OK;
 }
