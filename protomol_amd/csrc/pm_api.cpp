@@ -36,6 +36,8 @@
 #define PM_SPLIT_WAVES 1024
 // values of x or v up to which pm_md_get_state copies through pinned memory
 #define PM_STAGE_STATE 65536
+// tables of PME terms that a context keeps before it refills unused ones
+#define PM_PME_TABLES 4
 // work space that a context keeps between pm_lanczos calls
 #define PM_LANCZOS_KEEP_BYTES (256u << 20)
 
@@ -84,7 +86,19 @@ struct ForceDesc {
   // cached PME state (NonbondedPMEwaldSystemForce::initialize, :499-648)
   bool cached = false;
   double alpha = 0;
+  int tables = -1;   // index of the term's PmeTables, set by ensure_pme
   std::string id;
+};
+
+// what one PME reciprocal term needs besides the grids
+struct PmeTables {
+  int nx = 0, ny = 0, nz = 0, order = 0, prec = -1;
+  double alpha = 0;
+  bool current = false;           // filled for the box in place
+  unsigned long long group = 0;   // the last force group that used them
+  PmFftPlan plans[3];
+  void* theta = nullptr;          // theta(m) on the line-major half grid (grid precision)
+  double *bmod = nullptr, *expt = nullptr, *tw = nullptr;
 };
 
 template <typename T>
@@ -225,19 +239,18 @@ struct pm_context {
   long long epart_alloc = 0;
   double* d_ered = nullptr;       // reduction stage-1 partials
 
-  // PME buffers (one grid size at a time)
-  int pme_nx = 0, pme_ny = 0, pme_nz = 0, pme_prec = -1;
+  // PME grids, sized for the largest term so far: the terms of a group run one
+  // after the other on one stream and leave the fixed-point grid cleared
+  size_t pme_points = 0, pme_bytes_r = 0, pme_bytes_c = 0;
   unsigned long long* d_grid_fix = nullptr;
   void* d_grid_r = nullptr;
   void* d_grid_c = nullptr;
-  void* d_theta = nullptr;   // theta(m) on the line-major half grid (grid precision)
+  std::vector<PmeTables> pme_tables;
+  unsigned long long pme_group = 0;
+  int pme_nx = 0, pme_ny = 0;   // grid of the term prepared last (pm_get_option)
   double* d_lat = nullptr;   // lattice vectors of the PME real term in small boxes
   int nlat = 0;
   double lat_key[4] = {0, 0, 0, 0};   // rc and box edges d_lat was built for
-  double *d_bmod = nullptr, *d_expt = nullptr, *d_tw = nullptr;
-  PmFftPlan plans[3];
-  double pme_alpha_tables = -1;   // what d_bmod, d_expt and d_theta were made for
-  int pme_order_tables = 0;
 
   // MD
   std::vector<int> md_handles;
@@ -749,37 +762,50 @@ bool fft_plan(int n, PmFftPlan& p) {
   return m == 1;
 }
 
-int ensure_pme(pm_context* c, ForceDesc& f) {
-  if (!f.cached) {
-    f.alpha = f.alpha_in <= 0.0 ? pme_alpha(f.rc, f.accuracy) : f.alpha_in;
-    f.cached = true;
+void free_tables(PmeTables& t) {
+  if (t.theta) hipFree(t.theta);
+  dfree(t.bmod); dfree(t.expt); dfree(t.tw);
+  t = PmeTables();
+}
+
+// the grids for terms of up to `points` real and `cpoints` complex points of
+// `er` bytes a value
+int ensure_pme_grids(pm_context* c, size_t points, size_t cpoints, size_t er) {
+  int r;
+  if (points > c->pme_points) {
+    c->pme_points = 0;
+    if ((r = dalloc(c, &c->d_grid_fix, points))) return r;
+    HIPCHECK(c, hipMemset(c->d_grid_fix, 0, points * sizeof(unsigned long long)));
+    c->pme_points = points;
   }
-  const int nx = f.nx, ny = f.ny, nz = f.nz, nzc = nz / 2 + 1;
-  const bool same_grid = c->pme_nx == nx && c->pme_ny == ny && c->pme_nz == nz && c->pme_prec == c->precision;
-  if (!f.recip) return PM_OK;
-  if (!same_grid) {
-    if (nx > 4096 || ny > 4096 || nz > 4096 || nx < 8 || ny < 8 || nz < 8)
-      return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: 8 to 4096 points per axis", nx, ny, nz);
-    if (!fft_plan(nx, c->plans[0]) || !fft_plan(ny, c->plans[1]) || !fft_plan(nz, c->plans[2]))
+  auto grow = [&](void** p, size_t* have, size_t bytes) -> int {
+    if (bytes <= *have) return PM_OK;
+    c->gen++;
+    if (*p) hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+    HIPCHECK(c, hipMalloc(p, bytes));
+    *have = bytes;
+    return PM_OK;
+  };
+  if ((r = grow(&c->d_grid_r, &c->pme_bytes_r, points * er))) return r;
+  return grow(&c->d_grid_c, &c->pme_bytes_c, cpoints * er * 2);
+}
+
+// fill tables whose grid, order, alpha and precision are set
+int fill_tables(pm_context* c, PmeTables& t) {
+  const int nx = t.nx, ny = t.ny, nz = t.nz, nzc = nz / 2 + 1;
+  const size_t er = t.prec == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+  int r;
+  if (!t.tw) {
+    if (!fft_plan(nx, t.plans[0]) || !fft_plan(ny, t.plans[1]) || !fft_plan(nz, t.plans[2]))
       return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: the GPU FFT handles lengths with factors 2, 3, 5 and 7 only", nx, ny, nz);
-    size_t ng = (size_t)nx * ny * nz, ngc = (size_t)nx * ny * nzc;
-    size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
-    int r;
-    if ((r = dalloc(c, &c->d_grid_fix, ng))) return r;
-    HIPCHECK(c, hipMemset(c->d_grid_fix, 0, ng * sizeof(unsigned long long)));
-    if (c->d_grid_r) hipFree(c->d_grid_r);
-    if (c->d_grid_c) hipFree(c->d_grid_c);
-    if (c->d_theta) hipFree(c->d_theta);
-    c->d_grid_r = c->d_grid_c = c->d_theta = nullptr;
-    HIPCHECK(c, hipMalloc(&c->d_grid_r, ng * er));
-    HIPCHECK(c, hipMalloc(&c->d_grid_c, ngc * er * 2));
-    HIPCHECK(c, hipMalloc(&c->d_theta, ngc * er));
     // twiddles exp(-2 pi i m / n) for the three lengths
     std::vector<double> tw;
     int off = 0;
     for (int a = 0; a < 3; a++) {
-      int len = c->plans[a].n;
-      c->plans[a].tw = off;
+      int len = t.plans[a].n;
+      t.plans[a].tw = off;
       for (int m = 0; m < len; m++) {
         double ang = -2.0 * kPi * (double)m / len;
         tw.push_back(std::cos(ang));
@@ -787,42 +813,94 @@ int ensure_pme(pm_context* c, ForceDesc& f) {
       }
       off += len;
     }
-    if ((r = upload(c, &c->d_tw, tw))) return r;
-    c->pme_nx = nx; c->pme_ny = ny; c->pme_nz = nz; c->pme_prec = c->precision;
-    c->pme_alpha_tables = -1;
+    if (!t.theta) HIPCHECK(c, hipMalloc(&t.theta, (size_t)nx * ny * nzc * er));
+    if ((r = upload(c, &t.tw, tw))) return r;
   }
-  if (c->pme_alpha_tables != f.alpha || c->pme_order_tables != f.order) {
-    // Grid::initialize (base/Grid.h:557-648); bmod follows from the order
-    c->pme_alpha_tables = -1;
-    const double lx = c->box.L[0], ly = c->box.L[1], lz = c->box.L[2];
-    const double fac = kPi * kPi / (f.alpha * f.alpha);
-    std::vector<double> bm(nx + ny + nz), ex(nx + ny + nzc);
-    std::vector<double> th(f.order);
-    bspline_host(f.order, 0.0, th.data());
-    dftmod(f.order, nx, th.data(), bm.data());
-    dftmod(f.order, ny, th.data(), bm.data() + nx);
-    dftmod(f.order, nz, th.data(), bm.data() + nx + ny);
-    const double wr = 1.0 / lx, lr = 1.0 / ly, hr = 1.0 / lz;
-    for (int i = 0; i < nx; i++) { int i0 = i <= nx / 2 ? i : i - nx; double t = i0 * wr; ex[i] = std::exp(-fac * (t * t)); }
-    for (int j = 0; j < ny; j++) { int j0 = j <= ny / 2 ? j : j - ny; double t = j0 * lr; ex[nx + j] = std::exp(-fac * (t * t)); }
-    for (int k = 0; k < nzc; k++) { double t = k * hr; ex[nx + ny + k] = std::exp(-fac * (t * t)); }
-    int r;
-    if ((r = upload(c, &c->d_bmod, bm))) return r;
-    if ((r = upload(c, &c->d_expt, ex))) return r;
-    // theta(m) for the x passes that write no energy records
-    PmPmeLaunch t{};
-    t.nx = nx; t.ny = ny; t.nz = nz; t.nzc = nzc;
-    for (int k = 0; k < 3; k++) t.Lr[k] = 1.0 / c->box.L[k];
-    t.bmod = c->d_bmod;
-    t.expf_tab = c->d_expt;
-    t.inv_pi_v = 1.0 / (kPi * (c->box.L[0] * c->box.L[1] * c->box.L[2]));
-    t.theta = c->d_theta;
-    pm_launch_pme_theta(c->stream, t, c->precision);
-    HIPCHECK(c, hipGetLastError());
-    c->pme_alpha_tables = f.alpha;
-    c->pme_order_tables = f.order;
-  }
+  // Grid::initialize (base/Grid.h:557-648); bmod follows from the order
+  const double lx = c->box.L[0], ly = c->box.L[1], lz = c->box.L[2];
+  const double fac = kPi * kPi / (t.alpha * t.alpha);
+  std::vector<double> bm(nx + ny + nz), ex(nx + ny + nzc);
+  std::vector<double> th(t.order);
+  bspline_host(t.order, 0.0, th.data());
+  dftmod(t.order, nx, th.data(), bm.data());
+  dftmod(t.order, ny, th.data(), bm.data() + nx);
+  dftmod(t.order, nz, th.data(), bm.data() + nx + ny);
+  const double wr = 1.0 / lx, lr = 1.0 / ly, hr = 1.0 / lz;
+  for (int i = 0; i < nx; i++) { int i0 = i <= nx / 2 ? i : i - nx; double u = i0 * wr; ex[i] = std::exp(-fac * (u * u)); }
+  for (int j = 0; j < ny; j++) { int j0 = j <= ny / 2 ? j : j - ny; double u = j0 * lr; ex[nx + j] = std::exp(-fac * (u * u)); }
+  for (int k = 0; k < nzc; k++) { double u = k * hr; ex[nx + ny + k] = std::exp(-fac * (u * u)); }
+  if ((r = upload(c, &t.bmod, bm))) return r;
+  if ((r = upload(c, &t.expt, ex))) return r;
+  // theta(m) for the x passes that write no energy records
+  PmPmeLaunch a{};
+  a.nx = nx; a.ny = ny; a.nz = nz; a.nzc = nzc;
+  for (int k = 0; k < 3; k++) a.Lr[k] = 1.0 / c->box.L[k];
+  a.bmod = t.bmod;
+  a.expf_tab = t.expt;
+  a.inv_pi_v = 1.0 / (kPi * (c->box.L[0] * c->box.L[1] * c->box.L[2]));
+  a.theta = t.theta;
+  pm_launch_pme_theta(c->stream, a, t.prec);
+  HIPCHECK(c, hipGetLastError());
+  t.current = true;
   return PM_OK;
+}
+
+// Alphas, grids and tables of a group's PME terms.  Every term has tables of
+// its own; tables that no term of the group uses are refilled once there are
+// PM_PME_TABLES of them (one with the same grid first: it keeps its buffers).
+int ensure_pme(pm_context* c, const std::vector<int>& handles) {
+  c->pme_group++;
+  size_t points = 0, cpoints = 0;
+  for (int h : handles) {
+    ForceDesc& f = c->forces[h];
+    if (!f.pme) continue;
+    if (!f.cached) {
+      f.alpha = f.alpha_in <= 0.0 ? pme_alpha(f.rc, f.accuracy) : f.alpha_in;
+      f.cached = true;
+    }
+    if (!f.recip) continue;
+    const int nx = f.nx, ny = f.ny, nz = f.nz;
+    if (nx > 4096 || ny > 4096 || nz > 4096 || nx < 8 || ny < 8 || nz < 8)
+      return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: 8 to 4096 points per axis", nx, ny, nz);
+    points = std::max(points, (size_t)nx * ny * nz);
+    cpoints = std::max(cpoints, (size_t)nx * ny * (nz / 2 + 1));
+    c->pme_nx = nx; c->pme_ny = ny;
+  }
+  int r;
+  for (int h : handles) {
+    ForceDesc& f = c->forces[h];
+    if (!f.pme || !f.recip) continue;
+    int at = -1;
+    auto grid = [&](const PmeTables& t) { return t.nx == f.nx && t.ny == f.ny && t.nz == f.nz && t.prec == c->precision; };
+    const int count = (int)c->pme_tables.size();
+    for (int k = 0; k < count && at < 0; k++)
+      if (grid(c->pme_tables[k]) && c->pme_tables[k].order == f.order && c->pme_tables[k].alpha == f.alpha) at = k;
+    if (at < 0 && count >= PM_PME_TABLES) {
+      // refill: of the group's unused ones the same grid, else the longest unused
+      for (int k = 0; k < count; k++) {
+        const PmeTables& t = c->pme_tables[k];
+        if (t.group == c->pme_group) continue;
+        if (at < 0 || (grid(t) && !grid(c->pme_tables[at])) ||
+            (grid(t) == grid(c->pme_tables[at]) && t.group < c->pme_tables[at].group))
+          at = k;
+      }
+    }
+    if (at < 0) {
+      at = count;
+      c->pme_tables.push_back(PmeTables());
+    }
+    PmeTables& t = c->pme_tables[at];
+    if (!grid(t)) free_tables(t);
+    if (!grid(t) || t.order != f.order || t.alpha != f.alpha) t.current = false;
+    t.nx = f.nx; t.ny = f.ny; t.nz = f.nz; t.prec = c->precision;
+    t.order = f.order;
+    t.alpha = f.alpha;
+    t.group = c->pme_group;
+    f.tables = at;
+    if (!t.current && (r = fill_tables(c, t))) return r;
+  }
+  const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+  return points ? ensure_pme_grids(c, points, cpoints, er) : PM_OK;
 }
 
 // ------------------------------------------------------------ force parsing
@@ -1193,12 +1271,10 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   c->disp_prechecked = false;
   c->md_prebinned = false;
   int r;
+  if ((r = ensure_pme(c, handles))) return r;
   for (int h : handles) {
     ForceDesc& f = c->forces[h];
-    if (f.pme) {
-      if ((r = ensure_pme(c, f))) return r;
-      if (f.real && pme_lattice(c, f) && (r = ensure_lattice(c, f.rc))) return r;
-    }
+    if (f.pme && f.real && pme_lattice(c, f) && (r = ensure_lattice(c, f.rc))) return r;
   }
   std::vector<PairPass> passes = plan_passes(c, handles);
   bool any_pme = false;
@@ -1363,12 +1439,25 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       pl.first.icount = c->d_icount;
     }
   }
-  std::vector<std::pair<PmPmeLaunch, int>> pme_launch;   // (launch, handle)
+  struct PmeLaunch { PmPmeLaunch a; int handle; const PmFftPlan* plans; };
+  std::vector<PmeLaunch> pme_launch;
+  if (adj) {
+    // two grids of the adjoint's own, so that the charges' potential outlives
+    // the direction's convolution, for the largest term
+    const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+    size_t bytes = 0;
+    for (auto& hr : pme_rec) {
+      const ForceDesc& f = c->forces[hr.first];
+      if (f.recip) bytes = std::max(bytes, 2 * er * (size_t)f.nx * f.ny * (f.nz / 2 + 1) * 2);
+    }
+    if ((r = ensure_adj_grids(c, bytes))) return r;
+  }
   double const_coul = 0.0, const_vir = 0.0;
   for (auto& hr : pme_rec) {
     ForceDesc& f = c->forces[hr.first];
     long long off = hr.second;
     if (f.recip) {
+      const PmeTables& t = c->pme_tables[f.tables];
       PmPmeLaunch a{};
       a.n = n;
       a.nx = f.nx; a.ny = f.ny; a.nz = f.nz; a.nzc = f.nz / 2 + 1;
@@ -1386,11 +1475,11 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       a.grid_fix = c->d_grid_fix;
       a.grid_r = c->d_grid_r;
       a.grid_c = c->d_grid_c;
-      a.bmod = c->d_bmod;
-      a.expf_tab = c->d_expt;
+      a.bmod = t.bmod;
+      a.expf_tab = t.expt;
       a.inv_pi_v = 1.0 / (kPi * (c->box.L[0] * c->box.L[1] * c->box.L[2]));
       a.fac = kPi * kPi / (f.alpha * f.alpha);
-      a.tw = c->d_tw;
+      a.tw = t.tw;
       a.err = c->d_overflow;
       a.prio = pme_priority(c);
       a.force_fix = c->d_force_side;
@@ -1398,7 +1487,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       a.epart = c->d_epart + off * PM_NE;
       a.want_virial = vir ? 1 : 0;
       a.want_energy = want_energy ? 1 : 0;
-      a.theta = c->d_theta;
+      a.theta = t.theta;
       // spread bricks: 2x2x2 cells per brick (fewer where the tile would not fit 48 KB of LDS)
       a.cell_slot = c->d_cell_slot;
       a.cell_count = c->d_cell_count;
@@ -1431,10 +1520,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       const double drift_A = (reuse ? 0.5 * skin * (1.0 + 1e-3) : 0.0) + 1e-3;
       for (int d = 0; d < 3; d++) a.drift_u[d] = drift_A * ng[d] / c->box.L[d] + 0.01;
       if (adj) {
-        // two grids of its own, so that the charges' potential outlives the
-        // direction's convolution; line-major, with theta from the table
-        const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
-        if ((r = ensure_adj_grids(c, 2 * er * (size_t)a.nx * a.ny * a.nzc * 2))) return r;
+        // line-major, with theta from the table
         a.grid_r = c->d_adj_grid_r;
         a.grid_c = c->d_adj_grid_c;
         a.plane = 0;
@@ -1443,7 +1529,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
       a.spread_zfwd = c->pme_spread_option != 0 ? pm_pme_spread_zfwd_fits(a, c->precision) : 0;
       if (!a.spread_zfwd && (size_t)a.tile[0] * a.tile[1] * a.tile[2] * 8 > 64 * 1024)
         return fail(c, PM_ERR_UNSUPPORTED, "PME grid too fine for the cell size: spread tile exceeds 64 KB of LDS (use a smaller cellsize)");
-      pme_launch.push_back(std::make_pair(a, hr.first));
+      pme_launch.push_back(PmeLaunch{a, hr.first, t.plans});
     }
     if (f.corr && !adj) {
       // point self energy and charged-system term (:604-628)
@@ -1482,7 +1568,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
                            nullptr, 0);
     if (pme_launch.empty()) pm_launch_zero_d(s2, out, adj->mode == 1 ? 3LL * n : n);
     for (auto& pl : pme_launch)
-      pm_launch_pme_adjoint(s2, pl.first, c->plans, c->d_slot_pos64, c->precision, adj->mode == 1 ? 1 : 0,
+      pm_launch_pme_adjoint(s2, pl.a, pl.plans, c->d_slot_pos64, c->precision, adj->mode == 1 ? 1 : 0,
                             adj->kept && pme_launch.size() == 1, adj->slot_v, out);
     for (auto& hr : pme_rec) {
       ForceDesc& f = c->forces[hr.first];
@@ -1542,9 +1628,9 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   // with one PME reciprocal term, the gather kernel's thread for an atom
   // also adds that atom's correction force (a launch fewer)
   PmAtomTail tail{};
-  const bool fuse = pme_launch.size() == 1 && c->forces[pme_launch[0].second].corr;
+  const bool fuse = pme_launch.size() == 1 && c->forces[pme_launch[0].handle].corr;
   if (fuse) {
-    const ForceDesc& f = c->forces[pme_launch[0].second];
+    const ForceDesc& f = c->forces[pme_launch[0].handle];
     tail.box = c->box;
     tail.pos = c->d_pos; tail.q = c->d_q;
     tail.row = c->d_cx_row; tail.partner = c->d_cx_partner; tail.cls = c->d_cx_cls;
@@ -1552,7 +1638,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   }
   for (auto& pl : pme_launch) {
     TimedScope ts(c, PM_T_PME, s2);
-    pm_launch_pme_plans(s2, pl.first, c->plans, c->d_slot_pos64, c->precision, fuse ? &tail : nullptr);
+    pm_launch_pme_plans(s2, pl.a, pl.plans, c->d_slot_pos64, c->precision, fuse ? &tail : nullptr);
   }
   // (a correction without a reciprocal term is the array's first writer)
   bool side_forces = !pme_launch.empty();
@@ -1561,7 +1647,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     if (!f.corr) continue;
     if (!side_forces) pm_launch_zero_ll(s2, c->d_force_side, 3LL * n);
     side_forces = true;
-    const bool in_tail = fuse && hr.first == pme_launch[0].second;
+    const bool in_tail = fuse && hr.first == pme_launch[0].handle;
     long long off = hr.second + (f.recip ? pm_pme_xpass_blocks(f.nx, f.ny, f.nz, c->precision, pme_plane(c, f)) : 0);
     int ntab = (int)c->tab_a.size();
     int nblk = (ntab + 255) / 256;
@@ -1835,11 +1921,12 @@ void free_all(pm_context* c) {
   dfree(c->d_grid_fix);
   if (c->d_grid_r) hipFree(c->d_grid_r);
   if (c->d_grid_c) hipFree(c->d_grid_c);
-  if (c->d_theta) hipFree(c->d_theta);
-  c->d_grid_r = c->d_grid_c = c->d_theta = nullptr;
+  c->d_grid_r = c->d_grid_c = nullptr;
+  c->pme_points = c->pme_bytes_r = c->pme_bytes_c = 0;
+  for (PmeTables& t : c->pme_tables) free_tables(t);
+  c->pme_tables.clear();
   dfree(c->d_lat);
   c->nlat = 0;
-  dfree(c->d_bmod); dfree(c->d_expt); dfree(c->d_tw);
   dfree(c->d_b_a); dfree(c->d_b_b); dfree(c->d_b_k); dfree(c->d_b_r0);
   dfree(c->d_a_a); dfree(c->d_a_b); dfree(c->d_a_c);
   dfree(c->d_a_k); dfree(c->d_a_t0); dfree(c->d_a_kub); dfree(c->d_a_rub);
@@ -1859,8 +1946,7 @@ void free_all(pm_context* c) {
   c->cells_alloc = 0;
   c->jlist_alloc = 0;
   c->epart_alloc = 0;
-  c->pme_nx = c->pme_ny = c->pme_nz = 0;
-  c->pme_prec = -1;
+  c->pme_nx = c->pme_ny = 0;
 }
 
 int set_device(pm_context* c) {
@@ -2275,7 +2361,7 @@ int pm_set_boundary(pm_context* c, const double* e1, const double* e2, const dou
   c->cellsize = cellsize;
   free_stencils(c);
   c->cells_alloc = 0;
-  c->pme_alpha_tables = -1;
+  for (PmeTables& t : c->pme_tables) t.current = false;
   c->have_box = true;
   c->list_stale = true;
   for (auto& f : c->forces) f.cached = false;
@@ -2299,7 +2385,7 @@ int pm_force_uncache(pm_context* c, int handle) {
   if (!c) return PM_ERR_ARGUMENT;
   if (handle < 0 || handle >= (int)c->forces.size()) return fail(c, PM_ERR_ARGUMENT, "unknown force handle %d", handle);
   c->forces[handle].cached = false;
-  c->pme_alpha_tables = -1;
+  for (PmeTables& t : c->pme_tables) t.current = false;
   return PM_OK;
 }
 

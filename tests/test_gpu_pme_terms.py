@@ -42,3 +42,49 @@ def test_terms_in_turn(gpu_ctx_factory, precision, other):
     for k in (0, 1, 0, 1):
         for got, want in zip(results(c, hs[k]), own[k]):
             np.testing.assert_array_equal(got, want)
+
+
+# two reciprocal terms in one group, the smaller grid first and last, and the
+# same term twice: each part is computed on its own in either case, so the sum
+# of the parts agrees to FP64 round-off of the sums (and, forces, to the 2^-40
+# steps that the parts are rounded to)
+@pytest.mark.parametrize("precision", ["mixed", "double"])
+@pytest.mark.parametrize("spread", [1, 0])
+@pytest.mark.parametrize("values", [[term(), term(grid=32, order=6)], [term(grid=32, order=6), term()],
+                                    [term(), term(accuracy=1e-4)], [term(), term()],
+                                    [term(), term(grid=20), term(grid=30), term(order=6), term(grid=32, order=8)]])
+def test_terms_of_a_group_add_up(gpu_ctx_factory, precision, spread, values):
+    print("case: pme terms of a group", precision, spread, values, flush=True)
+    s = water.named("water648", seed=6, jitter=0.3)
+    v = np.random.default_rng(2).standard_normal((s.n, 3))
+    c = context(gpu_ctx_factory, s, precision)
+    c.set_option("pme_spread", spread)
+    hs = [c.force(PME, t) for t in values]
+    for _ in range(2):
+        f, e = c.evaluate(hs, s.pos, virial=True)
+        hv = c.hessian_vec(hs, s.pos, v)
+        dq = c.param_gradients(hs, s.pos, lj=False)[0]
+        vals, _, _, alpha, beta = c.lanczos(hs, s.pos, v, steps=3)
+        parts = [c.evaluate([h], s.pos, virial=True) for h in hs]
+        want = sum(p[0] for p in parts)
+        assert np.abs(f - want).max() <= 16 * 2.0 ** -40 + 1e-14 * np.abs(want).max()
+        np.testing.assert_allclose(e, sum(p[1] for p in parts), rtol=1e-12, atol=1e-9)
+        want = sum(c.hessian_vec([h], s.pos, v) for h in hs)
+        assert np.abs(hv - want).max() <= 1e-12 * np.abs(want).max()
+        want = sum(c.param_gradients([h], s.pos, lj=False)[0] for h in hs)
+        assert np.abs(dq - want).max() <= 1e-12 * np.abs(want).max()
+        # the Lanczos recurrence over single products
+        V, ra, rb = [v.reshape(-1) / np.linalg.norm(v)], [], []
+        for _ in range(3):
+            w = c.hessian_vec(hs, s.pos, V[-1].reshape(-1, 3)).reshape(-1)
+            ra.append(V[-1] @ w)
+            for _ in range(2):
+                for u in V:
+                    w = w - (u @ w) * u
+            rb.append(np.linalg.norm(w))
+            V.append(w / rb[-1])
+        # (the directions agree to FP64 round-off; their FP32 copies in mixed
+        # precision to 6e-8, which three steps amplify by a few tens)
+        tol = (1e-5 if precision == "mixed" else 1e-11) * max(np.abs(ra).max(), np.abs(rb).max())
+        np.testing.assert_allclose(alpha, ra, rtol=0, atol=tol)
+        np.testing.assert_allclose(beta, rb, rtol=0, atol=tol)
