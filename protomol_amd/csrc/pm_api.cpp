@@ -289,6 +289,7 @@ struct pm_context {
   long long ilist_alloc = 0;
   bool inner_last = false;           // the last evaluation's pair pass kept inner lists
   bool list_stale = true;            // x_build must be invalidated before the next reuse
+  double list_cut = -1.0, list_built_skin = -1.0;   // pair cutoff and skin the kept lists are for
   unsigned long long gen = 1;        // bumped by every allocation and every setter
   hipGraphExec_t md_exec = nullptr;
   int md_exec_steps = 0, md_exec_kind = -1;
@@ -653,6 +654,7 @@ int ensure_lists(pm_context* c, int lcap) {
   long long need = (long long)c->ncl_max * lcap;
   if (need <= c->jlist_alloc && c->d_jlist) { c->lcap = lcap; return PM_OK; }
   int r;
+  c->list_stale = true;   // the new buffers hold no lists
   if ((r = dalloc(c, &c->d_jlist, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jmask, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jcount, c->ncl_max))) return r;
@@ -667,6 +669,7 @@ int ensure_inner_lists(pm_context* c) {
   const long long need = (long long)c->ncl_max * c->lcap;
   if (need <= c->ilist_alloc && c->d_ilist) return PM_OK;
   int r;
+  c->list_stale = true;
   if ((r = dalloc(c, &c->d_ilist, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_imask, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_icount, c->ncl_max))) return r;
@@ -1213,6 +1216,12 @@ bool list_reuse(const pm_context* c, const std::vector<PairPass>& passes) {
   return passes[0].algo_cutoff >= pc;
 }
 
+// Whether the kept lists were built for this pass: another pair cutoff (or
+// skin) lists other pairs, near ones by another distance, at another stride
+bool lists_match(const pm_context* c, const PairPass& p) {
+  return c->list_cut == std::sqrt(pair_params(p.terms, c->csf).cut2) && c->list_built_skin == list_skin(c);
+}
+
 // Inner lists: with list reuse, an inner skin below the list skin
 bool inner_lists(const pm_context* c) {
   const double ps = prune_skin(c);
@@ -1238,7 +1247,8 @@ bool md_step_work(pm_context* c, PmStepWork* w) {
   w->bin_count = c->d_bin_count;
   c->md_prebinned = true;
   c->prebin_gen = c->layout_gen;
-  if (!c->list_stale && c->d_xbuild && c->d_rebuild && list_reuse(c, plan_passes(c, c->md_handles))) {
+  const std::vector<PairPass> passes = plan_passes(c, c->md_handles);
+  if (!c->list_stale && c->d_xbuild && c->d_rebuild && list_reuse(c, passes) && lists_match(c, passes[0])) {
     const double half = 0.5 * list_skin(c);
     for (int k = 0; k < 3; k++) {
       w->to_fix[k] = c->box.to_fix[k];
@@ -1295,8 +1305,19 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   const int* rb = reuse ? c->d_rebuild : nullptr;
   const bool inner = reuse && inner_lists(c);
   c->inner_last = inner;
+  if (reuse) {
+    // the buffers before the displacement test, which decides on a build
+    const double pcut = std::sqrt(pair_params(passes[0].terms, c->csf).cut2);
+    if ((r = ensure_lists(c, list_capacity(c, pcut + skin)))) return r;
+    if (inner && (r = ensure_inner_lists(c))) return r;
+    if (!lists_match(c, passes[0])) c->list_stale = true;
+    c->list_cut = pcut;
+    c->list_built_skin = skin;
+  }
   if (!adj || !adj->kept) {
   TimedScope ts(c, PM_T_BIN);
+  // (a test queued ahead of this evaluation saw the build positions as they were)
+  const bool tested = prechecked && !c->list_stale;
   if (reuse && c->list_stale) {
     pm_launch_invalidate_build(s, n, c->d_xbuild);
     pm_launch_invalidate_build(s, n, c->d_xprune);
@@ -1306,7 +1327,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   // kernel sequence the same with and without reuse)
   const float half = (float)(0.5 * skin);
   const float hin = (float)(0.5 * prune_skin(c));
-  pm_launch_check_disp(s, c->box, reuse && !prechecked ? n : 0, c->d_pos, c->d_xbuild, half * half, c->d_rebuild,
+  pm_launch_check_disp(s, c->box, reuse && !tested ? n : 0, c->d_pos, c->d_xbuild, half * half, c->d_rebuild,
                        inner ? c->d_xprune : nullptr, hin * hin);
   // (the MD position update may have binned the atoms and cleared the forces
   // already, for the layout in place; the last fold cleared the slot forces)

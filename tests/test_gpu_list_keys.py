@@ -1,0 +1,69 @@
+"""Kept pair lists belong to the pair cutoff that they were built for: force
+evaluations of different cutoffs in turn on one context, at positions that
+would keep any of the lists, against contexts of their own, and MD runs with
+such evaluations between them.  FP64: round-off of sums in another order
+(1e-11; 1e-8 A after 20 steps)."""
+import numpy as np
+import pytest
+
+from protomol_amd import water
+from tests.cases import rms_rel
+
+pytestmark = pytest.mark.gpu
+LJ = "LennardJones CoulombEwaldReal -algorithm NonbondedCutoff -switchingFunction C2 -switchingFunction Cutoff"
+
+
+def values(rc):
+    return [rc - 1.0, rc, 0.4, rc, rc]
+
+
+def context(make, s, precision, **options):
+    c = make(precision)
+    c.set_topology(s)
+    c.set_boundary(s.box, s.origin, 4.0)
+    for k, v in options.items():
+        c.set_option(k, v)
+    return c
+
+
+@pytest.mark.parametrize("precision,tol", [("mixed", 5e-6), ("double", 1e-11)])
+@pytest.mark.parametrize("options", [{}, {"pair_lanes": 0}, {"prune_skin": 300}, {"cluster_size": 4}])
+@pytest.mark.parametrize("cutoffs", [(8.0, 5.0), (5.0, 8.0), (8.0, 9.0, 6.0)])
+def test_cutoffs_in_turn(gpu_ctx_factory, precision, tol, options, cutoffs):
+    print("case: list cutoffs in turn", precision, options, cutoffs, flush=True)
+    s = water.named("water648", seed=5, jitter=0.3)
+    own = []
+    for rc in cutoffs:
+        c = context(gpu_ctx_factory, s, precision, **options)
+        own.append(c.evaluate([c.force(LJ, values(rc))], s.pos))
+    c = context(gpu_ctx_factory, s, precision, **options)
+    hs = [c.force(LJ, values(rc)) for rc in cutoffs]
+    for k in list(range(len(cutoffs))) * 2:
+        f, e = c.evaluate([hs[k]], s.pos + 0.01)     # (all atoms alike: the same forces)
+        assert rms_rel(f, own[k][0]) < tol
+        np.testing.assert_allclose(e[:2], own[k][1][:2], rtol=10 * tol)
+
+
+@pytest.mark.parametrize("integrator", ["leapfrog", "langevin"])
+@pytest.mark.parametrize("other", [5.0, 9.0])
+def test_md_after_another_cutoff(gpu_ctx_factory, integrator, other):
+    print("case: md after another cutoff", integrator, other, flush=True)
+    s = water.named("water648", seed=6, jitter=0.2)
+    got = []
+    for between in (True, False):
+        c = context(gpu_ctx_factory, s, "double")
+        hs = [c.force(LJ, values(8.0)), c.force("Bond", []), c.force("Angle", [])]
+        o = c.force(LJ, values(other))
+        kw = dict(temperature=300.0, gamma=5.0, seed=3) if integrator == "langevin" else {}
+        c.md_setup(hs, integrator, dt=1.0, **kw)
+        c.md_set_state(s.pos, s.vel)
+        for _ in range(3):
+            c.md_run(20)
+            x, v, _ = c.md_get_state()
+            if between:
+                c.evaluate([o], x)
+            else:
+                c.md_set_state(x, v)
+        got.append(c.md_get_state()[:2])
+    np.testing.assert_allclose(got[0][0], got[1][0], rtol=0, atol=1e-7)
+    np.testing.assert_allclose(got[0][1], got[1][1], rtol=0, atol=1e-6 * np.abs(got[1][1]).max())
