@@ -1305,11 +1305,13 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   const int* rb = reuse ? c->d_rebuild : nullptr;
   const bool inner = reuse && inner_lists(c);
   c->inner_last = inner;
+  // the list buffers, for the widest pass, before the displacement test, which
+  // decides on a build
+  double pcut = 0.0;
+  for (const PairPass& p : passes) pcut = std::max(pcut, std::sqrt(pair_params(p.terms, c->csf).cut2));
+  if (!passes.empty() && (r = ensure_lists(c, list_capacity(c, pcut + (reuse ? skin : 0.0))))) return r;
+  if (inner && (r = ensure_inner_lists(c))) return r;
   if (reuse) {
-    // the buffers before the displacement test, which decides on a build
-    const double pcut = std::sqrt(pair_params(passes[0].terms, c->csf).cut2);
-    if ((r = ensure_lists(c, list_capacity(c, pcut + skin)))) return r;
-    if (inner && (r = ensure_inner_lists(c))) return r;
     if (!lists_match(c, passes[0])) c->list_stale = true;
     c->list_cut = pcut;
     c->list_built_skin = skin;
@@ -1397,9 +1399,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     if ((r = get_stencil(c, ps.algo_cutoff + lskin, false, &st, &nst))) return r;
     if (nst > 650)
       return fail(c, PM_ERR_UNSUPPORTED, "cell stencil of %d columns (cellsize %g, cutoff %g): use a cellsize of at least cutoff/4", nst, c->cellsize, ps.algo_cutoff);
-    double pcut = std::sqrt(pp.cut2);
-    if ((r = ensure_lists(c, list_capacity(c, pcut + lskin)))) return r;
-    if (inner && (r = ensure_inner_lists(c))) return r;
+    const double pcut = std::sqrt(pp.cut2);
     pair_launch.push_back(std::make_pair(PmNbLaunch{}, pp));
     PmNbLaunch& a = pair_launch.back().first;
     a.slot_pos = c->d_slot_pos;
@@ -1413,6 +1413,10 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.cell_count = c->d_cell_count;
     a.stencil = st;
     a.nstencil = nst;
+    a.jlist = c->d_jlist;
+    a.jmask = c->d_jmask;
+    a.jcount = c->d_jcount;
+    a.jnear = c->d_jnear;
     a.lcap = c->lcap;
     a.overflow = c->d_overflow;
     a.bbox_filter = !list_exact(c) && lmin_half > pcut + lskin + cdiag + 1e-3 ? 1 : 0;
@@ -1441,23 +1445,15 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.epart = c->d_epart + (long long)pi * pair_rec * PM_NE;
     a.want_virial = vir ? 1 : 0;
     a.want_energy = want_energy ? 1 : 0;
-  }
-  // the list buffers may have grown while the passes were set up
-  for (auto& pl : pair_launch) {
-    pl.first.jlist = c->d_jlist;
-    pl.first.jmask = c->d_jmask;
-    pl.first.jcount = c->d_jcount;
-    pl.first.jnear = c->d_jnear;
-    pl.first.lcap = c->lcap;
     if (inner) {
       // the pair cutoff + the inner skin, padded as the list cutoff is
-      const double cp = std::sqrt(pl.second.cut2) + prune_skin(c);
+      const double cp = pcut + prune_skin(c);
       const float cf = (float)(cp * (1.0 + 1e-5) + 1e-4);
-      pl.first.inner = 1;
-      pl.first.cut2_prune = cf * cf;
-      pl.first.ilist = c->d_ilist;
-      pl.first.imask = c->d_imask;
-      pl.first.icount = c->d_icount;
+      a.inner = 1;
+      a.cut2_prune = cf * cf;
+      a.ilist = c->d_ilist;
+      a.imask = c->d_imask;
+      a.icount = c->d_icount;
     }
   }
   struct PmeLaunch { PmPmeLaunch a; int handle; const PmFftPlan* plans; };

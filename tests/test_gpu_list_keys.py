@@ -67,3 +67,23 @@ def test_md_after_another_cutoff(gpu_ctx_factory, integrator, other):
         got.append(c.md_get_state()[:2])
     np.testing.assert_allclose(got[0][0], got[1][0], rtol=0, atol=1e-7)
     np.testing.assert_allclose(got[0][1], got[1][1], rtol=0, atol=1e-6 * np.abs(got[1][1]).max())
+
+
+# a group whose last pass has the smaller cutoff: the lists have room for the
+# widest pass (each pass is rounded to 2^-40 on its own, so the sums agree)
+@pytest.mark.parametrize("precision", ["mixed", "double"])
+@pytest.mark.parametrize("order", [(0, 1), (1, 0)])
+def test_capacity_of_the_widest_pass(gpu_ctx_factory, precision, order):
+    print("case: list capacity over passes", precision, order, flush=True)
+    s = water.named("water8k", seed=5, jitter=0.3)
+    c = context(gpu_ctx_factory, s, precision, list_skin=0)
+    hs = [c.force("LennardJones -algorithm NonbondedCutoff -switchingFunction C2", [11.0, 12.0, 12.0]),
+          c.force("Coulomb -algorithm NonbondedCutoff -switchingFunction C2", [3.0, 4.0, 4.0])]
+    parts = [c.evaluate([h], s.pos) for h in hs]
+    f, e = c.evaluate([hs[k] for k in order], s.pos)
+    want = parts[0][0] + parts[1][0]
+    assert np.abs(f - want).max() <= 4 * 2.0 ** -40 + 1e-14 * np.abs(want).max()
+    np.testing.assert_allclose(e, parts[0][1] + parts[1][1], rtol=1e-12, atol=1e-9)
+    v = np.random.default_rng(3).standard_normal((s.n, 3))
+    want = c.hessian_vec(hs[:1], s.pos, v) + c.hessian_vec(hs[1:], s.pos, v)
+    assert np.abs(c.hessian_vec([hs[k] for k in order], s.pos, v) - want).max() <= 1e-10 * np.abs(want).max()
