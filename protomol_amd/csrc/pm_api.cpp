@@ -290,6 +290,7 @@ struct pm_context {
   bool inner_last = false;           // the last evaluation's pair pass kept inner lists
   bool list_stale = true;            // x_build must be invalidated before the next reuse
   double list_cut = -1.0, list_built_skin = -1.0;   // pair cutoff and skin the kept lists are for
+  bool list_sorted = false;          // the kept lists hold their near entries first
   unsigned long long gen = 1;        // bumped by every allocation and every setter
   hipGraphExec_t md_exec = nullptr;
   int md_exec_steps = 0, md_exec_kind = -1;
@@ -1217,9 +1218,12 @@ bool list_reuse(const pm_context* c, const std::vector<PairPass>& passes) {
 }
 
 // Whether the kept lists were built for this pass: another pair cutoff (or
-// skin) lists other pairs, near ones by another distance, at another stride
+// skin) lists other pairs, near ones by another distance, at another stride;
+// and a run that replicas repeat sums its entries in their unsorted order
+// whatever was evaluated before it
 bool lists_match(const pm_context* c, const PairPass& p) {
-  return c->list_cut == std::sqrt(pair_params(p.terms, c->csf).cut2) && c->list_built_skin == list_skin(c);
+  return c->list_cut == std::sqrt(pair_params(p.terms, c->csf).cut2) && c->list_built_skin == list_skin(c) &&
+         c->list_sorted == !replica_form(c);
 }
 
 // Inner lists: with list reuse, an inner skin below the list skin
@@ -1315,6 +1319,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     if (!lists_match(c, passes[0])) c->list_stale = true;
     c->list_cut = pcut;
     c->list_built_skin = skin;
+    c->list_sorted = !replica_form(c);
   }
   if (!adj || !adj->kept) {
   TimedScope ts(c, PM_T_BIN);

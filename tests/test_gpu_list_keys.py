@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from protomol_amd import water
-from tests.cases import rms_rel
+from tests.cases import gpu_forces_c1, rms_rel
 
 pytestmark = pytest.mark.gpu
 LJ = "LennardJones CoulombEwaldReal -algorithm NonbondedCutoff -switchingFunction C2 -switchingFunction Cutoff"
@@ -87,3 +87,27 @@ def test_capacity_of_the_widest_pass(gpu_ctx_factory, precision, order):
     v = np.random.default_rng(3).standard_normal((s.n, 3))
     want = c.hessian_vec(hs[:1], s.pos, v) + c.hessian_vec(hs[1:], s.pos, v)
     assert np.abs(c.hessian_vec([hs[k] for k in order], s.pos, v) - want).max() <= 1e-10 * np.abs(want).max()
+
+
+# the lists of a run that replicas repeat are in their own order whatever the
+# context evaluated before the run was set up: the same bits
+@pytest.mark.parametrize("before", ["evaluate", "leapfrog"])
+def test_replica_run_after_other_work(gpu_ctx_factory, before):
+    print("case: replica run after", before, flush=True)
+    s = water.water_box(300, (300 / 0.0334) ** (1.0 / 3.0), seed=8, jitter=0.2)
+    got = []
+    for prepare in (True, False):
+        c = context(gpu_ctx_factory, s, "mixed")
+        hs = gpu_forces_c1(c) + [c.force("Bond", []), c.force("Angle", [])]
+        if prepare and before == "evaluate":
+            c.evaluate(hs, s.pos)
+        elif prepare:
+            c.md_setup(hs, "leapfrog", dt=1.0)
+            c.md_set_state(s.pos, s.vel)
+            c.md_run(1)
+        c.md_setup(hs, "langevin", dt=1.0, temperature=400.0, gamma=5.0, seed=3)
+        c.md_set_state(s.pos, s.vel)
+        c.md_run(30)
+        got.append(c.md_get_state())
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
