@@ -3069,6 +3069,31 @@ static int adjoint_run(pm_context* c, const int* handles, int nh, const double* 
   return PM_OK;
 }
 
+// `parts` runs of `each` values in d_scratch3 to the caller's arrays (null: not
+// wanted), which are left alone when the kernels flagged an error
+static int adjoint_results(pm_context* c, size_t each, int parts, double* const* out) {
+  double* h = host_stage(c, parts * each + 1);
+  std::vector<double> pageable;
+  if (!h) {
+    pageable.resize(parts * each + 1);
+    h = pageable.data();
+  }
+  int* word = reinterpret_cast<int*>(h + parts * each);
+  hipError_t e = hipGetLastError();
+  for (int k = 0; k < parts; k++)
+    if (out[k] && e == hipSuccess)
+      e = hipMemcpyAsync(h + k * each, c->d_scratch3 + k * each, each * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(word, c->d_overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
+  if (e != hipSuccess) return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
+  const int r = check_overflow(c, word);
+  if (r) return r;
+  for (int k = 0; k < parts; k++)
+    if (out[k]) std::copy(h + k * each, h + (k + 1) * each, out[k]);
+  return PM_OK;
+}
+
 int pm_hessian_vec(pm_context* c, const int* handles, int nh, const double* positions, const double* v,
                    double* hv) {
   if (!c || !v || !hv) return PM_ERR_ARGUMENT;
@@ -3077,14 +3102,7 @@ int pm_hessian_vec(pm_context* c, const int* handles, int nh, const double* posi
   if ((r = adjoint_run(c, handles, nh, positions, v, 1))) return r;
   const int n3 = 3 * c->n;
   pm_launch_fix_combine(c->stream, n3, c->d_adj_fix, c->d_adj_out, nullptr, c->d_scratch3);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(hv, c->d_scratch3, (size_t)n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  if (e != hipSuccess) {
-    hipStreamSynchronize(c->stream);
-    return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
-  }
-  return check_overflow(c);
+  return adjoint_results(c, n3, 1, &hv);
 }
 
 int pm_param_gradients(pm_context* c, const int* handles, int nh, const double* positions, double* dE_dq,
@@ -3098,17 +3116,8 @@ int pm_param_gradients(pm_context* c, const int* handles, int nh, const double* 
   const int n = c->n;
   // dE/dq, dE/dsigma = dE/dR dR/dsigma, dE/deps = dE/de / (2 e) one after the other
   pm_launch_param_out(c->stream, n, c->d_adj_fix, c->d_adj_out, c->d_atom_lj_d, std::pow(2.0, -5.0 / 6.0), c->d_scratch3);
-  hipError_t e = hipGetLastError();
-  double* host[3] = {dE_dq, dE_dsigma, dE_depsilon};
-  for (int k = 0; k < 3; k++)
-    if (host[k] && e == hipSuccess)
-      e = hipMemcpyAsync(host[k], c->d_scratch3 + (size_t)k * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost,
-                         c->stream);
-  if (e != hipSuccess) {
-    hipStreamSynchronize(c->stream);
-    return fail(c, PM_ERR_DEVICE, "HIP error %s copying the results", hipGetErrorString(e));
-  }
-  return check_overflow(c);
+  double* const out[3] = {dE_dq, dE_dsigma, dE_depsilon};
+  return adjoint_results(c, n, 3, out);
 }
 
 int pm_set_charges(pm_context* c, const double* q) {

@@ -89,3 +89,30 @@ def test_molecular_virial_request_is_refused(gpu_ctx_factory):
     with pytest.raises(gpu.PmError) as ei:
         c.evaluate(gpu_forces_c1(c), s.pos, virial=True, molecular_virial=True)
     assert ei.value.code == gpu.PM_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("precision", ["mixed", "double"])
+def test_derivatives_leave_the_outputs_on_an_error(gpu_ctx_factory, precision):
+    """A Hessian-vector product and parameter gradients that end in an error
+    (a position that is not finite) have not touched the caller's arrays, the
+    product not even where it is written over its direction."""
+    say(f"case: derivative outputs on an error water648 {precision}")
+    s = water.named("water648", seed=16, jitter=0.3)
+    c = _ctx(gpu_ctx_factory, s, precision)
+    c.set_lj_per_atom(np.where(s.type == 0, 3.15, 0.0), np.where(s.type == 0, 0.15, 0.0))
+    hs = np.array(gpu_forces_c1(c), np.int32)
+    bad = s.pos.copy()
+    bad[17, 1] = np.nan
+    bad = np.ascontiguousarray(bad).reshape(-1)
+    v = np.random.default_rng(4).standard_normal(3 * s.n)
+    hv = v.copy()
+    call = c.lib.pm_hessian_vec(c.h, gpu._ip(hs), len(hs), gpu._dp(bad), gpu._dp(hv), gpu._dp(hv))
+    assert call == gpu.PM_ERR_NUMERIC
+    np.testing.assert_array_equal(hv, v)
+    out = [np.full(s.n, 7.0) for _ in range(3)]
+    assert c.lib.pm_param_gradients(c.h, gpu._ip(hs), len(hs), gpu._dp(bad), *[gpu._dp(o) for o in out]) == gpu.PM_ERR_NUMERIC
+    assert all((o == 7.0).all() for o in out)
+    # the next valid calls find clean state
+    x = np.ascontiguousarray(s.pos).reshape(-1)
+    assert c.lib.pm_hessian_vec(c.h, gpu._ip(hs), len(hs), gpu._dp(x), gpu._dp(hv), gpu._dp(hv)) == gpu.PM_OK
+    np.testing.assert_array_equal(hv, c.hessian_vec(hs, s.pos, v).reshape(-1))
