@@ -2433,6 +2433,9 @@ int pm_evaluate(pm_context* c, const int* handles, int nh, const double* positio
   if (flags & ~(PM_EVAL_VIRIAL | PM_EVAL_MOLVIRIAL))
     return fail(c, PM_ERR_ARGUMENT, "pm_evaluate: unknown flags 0x%x", flags);
   const int n = c->n;
+  // (before anything can fail: the positions and lists change in any case)
+  c->md_forces_valid = false;
+  c->gen++;
   HIPCHECK(c, hipMemcpyAsync(c->d_pos, positions, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   std::vector<int> hv(handles, handles + nh);
   if ((r = evaluate_group(c, hv, flags))) return r;
@@ -2457,8 +2460,6 @@ int pm_evaluate(pm_context* c, const int* handles, int nh, const double* positio
   if ((r = check_overflow(c, word))) return r;
   for (size_t k = 0; k < n3; k++) forces[k] += f[k];
   for (int k = 0; k < PM_NE; k++) energies[k] += e[k];
-  c->md_forces_valid = false;
-  c->gen++;
   return PM_OK;
 }
 
@@ -2474,7 +2475,10 @@ int pm_cell_diagnostics(pm_context* c, const double* positions, double algorithm
   if ((r = ensure_cells(c))) return r;
   hipStream_t s = c->stream;
   HIPCHECK(c, hipMemcpyAsync(c->d_pos, positions, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
-  c->list_stale = true;   // the binning below replaces the layout's cell lists
+  // the positions and the binning below replace the MD state's and the layout's
+  c->list_stale = true;
+  c->md_forces_valid = false;
+  c->gen++;
   pm_launch_zero_i(s, c->d_bin_count, nc);
   pm_launch_bin(s, c->box, n, c->d_pos, c->d_cell_of, c->d_bin_count, c->d_cell_rank, c->d_key, nullptr);
   pm_launch_scan_cells(s, nc, c->box.n[2], c->d_bin_count, c->d_cell_count, c->d_cell_start, c->d_cell_slot, c->d_counts,

@@ -111,3 +111,32 @@ def test_replica_run_after_other_work(gpu_ctx_factory, before):
         got.append(c.md_get_state())
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+# cell diagnostics between two runs replace positions and cell lists: the next
+# run starts from their positions with forces and lists of its own
+@pytest.mark.parametrize("integrator", ["leapfrog", "langevin"])
+def test_md_after_cell_diagnostics(gpu_ctx_factory, integrator):
+    print("case: md after cell diagnostics", integrator, flush=True)
+    s = water.named("water648", seed=7, jitter=0.2)
+    move = np.repeat(np.random.default_rng(5).uniform(-0.15, 0.15, (s.n // 3, 3)), 3, axis=0)
+    got = []
+    for diagnostics in (True, False):
+        c = context(gpu_ctx_factory, s, "double")
+        hs = [c.force(LJ, values(8.0)), c.force("Bond", []), c.force("Angle", []),
+              c.force("Coulomb -algorithm PMEwald -reciprocal -correction -interpolation BSpline",
+                      [24, 24, 24, 8.0, 4, 1e-6, 0.4])]
+        kw = dict(temperature=300.0, gamma=5.0, seed=3) if integrator == "langevin" else {}
+        c.md_setup(hs, integrator, dt=0.5, **kw)
+        c.md_set_state(s.pos, s.vel)
+        for _ in range(3):
+            c.md_run(20)
+            x, v, _ = c.md_get_state()
+            if diagnostics:
+                c.cell_diagnostics(x + move, 8.0, 8.0)
+            else:
+                c.md_set_state(x + move, v)
+        c.md_run(20)
+        got.append(c.md_get_state()[:2])
+    np.testing.assert_allclose(got[0][0], got[1][0], rtol=0, atol=1e-7)
+    np.testing.assert_allclose(got[0][1], got[1][1], rtol=0, atol=1e-6 * np.abs(got[1][1]).max())
