@@ -2223,6 +2223,13 @@ int pm_set_lj_per_atom(pm_context* c, const double* sigma, const double* epsilon
   int r;
   if ((r = set_device(c))) return r;
   if (!c->have_topo) return fail(c, PM_ERR_STATE, "no topology: call pm_set_topology first");
+  const int n = c->n;
+  if (sigma) {   // (a refused call changes nothing)
+    if (!epsilon) return fail(c, PM_ERR_ARGUMENT, "pm_set_lj_per_atom: epsilon missing");
+    for (int i = 0; i < n; i++)
+      if (!(sigma[i] >= 0) || !(epsilon[i] >= 0) || (sigma14 && !(sigma14[i] >= 0)) || (epsilon14 && !(epsilon14[i] >= 0)))
+        return fail(c, PM_ERR_ARGUMENT, "atom %d: sigma and epsilon must be >= 0", i);
+  }
   c->gen++;
   c->md_forces_valid = false;
   if (!sigma) {
@@ -2232,8 +2239,6 @@ int pm_set_lj_per_atom(pm_context* c, const double* sigma, const double* epsilon
     c->lj_e.clear();
     return PM_OK;
   }
-  if (!epsilon) return fail(c, PM_ERR_ARGUMENT, "pm_set_lj_per_atom: epsilon missing");
-  const int n = c->n;
   const double rfac = std::pow(2.0, -5.0 / 6.0);   // Rmin/2 = sigma 2^(1/6) / 2
   std::vector<float4> f(n);
   std::vector<double4> d(n);
@@ -2242,8 +2247,6 @@ int pm_set_lj_per_atom(pm_context* c, const double* sigma, const double* epsilon
   for (int i = 0; i < n; i++) {
     const double s1 = sigma[i], e1 = epsilon[i];
     const double s4 = sigma14 ? sigma14[i] : s1, e4 = epsilon14 ? epsilon14[i] : e1;
-    if (!(s1 >= 0) || !(e1 >= 0) || !(s4 >= 0) || !(e4 >= 0))
-      return fail(c, PM_ERR_ARGUMENT, "atom %d: sigma and epsilon must be >= 0", i);
     const double R1 = s1 * rfac, E1 = std::sqrt(e1), R4 = s4 * rfac, E4 = std::sqrt(e4);
     c->lj_R[i] = R1;
     c->lj_e[i] = E1;

@@ -9,7 +9,7 @@ sums, of about 1e3 terms each (1e-9)."""
 import numpy as np
 import pytest
 
-from protomol_amd import water
+from protomol_amd import gpu, water
 from tests.cases import ALPHA_RC8, rms_rel
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +75,24 @@ def test_lanczos_matches_single_products(gpu_ctx_factory, forces, pme, spread):
     scale = max(np.abs(ra).max(), np.abs(rb).max())
     np.testing.assert_allclose(alpha, ra, rtol=0, atol=1e-8 * scale)
     np.testing.assert_allclose(beta, rb, rtol=0, atol=1e-8 * scale)
+
+
+def test_refused_parameters_change_nothing(gpu_ctx_factory):
+    """A refused pm_set_lj_per_atom leaves a context without per-atom
+    parameters without them, and one with them as it was."""
+    print("case: refused per-atom parameters", flush=True)
+    s, sigma, eps = water.perturbed_box("water648", seed=3)
+    bad = sigma.copy()
+    bad[5] = -1.0
+    c, hs = context(gpu_ctx_factory, s, "one pass", 4)
+    with pytest.raises(gpu.PmError):
+        c.set_lj_per_atom(bad, eps)
+    with pytest.raises(gpu.PmError) as e:
+        c.param_gradients(hs, s.pos)
+    assert e.value.code == gpu.PM_ERR_STATE
+    c.set_lj_per_atom(sigma, eps)
+    want = c.param_gradients(hs, s.pos)
+    with pytest.raises(gpu.PmError):
+        c.set_lj_per_atom(2.0 * bad, 3.0 * eps)
+    for a, b in zip(c.param_gradients(hs, s.pos), want):
+        np.testing.assert_array_equal(a, b)
