@@ -248,9 +248,7 @@ struct pm_context {
   std::vector<PmeTables> pme_tables;
   unsigned long long pme_group = 0;
   int pme_nx = 0, pme_ny = 0;   // grid of the term prepared last (pm_get_option)
-  double* d_lat = nullptr;   // lattice vectors of the PME real term in small boxes
-  int nlat = 0;
-  double lat_key[4] = {0, 0, 0, 0};   // rc and box edges d_lat was built for
+  std::map<double, std::pair<double*, int>> lattices;   // lattice vectors of the PME real term in small boxes, by cutoff
 
   // MD
   std::vector<int> md_handles;
@@ -489,11 +487,14 @@ int get_stencil(pm_context* c, double cutoff, bool half, int4** dptr, int* count
   return PM_OK;
 }
 
-void free_stencils(pm_context* c) {
+// what follows from the box: stencils and lattice vectors
+void free_box_tables(pm_context* c) {
   for (auto& kv : c->stencils) hipFree(kv.second.first);
   for (auto& kv : c->half_stencils) hipFree(kv.second.first);
+  for (auto& kv : c->lattices) hipFree(kv.second.first);
   c->stencils.clear();
   c->half_stencils.clear();
+  c->lattices.clear();
 }
 
 // ------------------------------------------------------------ allocation
@@ -1113,8 +1114,7 @@ bool pme_lattice(const pm_context* c, const ForceDesc& f) {
 // reference's std::sort leaves their order unspecified, which matters only
 // for a MODIFIED pair whose primary image lies beyond the cutoff)
 int ensure_lattice(pm_context* c, double rc) {
-  const double key[4] = {rc, c->box.L[0], c->box.L[1], c->box.L[2]};
-  if (c->d_lat && std::equal(key, key + 4, c->lat_key)) return PM_OK;
+  if (c->lattices.count(rc)) return PM_OK;
   const double lx = c->box.L[0], ly = c->box.L[1], lz = c->box.L[2];
   const int bk = (int)std::floor(rc / lx + 1.0), bl = (int)std::floor(rc / ly + 1.0), bm = (int)std::floor(rc / lz + 1.0);
   std::vector<std::array<double, 3>> v;
@@ -1134,9 +1134,9 @@ int ensure_lattice(pm_context* c, double rc) {
   std::vector<double> flat = {0.0, 0.0, 0.0};
   for (auto& a : v) flat.insert(flat.end(), a.begin(), a.end());
   int r;
-  if ((r = upload(c, &c->d_lat, flat))) return r;
-  c->nlat = (int)v.size() + 1;
-  std::copy(key, key + 4, c->lat_key);
+  double* d = nullptr;
+  if ((r = upload(c, &d, flat))) { dfree(d); return r; }
+  c->lattices[rc] = std::make_pair(d, (int)v.size() + 1);
   return PM_OK;
 }
 
@@ -1685,7 +1685,8 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     long long off = hr.second + (f.recip ? pm_pme_xpass_blocks(f.nx, f.ny, f.nz, c->precision, pme_plane(c, f)) : 0) +
                     (f.corr ? ((long long)c->tab_a.size() + 255) / 256 : 0);
     TimedScope ts(c, PM_T_PME, s2);
-    pm_launch_ewald_lattice(s2, c->box, n, c->d_pos, c->d_q, c->d_xs_row, c->d_xs_part, c->d_lat, c->nlat,
+    const auto& lat = c->lattices[f.rc];
+    pm_launch_ewald_lattice(s2, c->box, n, c->d_pos, c->d_q, c->d_xs_row, c->d_xs_part, lat.first, lat.second,
                             f.rc * f.rc, f.alpha, c->csf, vir ? 1 : 0, c->d_force, c->d_epart + off * PM_NE,
                             lattice_blocks(n));
   }
@@ -1947,8 +1948,6 @@ void free_all(pm_context* c) {
   c->pme_points = c->pme_bytes_r = c->pme_bytes_c = 0;
   for (PmeTables& t : c->pme_tables) free_tables(t);
   c->pme_tables.clear();
-  dfree(c->d_lat);
-  c->nlat = 0;
   dfree(c->d_b_a); dfree(c->d_b_b); dfree(c->d_b_k); dfree(c->d_b_r0);
   dfree(c->d_a_a); dfree(c->d_a_b); dfree(c->d_a_c);
   dfree(c->d_a_k); dfree(c->d_a_t0); dfree(c->d_a_kub); dfree(c->d_a_rub);
@@ -1964,7 +1963,7 @@ void free_all(pm_context* c) {
   dfree(c->d_cons_x); dfree(c->d_cons_v); dfree(c->d_cons_xl);
   c->cons_built = false;
   c->cons_n = c->cons_ngroup = c->cons_err_cap = 0;
-  free_stencils(c);
+  free_box_tables(c);
   c->cells_alloc = 0;
   c->jlist_alloc = 0;
   c->epart_alloc = 0;
@@ -2384,7 +2383,7 @@ int pm_set_boundary(pm_context* c, const double* e1, const double* e2, const dou
     return fail(c, PM_ERR_CAPACITY, "Your systems is expanding such that the the ratio simulation box / cell size is to big.");
   c->ncells = (int)ncl;
   c->cellsize = cellsize;
-  free_stencils(c);
+  free_box_tables(c);
   c->cells_alloc = 0;
   for (PmeTables& t : c->pme_tables) t.current = false;
   c->have_box = true;

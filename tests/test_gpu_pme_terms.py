@@ -88,3 +88,19 @@ def test_terms_of_a_group_add_up(gpu_ctx_factory, precision, spread, values):
         tol = (1e-5 if precision == "mixed" else 1e-11) * max(np.abs(ra).max(), np.abs(rb).max())
         np.testing.assert_allclose(alpha, ra, rtol=0, atol=tol)
         np.testing.assert_allclose(beta, rb, rtol=0, atol=tol)
+
+
+# two real terms in a box no wider than twice their cutoffs, each with the
+# lattice images of its own cutoff
+@pytest.mark.parametrize("cutoffs", [(14.0, 9.4), (9.4, 14.0)])
+def test_real_terms_of_two_cutoffs(gpu_ctx_factory, cutoffs):
+    print("case: real terms of two cutoffs", cutoffs, flush=True)
+    s = water.named("water648", seed=8, jitter=0.3)
+    c = context(gpu_ctx_factory, s, "double")
+    hs = [c.force("Coulomb -algorithm PMEwald -real -correction -interpolation BSpline", [24, 24, 24, rc, 4, 1e-6, 0.15])
+          for rc in cutoffs]
+    f, e = c.evaluate(hs, s.pos)
+    parts = [c.evaluate([h], s.pos) for h in hs]
+    want = parts[0][0] + parts[1][0]
+    assert np.abs(f - want).max() <= 16 * 2.0 ** -40 + 1e-14 * np.abs(want).max()
+    np.testing.assert_allclose(e, parts[0][1] + parts[1][1], rtol=1e-12, atol=1e-9)
