@@ -2194,7 +2194,15 @@ void pm_launch_bin(hipStream_t s, const PmBox& box, int n, const double* pos, in
                        rebuild);
 }
 
-#define PM_SCAN_SCATTER 16384
+// Atoms up to which the scan's single block also scatters, in rounds of 1,024:
+// a launch less, whose boundary costs a step that keeps its lists 1-2 us (25
+// mixed-precision steps, us per step: 1,020 atoms 41 merged, 43 apart; 8,190 66
+// and 67; 12,000 68 and 69; 16,383 75 and 73.5), against the rounds on a step
+// that builds (every step a build: 3,000 atoms 86.5 and 86.5; 4,095 96.5 and 96;
+// 8,190 98.5 and 96; 16,383 112 and 105).  Hence one line for evaluations that may
+// keep their lists (one build in nine steps) and one for those that never do
+#define PM_SCAN_SCATTER 12288
+#define PM_SCAN_SCATTER_BUILD 3072
 static void launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank, const int* cell_start,
                            int* cell_atoms, const int* rebuild) {
   if (pm_recording()) {
@@ -2227,10 +2235,7 @@ void pm_launch_scan_cells(hipStream_t s, int ncells, int nz, int* bin_count, int
     launch_scatter(s, n, cell_of, rank, cell_start, cell_atoms, rebuild);
     return;
   }
-  // Up to PM_SCAN_SCATTER atoms the scan's block also scatters (16 rounds at
-  // most, on build steps only): a launch less on every step, and a launch that
-  // returns at once still costs its boundary, about 4.5 us
-  const bool merged = n <= PM_SCAN_SCATTER;
+  const bool merged = n <= (rebuild ? PM_SCAN_SCATTER : PM_SCAN_SCATTER_BUILD);
   hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(1024), 0, s, ncells, nz, bin_count, cell_count, cell_start,
                      cell_slot, counts, cluster_cell, ncl_max, m, rebuild, merged ? n : 0, cell_of, rank, cell_atoms);
   if (!merged) launch_scatter(s, n, cell_of, rank, cell_start, cell_atoms, rebuild);

@@ -57,13 +57,15 @@ def test_pair_forces_over_launch_shapes(gpu_ctx_factory, port, molecules, kind, 
         np.testing.assert_allclose(e[:2], er[:2], rtol=10 * TOL[precision], atol=1e-6 * np.abs(er[:2]).max())
 
 
-# the scan of up to 16,384 atoms also scatters them: a box on each side
-@pytest.mark.parametrize("molecules", [5461, 5462])
-def test_forces_over_layout_launches(gpu_ctx_factory, port, molecules):
-    print("case: layout launches", molecules, flush=True)
+# the scan of up to 12,288 atoms (3,072 where every evaluation builds its
+# lists) also scatters them: a box on each side, and two larger ones
+@pytest.mark.parametrize("molecules,skin", [(4096, -1), (4097, -1), (1024, 0), (1025, 0), (5461, -1), (5462, -1)])
+def test_forces_over_layout_launches(gpu_ctx_factory, port, molecules, skin):
+    print("case: layout launches", molecules, skin, flush=True)
     s = water.water_box(molecules, (molecules / 0.0334) ** (1.0 / 3.0), seed=molecules, jitter=0.3)
     c = gpu_ctx_factory("double")
     c.set_topology(s)
     c.set_boundary(s.box, s.origin, 4.0)
+    c.set_option("list_skin", skin)
     f, _ = c.evaluate(gpu_forces_c1(c), s.pos)
     assert rms_rel(f, reference(port, s, s.pos)[0]) < TOL["double"]
