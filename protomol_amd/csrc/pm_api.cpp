@@ -1433,6 +1433,7 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.xs_tcap = c->m * c->xs_maxdeg;
     a.m = c->m;
     a.jlanes = pair_lanes(c);
+    a.beside = pme_rec.empty() ? 0 : 1;
     a.split_log = adj ? adjoint_split(c) : slog;
     a.near_margin = replica_form(c) ? PM_NEAR_ALL : PM_NEAR_MARGIN;
     a.lj_types = c->lj_types;

@@ -53,9 +53,10 @@
 // iteration, the cluster's box): small, so that the kernel leaves most of a
 // CU's LDS to the PME kernels that run beside it on the other stream
 #define PM_JL_LDS(T) (3 * 64 * sizeof(T) + 64 * sizeof(int) + 8 * sizeof(T))
-// Waves per block of k_pair_jl at most, and the launches (waves) that take them
+// Waves per block of k_pair_jl at most, and the launches (slots times waves per
+// cluster, beside PME kernels) that take them
 #define PM_JL_WAVES(T) (sizeof(T) == 4 ? 8 : 4)
-#define PM_JL_WIDE_MAX 32768
+#define PM_JL_WIDE_MAX 163840
 // List entries within the pair cutoff + this many A of the cluster at the
 // build are near ones: the motion between two builds rarely takes a pair
 // beyond it (98k water: a hydrogen moves 0.2-0.3 A over the nine steps)
@@ -151,6 +152,7 @@ struct PmNbLaunch {
   int m;                     // atoms per cluster (4 or 8)
   int split_log;             // log2 of the waves per cluster of k_pair_jl and k_adjoint
   unsigned long long lj_types;  // bit t % 64: type t has Lennard-Jones parameters with some type
+  int beside;                // 1: PME kernels run beside the pair kernel
   int jlanes;                // pair kernel: 1 one lane per list entry (k_pair_jl), 0 rows of m lanes (k_pair)
   // topology
   const int* molecule;

@@ -2350,13 +2350,15 @@ static void launch_pair_t(hipStream_t s, const PmBox& box, const PmNbLaunch& a, 
     return;
   }
   if (a.jlanes) {
-    // Blocks of 8 waves in mixed precision where the launch is a few rounds
-    // of the chip: a CU then frees two waves per SIMD at a time, and the PME
-    // kernels of the second stream find room for a block sooner (98k water,
-    // 50 steps with PME: 11.40 ms with 8, 12.17 with 4, 12.2 / 11.7 / 12.0
-    // with 10 / 12 / 16).  In larger boxes the pair kernel bounds the step
-    // and 4 are better (a million atoms, 16 steps: 37.2 ms with 4, 38.9 with 8)
-    const int W = sizeof(T) == 4 && waves <= PM_JL_WIDE_MAX ? PM_JL_WAVES(T) : 4;
+    // Blocks of 8 waves in mixed precision beside PME where the launch is a few
+    // rounds of the chip: a CU then frees two waves per SIMD at a time, and the
+    // PME kernels of the second stream find room for a block sooner (98k water,
+    // 50 steps: 11.40 ms with 8, 12.17 with 4, 12.2 / 11.7 / 12.0 with 10 / 12 /
+    // 16).  us per step with 8 and with 4: 102,000 slots 233 and 249 (clusters of
+    // 4 atoms 290 and 302), 134,000 283 and 289, 168,000 344 and 342, 202,000
+    // 412 and 396; a million atoms, 16 steps: 38.9 and 37.2 ms.  Without PME beside it the kernel is faster with
+    // 4 (98k atoms, rc 8: 84 and 80 us; 142 and 138.5 us per step)
+    const int W = sizeof(T) == 4 && a.beside && waves * a.m <= PM_JL_WIDE_MAX ? PM_JL_WAVES(T) : 4;
     const size_t ljl = tab + (size_t)W * PM_JL_LDS(T);
     const dim3 g((waves + W - 1) / W), b(64 * W);
     if constexpr (LJ != PM_SWF_NONE) {

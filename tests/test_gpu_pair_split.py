@@ -23,9 +23,9 @@ def reference(port, s, x):
     return a["forces"] + b["forces"], a["energies"] + b["energies"]
 
 
-# molecules: 8, 4, 2 and 1 waves per cluster, and a launch on each side of a
-# change (about 1,024 waves)
-@pytest.mark.parametrize("molecules", [150, 217, 600, 1301, 2600])
+# molecules: 8 (two sizes), 4, 2 and 1 (two sizes) waves per cluster, as many
+# as keep the launch within 1,024 waves
+@pytest.mark.parametrize("molecules", [150, 217, 300, 600, 1301, 2600])
 @pytest.mark.parametrize("kind", ["water", "exclusions", "uncharged"])
 @pytest.mark.parametrize("precision", ["mixed", "double"])
 def test_pair_forces_over_launch_shapes(gpu_ctx_factory, port, molecules, kind, precision):
@@ -55,6 +55,30 @@ def test_pair_forces_over_launch_shapes(gpu_ctx_factory, port, molecules, kind, 
         print("rms rel force", err, flush=True)
         assert err < TOL[precision]
         np.testing.assert_allclose(e[:2], er[:2], rtol=10 * TOL[precision], atol=1e-6 * np.abs(er[:2]).max())
+
+
+# blocks of 8 waves beside PME in mixed precision up to 163,840 slots: 163,688
+# and 163,992, beside PME and alone, against the row-per-entry kernel
+# (5e-6: FP32 pair arithmetic on both sides)
+@pytest.mark.parametrize("molecules", [52600, 52700])
+def test_forces_over_block_widths(gpu_ctx_factory, molecules):
+    print("case: block widths", molecules, flush=True)
+    s = water.water_box(molecules, (molecules / 0.0334) ** (1.0 / 3.0), seed=molecules, jitter=0.3)
+    got = []
+    for lanes in (0, 1):
+        c = gpu_ctx_factory("mixed")
+        c.set_topology(s)
+        c.set_boundary(s.box, s.origin, 4.0)
+        c.set_option("pair_lanes", lanes)
+        hs = gpu_forces_c1(c)
+        pme = c.force("Coulomb -algorithm PMEwald -reciprocal -correction -interpolation BSpline",
+                      [108, 108, 108, 8.0, 4, 1e-6, -1.0])
+        alone, both = c.evaluate(hs, s.pos), c.evaluate(hs + [pme], s.pos)
+        p = c.evaluate([pme], s.pos)
+        got.append((alone, (both[0] - p[0], both[1] - p[1])))
+    for (f, e), (fr, er) in zip(got[1], got[0]):
+        assert rms_rel(f, fr) < TOL["mixed"]
+        np.testing.assert_allclose(e[:2], er[:2], rtol=1e-4)
 
 
 # the scan of up to 12,288 atoms (3,072 where every evaluation builds its
