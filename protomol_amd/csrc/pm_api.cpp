@@ -34,7 +34,10 @@
 #define PM_PRUNE_SKIN_AUTO 0.0
 // waves up to which a cluster's list is shared by several (pair_split)
 #define PM_SPLIT_WAVES 1024
-// values of x or v up to which pm_md_get_state copies through pinned memory
+// values of x or v up to which pm_md_get_state copies through pinned memory: a
+// bound on that memory (twice this many doubles), not the line where it stops
+// paying (us per call staged and straight: 648 atoms 27 and 57, 8,100 53 and
+// 200, 21,843 86 and 92 to 190, 98,304 325 and 355 to 396)
 #define PM_STAGE_STATE 65536
 // tables of PME terms that a context keeps before it refills unused ones
 #define PM_PME_TABLES 4
@@ -113,7 +116,7 @@ struct pm_context {
   int device = 0;
   int lds_max = 65536;             // LDS bytes a workgroup may use on this device
   hipStream_t stream = nullptr;
-  hipStream_t stream2 = nullptr;   // PME, correction and bonded work, beside the pair work
+  hipStream_t stream2 = nullptr;   // PME and correction work, beside the bonded and pair work
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::string err;
   int precision = PM_PRECISION_MIXED;
@@ -526,7 +529,7 @@ double prune_skin(const pm_context* c) {
 }
 
 // pair kernel layout in effect: the lane-per-entry kernel (1) unless the
-// option asks for rows (0) or its LDS (type table + four waves' areas) would
+// option asks for rows (0) or its LDS (type table + a block's wave areas) would
 // not fit a workgroup (FP64 with over 41 atom types)
 static int pair_lanes(const pm_context* c) {
   const bool dbl = c->precision == PM_PRECISION_DOUBLE;
@@ -539,7 +542,9 @@ static int pair_lanes(const pm_context* c) {
 // PME).  Replicas walk their lists unsorted with one wave per cluster, alone
 // as in a batch: their boxes share the chip, so that more waves only cost, and
 // a hot box amplifies a change of the summation order 20,000 times in 50
-// steps; this order gives the same trajectory alone and in a batch.
+// steps; this order gives the same trajectory alone and in a batch.  A small
+// box on its own pays for that: 648 atoms 65 us a step (FP64 74) where
+// leapfrog, with several waves per cluster, takes 38 (FP64 44).
 static bool replica_form(const pm_context* c) {
   if (c->md_handles.empty() || c->md_integrator != PM_INTEGRATOR_LANGEVIN) return false;
   for (int h : c->md_handles)
@@ -569,8 +574,9 @@ static int adjoint_split(const pm_context* c) {
 }
 
 // What the passes need of the charges: their sums, and the types with
-// Lennard-Jones parameters, for the pair kernel to leave the others' terms out.  With an uncharged atom every type counts: two atoms on
-// one point then still show as a force that is not finite.
+// Lennard-Jones parameters, for the pair kernel to leave the others' terms out.
+// With an uncharged atom every type counts: two atoms on one point then still
+// show as a force that is not finite.
 static void set_charge_data(pm_context* c) {
   c->q2_sum = c->q_sum = 0.0;
   for (double q : c->q) { c->q2_sum += q * q; c->q_sum += q; }
@@ -1607,12 +1613,12 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     return PM_OK;
   }
 
-  // fork: PME, correction and bonded terms on the second stream, the pair
-  // lists and pair kernels on the first; they write different force arrays
-  // (per atom, per slot) and different energy records
+  // fork: PME and correction on the second stream; the bonded terms, the pair
+  // lists and pair kernels on the first.  They write different force arrays
+  // (the side array; per atom, per slot), but for the lattice term, which adds
+  // to the per-atom one by integer atomics as the bonded terms do, and
+  // different energy records
   hipStream_t s2 = c->stream2;
-  // the second stream pays off beside the PME kernels; bonded terms alone
-  // stay on the first
   const bool side = !pme_rec.empty();
   if (!side) s2 = s;
   if (side) {
@@ -2685,8 +2691,10 @@ int pm_shake_noalloc(pm_context* c, double* x, double* v, const double* x_last, 
   HIPCHECK(c, hipMemcpyAsync(dxl, x_last, bytes, hipMemcpyHostToDevice, s));
   int sw = 0;
   if (c->cons_ngroup > 0) {
-    // every wave of the probe writes its error part for every sweep count and
-    // the apply kernel writes the sweep count, so nothing here starts at zero
+    // every wave of the probes writes its error part for every sweep count up
+    // to the one that is taken (later ones may hold anything: the first within
+    // epsilon counts) and the apply kernel writes the sweep count, so nothing
+    // here starts at zero
     PmConstraints k = constraint_launch(c, eps, max_iter, dt_fs);
     k.err = derr;
     k.sweeps = dsweeps;
@@ -2960,7 +2968,7 @@ int pm_md_get_state(pm_context* c, double* x, double* v, double* energies) {
   int r;
   if ((r = set_device(c))) return r;
   // small boxes: all results through pinned memory with one wait; large arrays
-  // go straight to the caller, whose copy would take longer than the wait
+  // go straight to the caller
   const size_t n3 = 3 * (size_t)c->n;
   const bool staged = n3 <= PM_STAGE_STATE;
   double* h = host_stage(c, (staged ? 2 * n3 : 0) + PM_NE + 1);

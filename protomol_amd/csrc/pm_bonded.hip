@@ -4,10 +4,10 @@
 // BondSystemForce::calcBond (forces/BondSystemForce.h:111-145),
 // AngleSystemForce::calcAngle (forces/AngleSystemForce.h:113-200) and
 // MTorsionSystemForce::calcTorsion (forces/MTorsionSystemForce.h:34-153) for
-// DihedralSystemForce and ImproperSystemForce.  Forces
-// are computed once per term and added to the atoms as 64-bit fixed-point
-// atomics (deterministic: integer sums do not depend on their order).  Energies and virials are summed per term in fixed-order block
-// reductions.
+// DihedralSystemForce and ImproperSystemForce.  Forces are computed once per
+// term and added to the atoms as 64-bit fixed-point atomics (deterministic:
+// integer sums do not depend on their order).  Energies and virials are summed
+// per term in fixed-order block reductions.
 #include "pm_internal.h"
 #include "pm_terms.h"
 

@@ -1458,12 +1458,12 @@ __device__ inline double min_image(long long a, long long b) {
 // in its lane and is added with one 64-bit integer atomic per component, with
 // no cross-lane sums; the i forces accumulate per lane in FP32 (one term per
 // iteration and i atom; FP64 in the FP64 kernel) and are summed over the
-// lanes in FP64 at the end, by halving shuffles in a fixed order.  Same pair arithmetic
-// and the same half-list rule as pair_cluster; only the order in which FP32
-// partial sums are formed differs.
+// lanes in FP64 at the end, by halving shuffles in a fixed order.  Same pair
+// arithmetic and the same half-list rule as pair_cluster; only the order in
+// which FP32 partial sums are formed differs.
 // VALU issue bounds it in boxes that fill the chip, so it leaves out what a
 // wave-uniform test can: the iterations of far entries whose 64 entries all
-// lie beyond the cutoff of the cluster's bounding box, the exclusion test of
+// lie beyond the cutoff of the cluster's bounding box, the mask loads of
 // iterations without a flagged entry, the pair arithmetic of an i atom none
 // of whose 64 pairs is within the cutoff, and the Lennard-Jones terms of an
 // i atom whose type has none with any type (the hydrogens of water models).
@@ -1614,19 +1614,15 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
     if constexpr (sizeof(T) == 4) qj = __int_as_float(pj.w); else qj = __longlong_as_double(pj.w);
     const int tj = mj & 0xff;
     T fjx = 0, fjy = 0, fjz = 0;
-    // the pair of this lane's entry with cluster atom ii: FL 0 for iterations
-    // without flagged entries, 1 for the ordinary pairs of the others (FULL
-    // and modified ones masked; xm is 0 for entries the list did not flag), 2
-    // for the modified (1-4) pairs, with the 1-4 LJ parameters and the
-    // Coulomb scaling
-    auto pair_ii = [&](const int ii, auto fl) {
-      constexpr int FL = decltype(fl)::value;
-      constexpr bool MOD = FL == 2;
+    // the pair of this lane's entry with cluster atom ii: MOD false for the
+    // ordinary pairs (FULL and modified ones masked; xm is 0 for entries the
+    // list did not flag), true for the modified (1-4) pairs, with the 1-4 LJ
+    // parameters and the Coulomb scaling
+    auto pair_ii = [&](const int ii, auto mod) {
+      constexpr bool MOD = decltype(mod)::value;
       const T dx = min_image(pj.x, ipx[ii]) * sx, dy = min_image(pj.y, ipy[ii]) * sy, dz = min_image(pj.z, ipz[ii]) * sz;
       const T r2 = dx * dx + dy * dy + dz * dz;
-      bool mask = r2 <= cut2;
-      if constexpr (FL == 1) mask = mask && (xm & (65537u << ii)) == 0u;
-      if constexpr (FL == 2) mask = mask && (xm & (65536u << ii)) != 0u;
+      const bool mask = r2 <= cut2 && (MOD ? (xm & (65536u << ii)) != 0u : (xm & (65537u << ii)) == 0u);
       if (__ballot(mask) == 0ull) return;   // no lane's pair with atom ii counts
       T rr2, rinv;
       if constexpr (sizeof(T) == 4) { rinv = Prec<T>::rsq(r2); rr2 = rinv * rinv; }
@@ -1718,11 +1714,11 @@ __device__ inline void pair_cluster_jl(const PmBox& box, const PmNbLaunch& a, co
     // (padding slots skipped: uniform)
 #pragma unroll
     for (int ii = 0; ii < M; ii++)
-      if ((rm >> ii) & 1u) pair_ii(ii, std::integral_constant<int, 1>{});
+      if ((rm >> ii) & 1u) pair_ii(ii, std::false_type{});
     if (any_mod) {
 #pragma unroll
       for (int ii = 0; ii < M; ii++)
-        if ((rm >> ii) & 1u) pair_ii(ii, std::integral_constant<int, 2>{});
+        if ((rm >> ii) & 1u) pair_ii(ii, std::true_type{});
     }
     // j forces: the 64 entries' x, y, z regrouped through LDS so that lane
     // v of round r adds component v % 3 of entry v / 3 (v = 64 r + lane):

@@ -34,7 +34,10 @@
 
 // Sweeps whose errors the first probe records: water at 2 fs and epsilon 1e-5
 // needs 12 or 13, a sweep of the probe takes 1 us, and a count beyond the first
-// probe repeats it (98k water, 25 steps: 9.02 ms at 16, 9.13 at 30, 9.64 at 12)
+// probe repeats it (98k water, 25 steps: 9.02 ms at 16, 9.13 at 30, 9.64 at 12).
+// Tighter epsilons, which need the second probe, in us per 98k step with one
+// probe of maxIter sweeps and blocks of four waves, and now: 1e-7 375 and 344,
+// 1e-9 (maxIter 40) 408 and 368, 1e-12 (60) 466 and 405; 1e-5 354 and 306
 #define PM_PROBE_FIRST 16
 // waves up to which a block is one wave
 #define PM_CONS_WAVE_BLOCKS 1024
