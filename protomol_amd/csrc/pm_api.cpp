@@ -658,11 +658,18 @@ int list_capacity(const pm_context* c, double cut) {
   return (int)std::max(cap, 64LL);
 }
 
+// whether the lists have room for `lcap` entries per cluster (else a build has
+// to follow: new buffers hold no lists)
+bool lists_fit(const pm_context* c, int lcap, bool inner) {
+  const long long need = (long long)c->ncl_max * lcap;
+  return c->d_jlist && need <= c->jlist_alloc && (!inner || (c->d_ilist && need <= c->ilist_alloc));
+}
+
 int ensure_lists(pm_context* c, int lcap) {
   long long need = (long long)c->ncl_max * lcap;
   if (need <= c->jlist_alloc && c->d_jlist) { c->lcap = lcap; return PM_OK; }
   int r;
-  c->list_stale = true;   // the new buffers hold no lists
+  c->jlist_alloc = 0;
   if ((r = dalloc(c, &c->d_jlist, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jmask, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_jcount, c->ncl_max))) return r;
@@ -677,7 +684,7 @@ int ensure_inner_lists(pm_context* c) {
   const long long need = (long long)c->ncl_max * c->lcap;
   if (need <= c->ilist_alloc && c->d_ilist) return PM_OK;
   int r;
-  c->list_stale = true;
+  c->ilist_alloc = 0;
   if ((r = dalloc(c, &c->d_ilist, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_imask, (size_t)need))) return r;
   if ((r = dalloc(c, &c->d_icount, c->ncl_max))) return r;
@@ -809,8 +816,9 @@ int fill_tables(pm_context* c, PmeTables& t) {
   const size_t er = t.prec == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
   int r;
   if (!t.tw) {
-    if (!fft_plan(nx, t.plans[0]) || !fft_plan(ny, t.plans[1]) || !fft_plan(nz, t.plans[2]))
-      return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: the GPU FFT handles lengths with factors 2, 3, 5 and 7 only", nx, ny, nz);
+    fft_plan(nx, t.plans[0]);
+    fft_plan(ny, t.plans[1]);
+    fft_plan(nz, t.plans[2]);
     // twiddles exp(-2 pi i m / n) for the three lengths
     std::vector<double> tw;
     int off = 0;
@@ -873,11 +881,16 @@ int ensure_pme(pm_context* c, const std::vector<int>& handles) {
     const int nx = f.nx, ny = f.ny, nz = f.nz;
     if (nx > 4096 || ny > 4096 || nz > 4096 || nx < 8 || ny < 8 || nz < 8)
       return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: 8 to 4096 points per axis", nx, ny, nz);
+    PmFftPlan p;
+    if (!fft_plan(nx, p) || !fft_plan(ny, p) || !fft_plan(nz, p))
+      return fail(c, PM_ERR_UNSUPPORTED, "PME grid %d x %d x %d: the GPU FFT handles lengths with factors 2, 3, 5 and 7 only", nx, ny, nz);
     points = std::max(points, (size_t)nx * ny * nz);
     cpoints = std::max(cpoints, (size_t)nx * ny * (nz / 2 + 1));
     c->pme_nx = nx; c->pme_ny = ny;
   }
   int r;
+  const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+  if (points && (r = ensure_pme_grids(c, points, cpoints, er))) return r;
   for (int h : handles) {
     ForceDesc& f = c->forces[h];
     if (!f.pme || !f.recip) continue;
@@ -910,8 +923,7 @@ int ensure_pme(pm_context* c, const std::vector<int>& handles) {
     f.tables = at;
     if (!t.current && (r = fill_tables(c, t))) return r;
   }
-  const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
-  return points ? ensure_pme_grids(c, points, cpoints, er) : PM_OK;
+  return PM_OK;
 }
 
 // ------------------------------------------------------------ force parsing
@@ -1315,15 +1327,21 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   const int* rb = reuse ? c->d_rebuild : nullptr;
   const bool inner = reuse && inner_lists(c);
   c->inner_last = inner;
-  // the list buffers, for the widest pass, before the displacement test, which
-  // decides on a build
-  double pcut = 0.0;
-  for (const PairPass& p : passes) pcut = std::max(pcut, std::sqrt(pair_params(p.terms, c->csf).cut2));
-  if (!passes.empty() && (r = ensure_lists(c, list_capacity(c, pcut + (reuse ? skin : 0.0))))) return r;
-  if (inner && (r = ensure_inner_lists(c))) return r;
+  // the stencils of the passes, and room for the widest one's lists
+  const double lskin = reuse ? skin : 0.0;
+  std::vector<std::pair<int4*, int>> stencil(passes.size());
+  double pcut_max = 0.0;
+  for (size_t pi = 0; pi < passes.size(); pi++) {
+    const PairPass& ps = passes[pi];
+    if ((r = get_stencil(c, ps.algo_cutoff + lskin, false, &stencil[pi].first, &stencil[pi].second))) return r;
+    if (stencil[pi].second > 650)
+      return fail(c, PM_ERR_UNSUPPORTED, "cell stencil of %d columns (cellsize %g, cutoff %g): use a cellsize of at least cutoff/4", stencil[pi].second, c->cellsize, ps.algo_cutoff);
+    pcut_max = std::max(pcut_max, std::sqrt(pair_params(ps.terms, c->csf).cut2));
+  }
+  const int lcap = list_capacity(c, pcut_max + lskin);
   if (reuse) {
-    if (!lists_match(c, passes[0])) c->list_stale = true;
-    c->list_cut = pcut;
+    if (!lists_match(c, passes[0]) || !lists_fit(c, lcap, inner)) c->list_stale = true;
+    c->list_cut = pcut_max;
     c->list_built_skin = skin;
     c->list_sorted = !replica_form(c);
   }
@@ -1360,6 +1378,11 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
                        c->d_atom_of_slot, c->ntypes, c->nslot_max, c->m, rb, reuse ? c->d_xbuild : nullptr,
                        inner ? c->d_xprune : nullptr);
   if (!reuse) c->list_stale = true;   // a layout built without the skin is not reusable
+  }
+  // (allocated while the layout kernels run)
+  if ((!passes.empty() && (r = ensure_lists(c, lcap))) || (inner && (r = ensure_inner_lists(c)))) {
+    c->list_stale = true;
+    return r;
   }
 
   // energy records: pair passes, PME x-pass blocks, correction blocks
@@ -1404,12 +1427,6 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
   for (size_t pi = 0; pi < passes.size(); pi++) {
     PairPass& ps = passes[pi];
     PmPairParams pp = pair_params(ps.terms, c->csf);
-    int4* st;
-    int nst;
-    const double lskin = reuse ? skin : 0.0;
-    if ((r = get_stencil(c, ps.algo_cutoff + lskin, false, &st, &nst))) return r;
-    if (nst > 650)
-      return fail(c, PM_ERR_UNSUPPORTED, "cell stencil of %d columns (cellsize %g, cutoff %g): use a cellsize of at least cutoff/4", nst, c->cellsize, ps.algo_cutoff);
     const double pcut = std::sqrt(pp.cut2);
     pair_launch.push_back(std::make_pair(PmNbLaunch{}, pp));
     PmNbLaunch& a = pair_launch.back().first;
@@ -1422,8 +1439,8 @@ int evaluate_group(pm_context* c, const std::vector<int>& handles, int flags, bo
     a.dummy_slot = c->nslot_max;
     a.cell_slot = c->d_cell_slot;
     a.cell_count = c->d_cell_count;
-    a.stencil = st;
-    a.nstencil = nst;
+    a.stencil = stencil[pi].first;
+    a.nstencil = stencil[pi].second;
     a.jlist = c->d_jlist;
     a.jmask = c->d_jmask;
     a.jcount = c->d_jcount;

@@ -6,7 +6,7 @@ such evaluations between them.  FP64: round-off of sums in another order
 import numpy as np
 import pytest
 
-from protomol_amd import water
+from protomol_amd import gpu, water
 from tests.cases import gpu_forces_c1, rms_rel
 
 pytestmark = pytest.mark.gpu
@@ -140,3 +140,24 @@ def test_md_after_cell_diagnostics(gpu_ctx_factory, integrator):
         got.append(c.md_get_state()[:2])
     np.testing.assert_allclose(got[0][0], got[1][0], rtol=0, atol=1e-7)
     np.testing.assert_allclose(got[0][1], got[1][1], rtol=0, atol=1e-6 * np.abs(got[1][1]).max())
+
+
+def test_refused_cutoff_between(gpu_ctx_factory):
+    """A cutoff whose cell stencil is too large is refused before anything is
+    allocated or queued, and the lists around it still hold."""
+    print("case: refused cutoff between", flush=True)
+    s = water.named("water8k", seed=5, jitter=0.3)
+    c = gpu_ctx_factory("double")
+    c.set_topology(s)
+    c.set_boundary(s.box, s.origin, 1.2)
+    h, wide = c.force(LJ, values(8.0)), c.force(LJ, values(30.0))
+    want = c.evaluate([h], s.pos)
+    builds = c.stats()["list_builds"]
+    for _ in range(2):
+        with pytest.raises(gpu.PmError) as e:
+            c.evaluate([wide], s.pos)
+        assert e.value.code == gpu.PM_ERR_UNSUPPORTED
+        got = c.evaluate([h], s.pos)
+        np.testing.assert_array_equal(got[0], want[0])
+        np.testing.assert_array_equal(got[1], want[1])
+    assert c.stats()["list_builds"] == builds
