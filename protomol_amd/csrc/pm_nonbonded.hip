@@ -2191,13 +2191,13 @@ void pm_launch_bin(hipStream_t s, const PmBox& box, int n, const double* pos, in
 }
 
 // Atoms up to which the scan's single block also scatters, in rounds of 1,024:
-// a launch less, whose boundary costs a step that keeps its lists 1-2 us (25
-// mixed-precision steps, us per step: 1,020 atoms 41 merged, 43 apart; 8,190 66
-// and 67; 12,000 68 and 69; 16,383 75 and 73.5), against the rounds on a step
-// that builds (every step a build: 3,000 atoms 86.5 and 86.5; 4,095 96.5 and 96;
-// 8,190 98.5 and 96; 16,383 112 and 105).  Hence one line for evaluations that may
-// keep their lists (one build in nine steps) and one for those that never do
-#define PM_SCAN_SCATTER 12288
+// a launch less, whose boundary costs a step that keeps its lists 1-3 us (us per
+// step, merged and apart: 1,020 atoms 41 and 43, 9,999 64 and 65, 16,383 68.5
+// and 69, with PME 120 and 123), against the rounds on a step that builds (every
+// step a build: 3,000 atoms 86.5 and 86.5, 4,095 96.5 and 96, 8,190 98.5 and 96,
+// 16,383 112 and 105).  Hence one line for evaluations that may keep their lists
+// and one for those that never do
+#define PM_SCAN_SCATTER 16384
 #define PM_SCAN_SCATTER_BUILD 3072
 static void launch_scatter(hipStream_t s, int n, const int* cell_of, const int* rank, const int* cell_start,
                            int* cell_atoms, const int* rebuild) {
