@@ -273,7 +273,8 @@ int pm_hessian_vec(pm_context* ctx, const int* handles, int nhandles, const doub
 /* Gradients of the energy of a force group with respect to every atom's scaled
  * charge (dE_dq, double[n]), and, with per-atom LJ parameters set, its sigma and
  * epsilon (dE_dsigma, dE_depsilon; pairs that are not MODIFIED; 0 where
- * epsilon is 0).  Any output may be NULL.  No reference counterpart. */
+ * epsilon is 0).  Any output may be NULL.  On an error neither call has
+ * written its outputs.  No reference counterpart. */
 int pm_param_gradients(pm_context* ctx, const int* handles, int nhandles, const double* positions, double* dE_dq,
                        double* dE_dsigma, double* dE_depsilon);
 
