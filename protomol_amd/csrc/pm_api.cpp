@@ -39,8 +39,10 @@
 // paying (us per call staged and straight: 648 atoms 27 and 57, 8,100 53 and
 // 200, 21,843 86 and 92 to 190, 98,304 325 and 355 to 396)
 #define PM_STAGE_STATE 65536
-// tables of PME terms that a context keeps before it refills unused ones
+// tables of PME terms that a context keeps before it refills unused ones, and
+// the theta table beyond which unused ones go back when another is needed
 #define PM_PME_TABLES 4
+#define PM_PME_KEEP_BYTES (64u << 20)
 // work space that a context keeps between pm_lanczos calls
 #define PM_LANCZOS_KEEP_BYTES (256u << 20)
 
@@ -866,7 +868,8 @@ int fill_tables(pm_context* c, PmeTables& t) {
 
 // Alphas, grids and tables of a group's PME terms.  Every term has tables of
 // its own; tables that no term of the group uses are refilled once there are
-// PM_PME_TABLES of them (one with the same grid first: it keeps its buffers).
+// PM_PME_TABLES of them (one with the same grid first: it keeps its buffers),
+// large ones are given back before another term allocates.
 int ensure_pme(pm_context* c, const std::vector<int>& handles) {
   c->pme_group++;
   size_t points = 0, cpoints = 0;
@@ -890,15 +893,38 @@ int ensure_pme(pm_context* c, const std::vector<int>& handles) {
   }
   int r;
   const size_t er = c->precision == PM_PRECISION_DOUBLE ? sizeof(double) : sizeof(float);
+  auto same_grid = [&](const PmeTables& t, const ForceDesc& f) {
+    return t.nx == f.nx && t.ny == f.ny && t.nz == f.nz && t.prec == c->precision;
+  };
+  auto of = [&](const PmeTables& t, const ForceDesc& f) {
+    return same_grid(t, f) && t.order == f.order && t.alpha == f.alpha;
+  };
+  bool missing = false;
+  for (int h : handles) {
+    const ForceDesc& f = c->forces[h];
+    if (f.pme && f.recip)
+      missing |= std::none_of(c->pme_tables.begin(), c->pme_tables.end(), [&](const PmeTables& t) { return of(t, f); });
+  }
+  if (missing)
+    for (PmeTables& t : c->pme_tables) {
+      const size_t bytes = (size_t)t.nx * t.ny * (t.nz / 2 + 1) * (t.prec == PM_PRECISION_DOUBLE ? 8 : 4);
+      if (bytes > PM_PME_KEEP_BYTES && std::none_of(handles.begin(), handles.end(), [&](int h) {
+            const ForceDesc& f = c->forces[h];
+            return f.pme && f.recip && of(t, f);
+          })) {
+        c->gen++;
+        free_tables(t);
+      }
+    }
   if (points && (r = ensure_pme_grids(c, points, cpoints, er))) return r;
   for (int h : handles) {
     ForceDesc& f = c->forces[h];
     if (!f.pme || !f.recip) continue;
     int at = -1;
-    auto grid = [&](const PmeTables& t) { return t.nx == f.nx && t.ny == f.ny && t.nz == f.nz && t.prec == c->precision; };
+    auto grid = [&](const PmeTables& t) { return same_grid(t, f); };
     const int count = (int)c->pme_tables.size();
     for (int k = 0; k < count && at < 0; k++)
-      if (grid(c->pme_tables[k]) && c->pme_tables[k].order == f.order && c->pme_tables[k].alpha == f.alpha) at = k;
+      if (of(c->pme_tables[k], f)) at = k;
     if (at < 0 && count >= PM_PME_TABLES) {
       // refill: of the group's unused ones the same grid, else the longest unused
       for (int k = 0; k < count; k++) {
@@ -914,7 +940,10 @@ int ensure_pme(pm_context* c, const std::vector<int>& handles) {
       c->pme_tables.push_back(PmeTables());
     }
     PmeTables& t = c->pme_tables[at];
-    if (!grid(t)) free_tables(t);
+    if (!grid(t)) {
+      c->gen++;
+      free_tables(t);
+    }
     if (!grid(t) || t.order != f.order || t.alpha != f.alpha) t.current = false;
     t.nx = f.nx; t.ny = f.ny; t.nz = f.nz; t.prec = c->precision;
     t.order = f.order;

@@ -104,3 +104,20 @@ def test_real_terms_of_two_cutoffs(gpu_ctx_factory, cutoffs):
     want = parts[0][0] + parts[1][0]
     assert np.abs(f - want).max() <= 16 * 2.0 ** -40 + 1e-14 * np.abs(want).max()
     np.testing.assert_allclose(e, parts[0][1] + parts[1][1], rtol=1e-12, atol=1e-9)
+
+
+# tables of a large grid (theta over 64 MB) go back when another term needs
+# its own, and are filled again
+def test_large_grids_in_turn(gpu_ctx_factory):
+    print("case: large pme grids in turn", flush=True)
+    s = water.named("water648", seed=9, jitter=0.3)
+    c = context(gpu_ctx_factory, s, "double")
+    hs = [c.force(PME, term(grid=g)) for g in (256, 24, 288)]
+    want = [c.evaluate([h], s.pos) for h in hs]
+    for k in (0, 2, 1, 2, 0):
+        f, e = c.evaluate([hs[k]], s.pos)
+        np.testing.assert_array_equal(f, want[k][0])
+        np.testing.assert_array_equal(e, want[k][1])
+    f, _ = c.evaluate(hs, s.pos)
+    total = sum(w[0] for w in want)
+    assert np.abs(f - total).max() <= 16 * 2.0 ** -40 + 1e-14 * np.abs(total).max()
