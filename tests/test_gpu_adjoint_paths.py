@@ -11,6 +11,7 @@ import pytest
 
 from protomol_amd import gpu, water
 from tests.cases import ALPHA_RC8, rms_rel
+from tests.test_gpu_adjoint import away_from_cutoff, unit
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +97,22 @@ def test_refused_parameters_change_nothing(gpu_ctx_factory):
         c.set_lj_per_atom(2.0 * bad, 3.0 * eps)
     for a, b in zip(c.param_gradients(hs, s.pos), want):
         np.testing.assert_array_equal(a, b)
+
+
+# 16, 8, 4, 2 and 1 waves per cluster (as many as keep the launch within
+# 16,384): H v against central differences of the forces, h = 1e-4 A (FP64;
+# the truncation of second order is 1e-7 of the largest terms, round-off less).
+# The second derivative of a C2-switched term jumps at its cutoff: atoms of
+# pairs that the differences could carry across it stay put
+@pytest.mark.parametrize("molecules", [300, 4000, 9000, 20000, 30000])
+def test_products_over_launch_shapes(gpu_ctx_factory, molecules):
+    print("case: adjoint launch shapes", molecules, flush=True)
+    s = water.water_box(molecules, (molecules / 0.0334) ** (1.0 / 3.0), seed=molecules, jitter=0.3)
+    c = gpu_ctx_factory("double")
+    c.set_topology(s)
+    c.set_boundary(s.box, s.origin, 4.0)
+    hs = [c.force(*LJ), c.force("Coulomb -algorithm NonbondedCutoff -switchingFunction C2", [6.0, 7.0, 7.0])]
+    v, _ = away_from_cutoff(s, unit(np.random.default_rng(molecules), (s.n, 3)), 7.0)
+    h = 1e-4
+    fd = -(c.evaluate(hs, s.pos + h * v)[0] - c.evaluate(hs, s.pos - h * v)[0]) / (2 * h)
+    assert rms_rel(c.hessian_vec(hs, s.pos, v), fd) < 2e-6
